@@ -920,11 +920,10 @@ adjoint_group32_kernel(const Bucket* __restrict__ bk, const int32_t* __restrict_
 }
 
 // Pushes node cotangents to every particle through the closed-form moments of
-// its leaf and each ancestor (parent links up to the root).  head/head_pos
-// give the particle's bucket (head_pos[j] + head[j] - 1).
+// its leaf and each ancestor (parent links up to the root).
 __global__ void __launch_bounds__(256)
-adjoint_down_kernel(int64_t n, const uint32_t* __restrict__ head,
-                    const uint32_t* __restrict__ head_pos, const int32_t* __restrict__ bucket_node,
+adjoint_down_kernel(int64_t n, const uint32_t* __restrict__ bucket_of,
+                    const int32_t* __restrict__ bucket_node,
                     const int32_t* __restrict__ parent, const GravNode* __restrict__ gn,
                     const double* __restrict__ lam_node, int64_t nn,
                     const double* __restrict__ px, const double* __restrict__ py,
@@ -934,8 +933,7 @@ adjoint_down_kernel(int64_t n, const uint32_t* __restrict__ head,
                     double* __restrict__ gmass) {
   const int64_t j = blockIdx.x * 256ll + threadIdx.x;
   if (j >= n) return;
-  const int64_t bucket = (int64_t)head_pos[j] + head[j] - 1;
-  int32_t s = bucket_node[bucket];
+  int32_t s = bucket_node[bucket_of[j]];
   const double x = px[j], y = py[j], z = pz[j], m = pm[j], e = pe[j];
   double ax = 0.0, ay = 0.0, az = 0.0, am = 0.0;
   while (s >= 0) {
@@ -1176,13 +1174,13 @@ int pt_launch_adjoint_groups(int precision, const Bucket* bk, const int32_t* gfi
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-int pt_launch_adjoint_down(int64_t n, const uint32_t* head, const uint32_t* head_pos,
-                           const int32_t* bucket_node, const int32_t* parent, const GravNode* gn,
+int pt_launch_adjoint_down(int64_t n, const uint32_t* bucket_of, const int32_t* bucket_node,
+                           const int32_t* parent, const GravNode* gn,
                            const double* lam_node, int64_t nn, const double* x, const double* y,
                            const double* z, const double* m, const double* e, double* gx,
                            double* gy, double* gz, double* gm, hipStream_t s) {
   if (n <= 0) return 0;
-  adjoint_down_kernel<<<grid_for(n), 256, 0, s>>>(n, head, head_pos, bucket_node, parent, gn,
+  adjoint_down_kernel<<<grid_for(n), 256, 0, s>>>(n, bucket_of, bucket_node, parent, gn,
                                                   lam_node, nn, x, y, z, m, e, gx, gy, gz, gm);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }

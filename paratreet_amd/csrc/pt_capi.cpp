@@ -67,16 +67,17 @@ struct pt_ctx {
   int32_t max_depth = 0;
   DBuf<uint64_t> nkey;
   DBuf<int32_t> nbegin, ncount, ndepth, ntype, nparent, nfirst;
-  DBuf<int32_t> level_nodes, level_cnt;
-  DBuf<int64_t> tstat;  // build read-back: {nn, nb, overflow, level counts}
+  DBuf<int32_t> level_nodes;
+  DBuf<int64_t> tstat;     // build read-back (pt_launch_build)
+  DBuf<int2> tinternal;    // build: first particle and depth of each internal node
+  DBuf<uint16_t> tmeta;    // build: what starts at each particle
   std::vector<int64_t> level_off;  // internal nodes of depth d: [level_off[d], level_off[d+1])
-  int32_t split_levels = PT_MAX_DEPTH;  // split launches of the next build (last depth + 1)
   // key bits the last sort ordered (64: all; fewer: the top bits only, the
   // build then puts each leaf in full order) and those the next force
   // evaluation's sort will order (what the last tree's splits used)
   int32_t sort_bits = 64;
   int32_t sort_bits_next = 64;
-  DBuf<uint32_t> flag, fpos, head, head_pos, u32_total;
+  DBuf<uint32_t> bucket_of, u32_total;  // bucket of each particle (sorted order)
   DBuf<int32_t> bucket_node;
   DBuf<double> nd;
   DBuf<int32_t> ord_h;
@@ -372,9 +373,8 @@ void pt_ctx_destroy(pt_ctx* c) {
   release(c->box); release(c->bbox); release(c->box_parts);
   release(c->nkey); release(c->nbegin); release(c->ncount); release(c->ndepth); release(c->ntype);
   release(c->nparent); release(c->nfirst); release(c->level_nodes);
-  release(c->level_cnt);
-  release(c->flag); release(c->fpos); release(c->head); release(c->head_pos); release(c->u32_total);
-  release(c->tstat);
+  release(c->bucket_of); release(c->u32_total);
+  release(c->tstat); release(c->tinternal); release(c->tmeta);
   release(c->prec);
   release(c->ewt);
   release(c->ewcount);
@@ -438,8 +438,8 @@ pt_status pt_set_particles(pt_ctx* c, int64_t n, const double* x, const double* 
   PT_TRY_HIP(c, ensure(c->keys, std::max<int64_t>(n, 1)));
   PT_TRY_HIP(c, ensure(c->skeys, std::max<int64_t>(n, 1)));
   PT_TRY_HIP(c, ensure(c->perm, std::max<int64_t>(n, 1)));
-  PT_TRY_HIP(c, ensure(c->head, std::max<int64_t>(n, 1)));
-  PT_TRY_HIP(c, ensure(c->head_pos, std::max<int64_t>(n, 1)));
+  PT_TRY_HIP(c, ensure(c->bucket_of, std::max<int64_t>(n, 1)));
+  PT_TRY_HIP(c, ensure(c->tmeta, std::max<int64_t>(n, 1)));
   PT_TRY_HIP(c, ensure(c->bucket_node, std::max<int64_t>(n, 1)));
   c->n = n;
   c->have_forces = false;
@@ -549,9 +549,8 @@ extern "C" {
 
 pt_status pt_sort(pt_ctx* c) { return sort_stage(c, 64); }
 
-// Level-parallel build driven from the device: one split launch per level
-// (internal-node counts stay on the device), a host check every 4 levels, and
-// a rebuild with larger tables if a capacity was exceeded.
+// Builds every level on the device and reads the sizes back once; a tree of
+// more internal nodes than the tables hold is built again with room for it.
 pt_status pt_build_tree(pt_ctx* c) {
   pt_status st = check_ctx(c);
   if (st) return st;
@@ -559,36 +558,19 @@ pt_status pt_build_tree(pt_ctx* c) {
   const int B = c->cfg.max_particles_per_leaf;
   Timer t(c, PT_T_BUILD);
   // internal nodes of one level are disjoint and hold more than B particles
-  const int64_t per_level = c->n / (B + 1) + 1;
-  int64_t level_cap = std::max<int64_t>(64, 2 * per_level);
-  PT_TRY_HIP(c, ensure(c->level_cnt, PT_MAX_DEPTH + 2));
-  int capacity_retries = 0;
+  int64_t level_cap = std::max<int64_t>(64, 2 * (c->n / (B + 1) + 1));
+  PT_TRY_HIP(c, ensure(c->tstat, PT_TREE_STATUS));
+  if ((st = ensure_scratch(c, pt_tree_scratch_bytes(c->n)))) return st;
+  int64_t stat[PT_TREE_STATUS] = {0};
   for (int attempt = 0;; attempt++) {
-    const int64_t node_cap = 1 + 8 * level_cap;
     c->nn = 0;
-    if ((st = ensure_nodes(c, node_cap))) return st;
+    if ((st = ensure_nodes(c, 1 + 8 * level_cap))) return st;
     PT_TRY_HIP(c, ensure(c->level_nodes, level_cap));
+    PT_TRY_HIP(c, ensure(c->tinternal, level_cap));
     PtTree tr = tree_of(c);
-    PT_TRY_LAUNCH(c, pt_launch_fill_u32((uint32_t*)c->derr.p, 1, 0u, c->stream));
-    PT_TRY_LAUNCH(c, pt_launch_root(c->n, B, tr, c->level_cnt.p, c->stream));
-    PT_TRY_LAUNCH(c, pt_launch_fill_u32((uint32_t*)c->level_nodes.p, 1, 0u, c->stream));
-    // the splits of the previous build's depth plus one level (all levels the
-    // first time; a deeper tree is detected below and rebuilt with all);
-    // the buckets follow on the device and one read-back returns counts,
-    // sizes and the overflow flag
-    const int levels = c->split_levels;
-    int64_t bound = 1;  // upper bound of the level's internal-node count
-    for (int depth = 0; depth < levels; depth++) {
-      PT_TRY_LAUNCH(c, pt_launch_split_level(c->skeys.p, c->level_nodes.p, c->level_cnt.p, depth,
-                                             bound, B, tr, node_cap, level_cap, c->derr.p,
-                                             c->stream));
-      bound = std::min<int64_t>(bound * 8, per_level);
-    }
-    if ((st = ensure_scratch(c, pt_scan_scratch_bytes(c->n)))) return st;
-    PT_TRY_HIP(c, ensure(c->tstat, 3 + PT_MAX_DEPTH + 2));
-    PT_TRY_LAUNCH(c, pt_launch_buckets(tr, node_cap, c->n, levels, c->level_cnt.p, c->derr.p,
-                                       c->head.p, c->head_pos.p, c->scratch.p, c->u32_total.p,
-                                       c->bucket_node.p, c->tstat.p, c->stream));
+    PT_TRY_LAUNCH(c, pt_launch_build(c->skeys.p, c->n, B, c->sort_bits, tr, level_cap,
+                                     c->level_nodes.p, c->tinternal.p, c->tmeta.p, c->bucket_of.p,
+                                     c->bucket_node.p, c->scratch.p, c->tstat.p, c->stream));
     if (c->sort_bits < 64) {
       // top-bits sort: each leaf's particles into full key order, then the
       // sorted copies (idempotent if a retry below builds again)
@@ -597,43 +579,26 @@ pt_status pt_build_tree(pt_ctx* c) {
       PT_TRY_LAUNCH(c, pt_launch_gather(c->perm.p, c->n, c->prec.p, c->xs.p, c->ys.p, c->zs.p,
                                         c->ms.p, c->es.p, c->stream));
     }
-    int64_t stat[3 + PT_MAX_DEPTH + 2] = {0};
     PT_TRY_HIP(c, read_back(c, stat, c->tstat.p, sizeof(stat)));
-    if (c->sort_bits < 64) {
-      // valid when every split compared only sorted bits: a split creating
-      // depth d + 1 reads the top 3 (d + 1) + 1 bits
-      int dmax = 0;
-      for (int d = 0; d <= PT_MAX_DEPTH; d++)
-        if (stat[3 + d] > 0) dmax = d + 1;
-      if (stat[2] || stat[0] == 0 || 3 * dmax + 1 > c->sort_bits) return kRedoFullSort;
-    }
-    if (stat[2]) {
-      if (++capacity_retries > 3) return fail(c, PT_ERR_CAPACITY, "octree node table overflow");
-      level_cap *= 4;
-      continue;
-    }
-    if (stat[0] == 0) {
-      // deeper than predicted: all levels
-      if (levels >= PT_MAX_DEPTH || attempt > 8)
-        return fail(c, PT_ERR_CAPACITY, "octree build did not complete");
-      c->split_levels = PT_MAX_DEPTH;
-      continue;
-    }
-    // level table: internal nodes of depth d are [level_off[d], level_off[d+1])
-    const int64_t* cnt = stat + 3;
-    c->level_off.assign(1, 0);
-    c->max_depth = 0;
-    int64_t internal = 0;
-    for (int d = 0; d <= PT_MAX_DEPTH; d++) {
-      internal += cnt[d];
-      c->level_off.push_back(internal);
-      if (cnt[d] > 0) c->max_depth = d + 1;
-    }
-    c->nn = stat[0];
-    c->nb = stat[1];
-    c->split_levels = std::min<int32_t>(PT_MAX_DEPTH, c->max_depth + 1);
-    break;
+    // a split would have read bits the sort did not order
+    if (stat[PT_TREE_STATUS - 1] != 0) return kRedoFullSort;
+    if (stat[2] == 0) break;
+    if (attempt > 0 || 1 + 8 * stat[2] > 0x7fffffffll)
+      return fail(c, PT_ERR_CAPACITY, "octree node table overflow");
+    level_cap = stat[2];
   }
+  // level table: internal nodes of depth d are [level_off[d], level_off[d+1])
+  const int64_t* cnt = stat + 3;
+  c->level_off.assign(1, 0);
+  c->max_depth = 0;
+  int64_t internal = 0;
+  for (int d = 0; d <= PT_MAX_DEPTH; d++) {
+    internal += cnt[d];
+    c->level_off.push_back(internal);
+    if (cnt[d] > 0) c->max_depth = d + 1;
+  }
+  c->nn = stat[0];
+  c->nb = stat[1];
   c->stage = S_TREE;
   return PT_OK;
 }
@@ -678,7 +643,7 @@ pt_status pt_upward(pt_ctx* c) {
   PT_TRY_HIP(c, ensure(c->gn32, nn));
   PT_TRY_HIP(c, ensure(c->bk, std::max<int64_t>(c->nb, 1)));
   PtTree tr = tree_of(c);
-  const PtPackOut po{c->tnode.p, c->gn.p, c->gn32.p, c->bk.p, c->head_pos.p};
+  const PtPackOut po{c->tnode.p, c->gn.p, c->gn32.p, c->bk.p, c->bucket_of.p};
   PT_TRY_LAUNCH(c, pt_launch_leaf_moments(tr, nn, c->xs.p, c->ys.p, c->zs.p, c->ms.p, c->es.p,
                                           c->nd.p, po, c->stream));
   // internal nodes, deepest level first: a level of more than kRunNodes
@@ -1411,8 +1376,8 @@ pt_status vjp_accumulate(pt_ctx* c, int mode, double theta, const AdjViews& v, c
                        c->es.p, c->gpp_off.p, c->gpp.p, c->gppm.p, c->gpc_off.p, c->gpc.p,
                        c->gpcm.p, c->offset, v.wsx, v.wsy, v.wsz, v.gsx, v.gsy, v.gsz, v.gsm,
                        c->lam_node.p, nn, c->stream));
-  PT_TRY_LAUNCH(c, pt_launch_adjoint_down(n, c->head.p, c->head_pos.p, c->bucket_node.p,
-                                          c->nparent.p, c->gn.p, c->lam_node.p, nn, c->xs.p,
+  PT_TRY_LAUNCH(c, pt_launch_adjoint_down(n, c->bucket_of.p, c->bucket_node.p, c->nparent.p,
+                                          c->gn.p, c->lam_node.p, nn, c->xs.p,
                                           c->ys.p, c->zs.p, c->ms.p, c->es.p, v.gsx, v.gsy,
                                           v.gsz, v.gsm, c->stream));
   PT_TRY_LAUNCH(c, pt_launch_scatter_add4(c->perm.p, n, v.gsx, v.gsy, v.gsz, v.gsm, gx, gy, gz,

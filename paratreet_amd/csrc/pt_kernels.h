@@ -41,21 +41,27 @@ int pt_launch_iota(uint32_t* v, int64_t n, hipStream_t s);
 // Message of the calling thread's last failed pt_sort_noalloc, or NULL.
 const char* pt_noalloc_last_error();
 
-int pt_launch_root(int64_t n, int bucket, const PtTree& t, int32_t* level_cnt, hipStream_t s);
 // Largest leaf the fixup after a top-bits sort handles (larger buckets use
 // the full sort).
 constexpr int kFixupMax = 64;
 // status: the build read-back ({nn, nb, ...}); max_buckets bounds nb.
 int pt_launch_leaf_fixup(const PtTree& t, int64_t max_buckets, const int32_t* bucket_node,
                          const int64_t* status, uint64_t* keys, uint32_t* perm, hipStream_t s);
-int pt_launch_split_level(const uint64_t* keys, int32_t* level_nodes, int32_t* level_cnt, int d,
-                          int64_t max_frontier, int bucket, const PtTree& t, int64_t node_cap,
-                          int64_t level_cap, int32_t* overflow, hipStream_t s);
-// levels: the split launches done (depths 0 .. levels-1).
-int pt_launch_buckets(const PtTree& t, int64_t node_cap, int64_t n, int levels,
-                      const int32_t* level_cnt, const int32_t* overflow, uint32_t* head,
-                      uint32_t* head_pos, void* scan_scratch, uint32_t* nb_out,
-                      int32_t* bucket_node, int64_t* status, hipStream_t s);
+// The octree over keys whose top `bits` bits are in order (64: all), at most
+// level_cap internal nodes: the node table t (1 + 8 level_cap entries), the
+// internal nodes' ids in level order, each particle's bucket and each bucket's
+// node.  internal: level_cap entries of scratch, meta: n, scratch:
+// pt_tree_scratch_bytes(n).  status: PT_TREE_STATUS words, {nn, nb, internal
+// nodes needed when there are more than level_cap (else 0), internal nodes per
+// depth [PT_MAX_DEPTH + 2], places where the ordered bits did not suffice};
+// nn = nb = 0 and no tree when it does not fit or the last is not 0.
+#define PT_TREE_ROWS (PT_MAX_DEPTH + 2)
+#define PT_TREE_STATUS (3 + PT_MAX_DEPTH + 2 + 1)
+int64_t pt_tree_scratch_bytes(int64_t n);
+int pt_launch_build(const uint64_t* keys, int64_t n, int bucket, int bits, const PtTree& t,
+                    int64_t level_cap, int32_t* level_nodes, int2* internal, uint16_t* meta,
+                    uint32_t* bucket_of, int32_t* bucket_node, void* scratch, int64_t* status,
+                    hipStream_t s);
 
 // HEXADECAPOLE moments: raw third/fourth moments (SoA, PT_HEXA_RAW x nn) of
 // the buckets, then of each internal level (deepest first), then the records.
@@ -69,13 +75,13 @@ int pt_launch_hexa_pack(const PtTree& t, const double* nd, const double* raw, in
 // Leaf CentroidData of every leaf and the default record of every empty leaf.
 // Where the moment kernels write each node's walk and interaction records as
 // soon as its CentroidData is final, and each bucket's record (index
-// head_pos[first particle]).
+// bucket_of[first particle]).
 struct PtPackOut {
   TreeNode* tnode;
   GravNode* gn;
   GravNode32* gn32;
   Bucket* bk;
-  const uint32_t* head_pos;
+  const uint32_t* bucket_of;
 };
 int pt_launch_leaf_moments(const PtTree& t, int64_t nn, const double* x, const double* y,
                            const double* z, const double* m, const double* e, double* nd,
@@ -265,8 +271,8 @@ int pt_launch_adjoint_groups(int precision, const Bucket* bk, const int32_t* gfi
                              const double off[3], const double* wx, const double* wy,
                              const double* wz, double* gx, double* gy, double* gz, double* gm,
                              double* lam_node, int64_t nn, hipStream_t s);
-int pt_launch_adjoint_down(int64_t n, const uint32_t* head, const uint32_t* head_pos,
-                           const int32_t* bucket_node, const int32_t* parent, const GravNode* gn,
+int pt_launch_adjoint_down(int64_t n, const uint32_t* bucket_of, const int32_t* bucket_node,
+                           const int32_t* parent, const GravNode* gn,
                            const double* lam_node, int64_t nn, const double* x, const double* y,
                            const double* z, const double* m, const double* e, double* gx,
                            double* gy, double* gz, double* gm, hipStream_t s);

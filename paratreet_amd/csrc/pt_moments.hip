@@ -175,7 +175,7 @@ __device__ __forceinline__ float round_up_f32(double v) {
 // (the same values a pass over the SoA node table would read back).  Leaves
 // also get their reach and softening bounds (leaf_soft: the largest particle
 // softening) and, when non-empty, their bucket record (bucket index
-// head_pos[begin]).
+// bucket_of[begin]).
 __device__ __forceinline__ void pack_node(const PtTree& t, int64_t i, const CData& d,
                                           double leaf_soft, const PtPackOut& o) {
   TreeNode a;
@@ -249,7 +249,7 @@ __device__ __forceinline__ void pack_node(const PtTree& t, int64_t i, const CDat
     b.begin = a.begin;
     b.count = a.count;
     b.pad2 = 0;
-    o.bk[o.head_pos[a.begin]] = b;
+    o.bk[o.bucket_of[a.begin]] = b;
   }
 }
 
