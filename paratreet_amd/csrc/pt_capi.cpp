@@ -635,7 +635,7 @@ pt_status pt_upward(pt_ctx* c) {
   if ((st = need(c, S_TREE, "pt_upward"))) return st;
   Timer t(c, PT_T_MOMENTS);
   const int64_t nn = c->nn;
-  PT_TRY_HIP(c, ensure(c->nd, PT_CD_NFIELDS * nn));
+  PT_TRY_HIP(c, ensure(c->nd, PT_ND_STRIDE * nn));
   PT_TRY_HIP(c, ensure(c->ord_h, nn));
   PT_TRY_HIP(c, ensure(c->ord_b, nn));
   PT_TRY_HIP(c, ensure(c->tnode, nn));
@@ -648,7 +648,7 @@ pt_status pt_upward(pt_ctx* c) {
                                           c->nd.p, po, c->stream));
   // internal nodes, deepest level first: a level of more than kRunNodes
   // nodes gets its own launch, consecutive smaller ones share one work-group
-  constexpr int64_t kRunNodes = 64;
+  constexpr int64_t kRunNodes = 256;
   const int nlev = (int)c->level_off.size() - 1;
   PtLevelRun run{};
   for (int d = nlev - 1; d >= 0; d--) {
@@ -660,13 +660,13 @@ pt_status pt_upward(pt_ctx* c) {
       run.nlev++;
       continue;
     }
-    PT_TRY_LAUNCH(c, pt_launch_upward_run(tr, c->level_nodes.p, run, c->nd.p, nn, c->ord_h.p,
+    PT_TRY_LAUNCH(c, pt_launch_upward_run(tr, c->level_nodes.p, run, c->nd.p, c->ord_h.p,
                                           c->ord_b.p, po, c->stream));
     run.nlev = 0;
     PT_TRY_LAUNCH(c, pt_launch_upward_level(tr, c->level_nodes.p + a, (int32_t)(b - a), c->nd.p,
-                                            nn, c->ord_h.p, c->ord_b.p, po, c->stream));
+                                            c->ord_h.p, c->ord_b.p, po, c->stream));
   }
-  PT_TRY_LAUNCH(c, pt_launch_upward_run(tr, c->level_nodes.p, run, c->nd.p, nn, c->ord_h.p,
+  PT_TRY_LAUNCH(c, pt_launch_upward_run(tr, c->level_nodes.p, run, c->nd.p, c->ord_h.p,
                                         c->ord_b.p, po, c->stream));
   if (c->cfg.hexadecapole) {
     // third and fourth moments once every centre of mass is final
@@ -1584,10 +1584,21 @@ pt_status pt_get_node_data(pt_ctx* c, double* out) {
   if (st) return st;
   if ((st = need(c, S_MOMENTS, "pt_get_node_data"))) return st;
   const int64_t nn = c->nn;
-  std::vector<double> soa((size_t)nn * PT_CD_NFIELDS);
-  if ((st = d2h(c, soa.data(), c->nd.p, soa.size() * sizeof(double)))) return st;
-  for (int64_t i = 0; i < nn; i++)
-    for (int f = 0; f < PT_CD_NFIELDS; f++) out[i * PT_CD_NFIELDS + f] = soa[(size_t)f * nn + i];
+  std::vector<double> rec((size_t)nn * PT_ND_STRIDE);
+  if ((st = d2h(c, rec.data(), c->nd.p, rec.size() * sizeof(double)))) return st;
+  for (int64_t i = 0; i < nn; i++) {
+    const double* r = rec.data() + i * PT_ND_STRIDE;
+    double* f = out + i * PT_CD_NFIELDS;
+    f[0] = r[PT_ND_RADIUS];
+    f[1] = r[PT_ND_SOFT];
+    f[2] = r[PT_ND_MASS];
+    for (int k = 0; k < 3; k++) {
+      f[3 + k] = r[PT_ND_CM + k];
+      f[12 + k] = r[PT_ND_LO + k];
+      f[15 + k] = r[PT_ND_HI + k];
+    }
+    for (int k = 0; k < 6; k++) f[6 + k] = r[PT_ND_Q(k)];
+  }
   return PT_OK;
 }
 

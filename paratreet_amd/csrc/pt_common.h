@@ -14,16 +14,22 @@
 // Node types, same numbering as the oracle (EmptyLeaf, Leaf, Internal).
 enum { PT_NODE_EMPTY = 0, PT_NODE_LEAF = 1, PT_NODE_INTERNAL = 2 };
 
-// Per-node moment record fields (CentroidData flattened), SoA index order used
-// by pt_get_node_data: radius soft mass cmx cmy cmz xx xy xz yy yz zz lox loy
-// loz hix hiy hiz.
-#define PT_CD_RADIUS 0
-#define PT_CD_SOFT 1
-#define PT_CD_MASS 2
-#define PT_CD_CM 3
-#define PT_CD_Q 6
-#define PT_CD_LO 12
-#define PT_CD_HI 15
+// CentroidData of a node, five rows of four doubles (160 bytes): cm and
+// softening, the diagonal second moments and the mass, the mixed second
+// moments and the radius, lesser and greater box corners.  The moment kernels
+// give each of a row's columns to one lane of a quad, so a quad reads and
+// writes a row as 32 contiguous bytes.  PT_ND_Q(k), k = xx xy xz yy yz zz.
+#define PT_ND_STRIDE 20
+#define PT_ND_CM 0
+#define PT_ND_SOFT 3
+#define PT_ND_MASS 7
+#define PT_ND_RADIUS 11
+#define PT_ND_LO 12
+#define PT_ND_HI 16
+__host__ __device__ constexpr int PT_ND_Q(int k) {
+  return k == 0 ? 4 : k == 1 ? 8 : k == 2 ? 10 : k == 3 ? 5 : k == 4 ? 9 : 6;
+}
+// Fields per node of pt_get_node_data: radius soft mass cm[3] q[6] lo[3] hi[3].
 #define PT_CD_NFIELDS 18
 
 // Packed node record read by the tree walk: centre of mass, radius and
@@ -48,8 +54,8 @@ struct __align__(64) TreeNode {
 // tr = 0.5 * (qxx + qyy + qzz) as GravityVisitor::node computes it.
 struct __align__(32) GravNode {
   double cx, cy, cz, soft;
-  double mass, qxx, qxy, qxz;
-  double qyy, qyz, qzz, tr;
+  double qxx, qyy, qzz, mass;
+  double qxy, qyz, qxz, tr;
 };
 // Source record of the compensated-FP32 interactions in one 64-byte line: the
 // centre of mass and softening in FP64 (the centre is shifted per target
@@ -57,7 +63,7 @@ struct __align__(32) GravNode {
 // mass, softening and quadrupole.
 struct __align__(64) GravNode32 {
   double cx, cy, cz, soft64;
-  float mass, soft, qxx, qxy, qxz, qyy, qyz, qzz;
+  float qxx, qxy, qyy, qyz, qzz, qxz, mass, soft;
 };
 // HEXADECAPOLE build (-DHEXADECAPOLE, examples/Makefile:5).  Source record
 // of node(): centre of mass, mass, softening and the 21 reduced (trace-free)
@@ -83,9 +89,9 @@ struct __align__(64) ParticleRec {
 
 // Bucket (target leaf) record: particle range, box, centre of mass, softening.
 struct __align__(32) Bucket {
-  double lox, loy, loz, hix;
-  double hiy, hiz, cx, cy;
-  double cz, soft, pad0, pad1;
+  double lox, loy, loz, pad0;
+  double hix, hiy, hiz, pad1;
+  double cx, cy, cz, soft;
   int32_t node, begin, count, pad2;
 };
 
@@ -128,6 +134,24 @@ __device__ __forceinline__ float pt_wave_max_f32(float v) {
 // Sum over the 64 lanes (all active), as a wave-uniform value.
 __device__ __forceinline__ int pt_wave_sum_int(int v) {
   return __builtin_amdgcn_readlane(pt_wave_incl_scan(v), PT_WAVE - 1);
+}
+
+// Quad permutations (four neighbouring lanes): lane l reads lane
+// (CTRL >> 2 l) & 3 of its quad.
+template <int CTRL>
+__device__ __forceinline__ int pt_quad_i32(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true);
+}
+template <int CTRL>
+__device__ __forceinline__ unsigned long long pt_quad_u64(unsigned long long v) {
+  const unsigned lo = (unsigned)pt_quad_i32<CTRL>((int)(unsigned)v);
+  const unsigned hi = (unsigned)pt_quad_i32<CTRL>((int)(unsigned)(v >> 32));
+  return ((unsigned long long)hi << 32) | lo;
+}
+template <int CTRL>
+__device__ __forceinline__ double pt_quad_f64(double v) {
+  return __longlong_as_double(
+      (long long)pt_quad_u64<CTRL>((unsigned long long)__double_as_longlong(v)));
 }
 
 // A double moved by one DPP control (both 32-bit halves); lanes without a

@@ -44,7 +44,7 @@ __device__ __forceinline__ uint64_t pack(int32_t s, int32_t t, bool inverted) {
 
 struct DualNodes {
   const TreeNode* tn;
-  const double* nd;      // CentroidData fields, field-major (PT_CD_*)
+  const double* nd;      // CentroidData records (PT_ND_*)
   const int32_t* depth;
   const int32_t* bucket_of;
   int64_t nn;
@@ -58,8 +58,8 @@ __device__ __forceinline__ bool intersect_node_box(const DualNodes& N, int32_t t
   double dsq = 0.0;
 #pragma unroll
   for (int k = 0; k < 3; k++) {
-    const double lo = N.nd[(PT_CD_LO + k) * N.nn + t];
-    const double hi = N.nd[(PT_CD_HI + k) * N.nn + t];
+    const double lo = N.nd[(int64_t)t * PT_ND_STRIDE + PT_ND_LO + k];
+    const double hi = N.nd[(int64_t)t * PT_ND_STRIDE + PT_ND_HI + k];
     if (p[k] < lo) {
       const double d = lo - p[k];
       dsq += d * d;
@@ -86,8 +86,8 @@ __device__ __forceinline__ bool gv_cell(const DualNodes& N, int32_t s, int32_t t
   bool enclose = true;
 #pragma unroll
   for (int k = 0; k < 3; k++) {
-    enclose = enclose && N.nd[(PT_CD_LO + k) * N.nn + s] <= N.nd[(PT_CD_LO + k) * N.nn + t] &&
-              N.nd[(PT_CD_HI + k) * N.nn + t] <= N.nd[(PT_CD_HI + k) * N.nn + s];
+    enclose = enclose && N.nd[(int64_t)s * PT_ND_STRIDE + PT_ND_LO + k] <= N.nd[(int64_t)t * PT_ND_STRIDE + PT_ND_LO + k] &&
+              N.nd[(int64_t)t * PT_ND_STRIDE + PT_ND_HI + k] <= N.nd[(int64_t)s * PT_ND_STRIDE + PT_ND_HI + k];
   }
   return !enclose;
 }

@@ -95,11 +95,10 @@ struct PtLevelRun {
   int32_t cnt[PT_MAX_RUN];
 };
 int pt_launch_upward_run(const PtTree& t, const int32_t* level_nodes, const PtLevelRun& run,
-                         double* nd, int64_t nn, int32_t* ord_h, uint64_t* ord_b,
-                         const PtPackOut& o, hipStream_t s);
+                         double* nd, int32_t* ord_h, uint64_t* ord_b, const PtPackOut& o,
+                         hipStream_t s);
 int pt_launch_upward_level(const PtTree& t, const int32_t* level_nodes, int32_t nl, double* nd,
-                           int64_t nn, int32_t* ord_h, uint64_t* ord_b, const PtPackOut& o,
-                           hipStream_t s);
+                           int32_t* ord_h, uint64_t* ord_b, const PtPackOut& o, hipStream_t s);
 
 // List-producing traversal (count pass when fill is false).  partials holds
 // pt_traverse_blocks(nb) x 4 counters, reduced by pt_launch_reduce_counters.

@@ -207,9 +207,9 @@ constexpr double kPi = 3.14159265358979323846;
 __global__ void ewald_table_kernel(const double* __restrict__ nd, int64_t nn, double L,
                                    double* __restrict__ table, int32_t* __restrict__ count) {
   if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  const double mass = nd[PT_CD_MASS * nn];
+  const double mass = nd[PT_ND_MASS];
   double q[6];
-  for (int k = 0; k < 6; k++) q[k] = nd[(PT_CD_Q + k) * nn];
+  for (int k = 0; k < 6; k++) q[k] = nd[PT_ND_Q(k)];
   const double alpha = kEwAlphaFac / L, alpha2 = alpha * alpha;
   const double k4 = kPi * kPi / (alpha2 * L * L);
   const int hr = (int)ceil(kEwHCut);
@@ -243,10 +243,10 @@ ewald_kernel(int64_t n, const double* __restrict__ x, const double* __restrict__
              double* __restrict__ pot) {
   const int64_t i = blockIdx.x * 256ll + threadIdx.x;
   if (i >= n) return;
-  const double mass = nd[PT_CD_MASS * nn];
-  const double cm[3] = {nd[PT_CD_CM * nn], nd[(PT_CD_CM + 1) * nn], nd[(PT_CD_CM + 2) * nn]};
+  const double mass = nd[PT_ND_MASS];
+  const double cm[3] = {nd[PT_ND_CM], nd[PT_ND_CM + 1], nd[PT_ND_CM + 2]};
   double q[6];
-  for (int k = 0; k < 6; k++) q[k] = nd[(PT_CD_Q + k) * nn];
+  for (int k = 0; k < 6; k++) q[k] = nd[PT_ND_Q(k)];
   const double alpha = kEwAlphaFac / L, alpha2 = alpha * alpha;
   const double k1 = kPi / (alpha2 * L * L * L);
   const double ka = 2.0 * alpha / sqrt(kPi);
@@ -382,7 +382,7 @@ __global__ void ewald_hexa_table_kernel(const double* __restrict__ nd, int64_t n
                                         const HexNode* __restrict__ hn, double L,
                                         double* __restrict__ table, int32_t* __restrict__ count) {
   if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  const double mass = nd[PT_CD_MASS * nn];
+  const double mass = nd[PT_ND_MASS];
   Momc M;
   momc_from_reduced(mass, hn[0].h, M);
   const double alpha = kEwAlphaFac / L, alpha2 = alpha * alpha;
@@ -422,8 +422,8 @@ ewald_hexa_kernel(int64_t n, const double* __restrict__ x, const double* __restr
                   double* __restrict__ pot) {
   const int64_t i = blockIdx.x * 256ll + threadIdx.x;
   if (i >= n) return;
-  const double mass = nd[PT_CD_MASS * nn];
-  const double cm[3] = {nd[PT_CD_CM * nn], nd[(PT_CD_CM + 1) * nn], nd[(PT_CD_CM + 2) * nn]};
+  const double mass = nd[PT_ND_MASS];
+  const double cm[3] = {nd[PT_ND_CM], nd[PT_ND_CM + 1], nd[PT_ND_CM + 2]};
   Momc M;
   momc_from_reduced(mass, hn[0].h, M);
   const double Q4xx = 0.5 * (M.xxxx + M.xxyy + M.xxzz), Q4xy = 0.5 * (M.xxxy + M.xyyy + M.xyzz);

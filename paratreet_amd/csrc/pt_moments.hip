@@ -27,141 +27,85 @@
 
 namespace {
 
-struct CData {
-  double radius, soft, mass;
-  double cm[3];
-  double q[6];
-  double lo[3], hi[3];
-  int64_t count;
+// Quad layout of both passes: four neighbouring lanes hold one node, lane
+// l < 3 the l-th coordinate (cm_l, the second moments q_ll and q_{l,l+1 mod 3},
+// the box's l-th faces) and lane 3 the softening (and the node's mass and
+// radius when they are stored).  A merge is then one divide instead of four,
+// the other lanes' differences come by a quad permutation, and records are
+// read and written in 32-byte rows.  The operations on each field, and their
+// order, are those of the reference's expressions.
+constexpr int kNext = 0xC9;  // lane 0 <- 1, 1 <- 2, 2 <- 0, 3 <- 3
+
+struct QuadNode {
+  double v;         // cm_l, or the softening
+  double qd, qo;    // q_ll, q_{l,l+1 mod 3} (lane 3: not used)
+  double lo, hi;    // box faces
+  double mass;      // in every lane
 };
 
-__device__ __forceinline__ void cd_default(CData& d) {
-  d.radius = 0.0;
-  d.soft = 0.0;
-  d.mass = 0.0;
-  for (int k = 0; k < 3; k++) {
-    d.cm[k] = 0.0;
-    d.lo[k] = INFINITY;
-    d.hi[k] = -INFINITY;
-  }
-  for (int k = 0; k < 6; k++) d.q[k] = 0.0;
-  d.count = 0;
+__device__ __forceinline__ QuadNode quad_default() {
+  return QuadNode{0.0, 0.0, 0.0, INFINITY, -INFINITY, 0.0};
 }
 
-__device__ __forceinline__ void cd_store(const CData& d, double* __restrict__ nd, int64_t nn,
-                                         int64_t i) {
-  nd[PT_CD_RADIUS * nn + i] = d.radius;
-  nd[PT_CD_SOFT * nn + i] = d.soft;
-  nd[PT_CD_MASS * nn + i] = d.mass;
-  for (int k = 0; k < 3; k++) {
-    nd[(PT_CD_CM + k) * nn + i] = d.cm[k];
-    nd[(PT_CD_LO + k) * nn + i] = d.lo[k];
-    nd[(PT_CD_HI + k) * nn + i] = d.hi[k];
-  }
-  for (int k = 0; k < 6; k++) nd[(PT_CD_Q + k) * nn + i] = d.q[k];
+// q += m d d^T for this lane's two components, each product taken in the order
+// m * d_first * d_second of the reference (xy, yz: own first; xz: x first).
+__device__ __forceinline__ void quad_outer(double m, double d, bool swap, double& dd,
+                                           double& od) {
+  const double e = pt_quad_f64<kNext>(d);
+  dd = m * d * d;
+  od = m * (swap ? e : d) * (swap ? d : e);
 }
 
-// MultipoleMoments::operator+=(Particle) (examples/MultipoleMoments.h:275-353).
-__device__ __forceinline__ void mom_add_particle(CData& d, double px, double py, double pz,
-                                                 double pm, double pe) {
+// MultipoleMoments::operator+=(Particle) (examples/MultipoleMoments.h:275-353):
+// a particle of mass pm whose coordinate (lane 3: softening) is pv.
+__device__ __forceinline__ void quad_add_particle(QuadNode& d, double pm, double pv, bool swap) {
   const double m1 = d.mass;
   d.mass += pm;
-  if (d.mass == 0.0) {
-    d.soft = 0.5 * (d.soft + pe);
-    d.cm[0] = 0.5 * (d.cm[0] + px);
-    d.cm[1] = 0.5 * (d.cm[1] + py);
-    d.cm[2] = 0.5 * (d.cm[2] + pz);
-    return;
-  }
-  d.soft = (m1 * d.soft + pm * pe) / d.mass;
-  const double c1[3] = {d.cm[0], d.cm[1], d.cm[2]};
-  const double p[3] = {px, py, pz};
-  for (int k = 0; k < 3; k++) d.cm[k] = (m1 * d.cm[k] + pm * p[k]) / d.mass;
-  double dr[3] = {c1[0] - d.cm[0], c1[1] - d.cm[1], c1[2] - d.cm[2]};
-  d.q[0] += m1 * dr[0] * dr[0];
-  d.q[3] += m1 * dr[1] * dr[1];
-  d.q[5] += m1 * dr[2] * dr[2];
-  d.q[1] += m1 * dr[0] * dr[1];
-  d.q[2] += m1 * dr[0] * dr[2];
-  d.q[4] += m1 * dr[1] * dr[2];
-  for (int k = 0; k < 3; k++) dr[k] = p[k] - d.cm[k];
-  d.q[0] += pm * dr[0] * dr[0];
-  d.q[3] += pm * dr[1] * dr[1];
-  d.q[5] += pm * dr[2] * dr[2];
-  d.q[1] += pm * dr[0] * dr[1];
-  d.q[2] += pm * dr[0] * dr[2];
-  d.q[4] += pm * dr[1] * dr[2];
+  const double old = d.v;
+  const bool none = d.mass == 0.0;
+  d.v = none ? 0.5 * (old + pv) : (m1 * old + pm * pv) / d.mass;
+  double dd, od;
+  quad_outer(m1, old - d.v, swap, dd, od);
+  d.qd = none ? d.qd : d.qd + dd;
+  d.qo = none ? d.qo : d.qo + od;
+  quad_outer(pm, pv - d.v, swap, dd, od);
+  d.qd = none ? d.qd : d.qd + dd;
+  d.qo = none ? d.qo : d.qo + od;
 }
 
-// MultipoleMoments::operator+=(MultipoleMoments) (examples/MultipoleMoments.h:204-271).
-__device__ __forceinline__ void mom_merge(CData& d, const CData& m) {
+// CentroidData::operator+= (examples/CentroidData.h:61-73) with
+// MultipoleMoments::operator+= (examples/MultipoleMoments.h:204-271), without
+// its last step, the radius: no merge reads the radius it sets (a merge into
+// a massless node copies the child's and the next radius overwrites it), so
+// one radius after the merges gives the value of the last one bit for bit.
+__device__ __forceinline__ void quad_merge(QuadNode& d, const QuadNode& c, bool swap) {
+  if (c.lo < d.lo) d.lo = c.lo;
+  if (c.hi > d.hi) d.hi = c.hi;
   const double m1 = d.mass;
-  d.mass += m.mass;
+  d.mass += c.mass;
+  const double old = d.v;
+  const double sum = (m1 * old + c.mass * c.v) / d.mass;
+  double dd, od, cd, co;
+  quad_outer(m1, old - sum, swap, dd, od);
+  quad_outer(c.mass, c.v - sum, swap, cd, co);
   if (d.mass == 0.0) {
-    d.soft = 0.5 * (d.soft + m.soft);
-    for (int k = 0; k < 3; k++) d.cm[k] = 0.5 * (d.cm[k] + m.cm[k]);
-    return;
+    d.v = 0.5 * (old + c.v);
+  } else if (m1 == 0.0) {
+    d.v = c.v;
+    d.qd = c.qd;
+    d.qo = c.qo;
+    d.mass = c.mass;
+  } else if (c.mass != 0.0) {
+    d.v = sum;
+    d.qd = (d.qd + dd) + (c.qd + cd);
+    d.qo = (d.qo + od) + (c.qo + co);
   }
-  if (m1 == 0.0) {
-    d.radius = m.radius;
-    d.soft = m.soft;
-    d.mass = m.mass;
-    for (int k = 0; k < 3; k++) d.cm[k] = m.cm[k];
-    for (int k = 0; k < 6; k++) d.q[k] = m.q[k];
-    return;
-  }
-  if (m.mass == 0.0) return;
-  d.soft = (m1 * d.soft + m.mass * m.soft) / d.mass;
-  const double c1[3] = {d.cm[0], d.cm[1], d.cm[2]};
-  for (int k = 0; k < 3; k++) d.cm[k] = (m1 * d.cm[k] + m.mass * m.cm[k]) / d.mass;
-  double dr[3] = {c1[0] - d.cm[0], c1[1] - d.cm[1], c1[2] - d.cm[2]};
-  d.q[0] += m1 * dr[0] * dr[0];
-  d.q[3] += m1 * dr[1] * dr[1];
-  d.q[5] += m1 * dr[2] * dr[2];
-  d.q[1] += m1 * dr[0] * dr[1];
-  d.q[2] += m1 * dr[0] * dr[2];
-  d.q[4] += m1 * dr[1] * dr[2];
-  for (int k = 0; k < 3; k++) dr[k] = m.cm[k] - d.cm[k];
-  d.q[0] += m.q[0] + m.mass * dr[0] * dr[0];
-  d.q[3] += m.q[3] + m.mass * dr[1] * dr[1];
-  d.q[5] += m.q[5] + m.mass * dr[2] * dr[2];
-  d.q[1] += m.q[1] + m.mass * dr[0] * dr[1];
-  d.q[2] += m.q[2] + m.mass * dr[0] * dr[2];
-  d.q[4] += m.q[4] + m.mass * dr[1] * dr[2];
 }
 
-__device__ __forceinline__ double len3(double x, double y, double z) {
-  return sqrt(x * x + y * y + z * z);
-}
-
-// CentroidData::operator+= (examples/CentroidData.h:61-73) without its last
-// step, the radius (cd_radius): no merge reads the radius it sets (a merge
-// into a massless node copies the child's and the next radius overwrites
-// it), so after a sequence of merges one cd_radius gives the value of the
-// last merge bit for bit.
-__device__ __forceinline__ void cd_merge(CData& d, const CData& c) {
-  for (int k = 0; k < 3; k++) {
-    if (c.lo[k] < d.lo[k]) d.lo[k] = c.lo[k];
-    if (c.hi[k] > d.hi[k]) d.hi[k] = c.hi[k];
-  }
-  mom_merge(d, c);
-  d.count += c.count;
-}
-
-// The radius step of CentroidData::operator+=: calculateRadiusFarthestCorner
-// (examples/MultipoleMoments.h:458-469) when count > 1, else 1.0.
-__device__ __forceinline__ void cd_radius(CData& d) {
-  if (d.count > 1) {
-    double dl[3];
-    for (int k = 0; k < 3; k++) {
-      const double d1 = d.cm[k] - d.lo[k];
-      const double d2 = d.hi[k] - d.cm[k];
-      dl[k] = (d1 > d2 ? d1 : d2);
-    }
-    d.radius = len3(dl[0], dl[1], dl[2]);
-  } else {
-    d.radius = 1.0;
-  }
+// x^2 + y^2 + z^2 over the quad's first three lanes, in every lane.
+__device__ __forceinline__ double quad_len2(double e) {
+  const double s = e * e;
+  return pt_quad_f64<0x00>(s) + pt_quad_f64<0x55>(s) + pt_quad_f64<0xAA>(s);
 }
 
 // The smallest float >= v (v >= 0, finite).
@@ -171,149 +115,109 @@ __device__ __forceinline__ float round_up_f32(double v) {
   return f;
 }
 
-// Writes node i's walk and interaction records from its final CentroidData
-// (the same values a pass over the SoA node table would read back).  Leaves
-// also get their reach and softening bounds (leaf_soft: the largest particle
-// softening) and, when non-empty, their bucket record (bucket index
+// Stores node i's CentroidData and its walk and interaction records from the
+// quad's final values.  Leaves also get their reach and softening bounds
+// (leaf_soft: the largest particle softening, any value in other lanes than
+// 3) and, when non-empty, their bucket record (bucket index
 // bucket_of[begin]).
-__device__ __forceinline__ void pack_node(const PtTree& t, int64_t i, const CData& d,
-                                          double leaf_soft, const PtPackOut& o) {
-  TreeNode a;
-  a.cx = d.cm[0];
-  a.cy = d.cm[1];
-  a.cz = d.cm[2];
-  a.radius = d.radius;
-  a.count = t.count[i];
-  a.first_child = t.first_child[i];
-  a.type = t.type[i];
-  a.begin = t.begin[i];
-  a.leaf_reach = 0.f;
-  a.leaf_soft = 0.f;
-  a.node_soft = a.type == PT_NODE_INTERNAL ? round_up_f32(d.soft) : 0.f;
-  if (a.type == PT_NODE_LEAF) {
-    double r2 = 0.0;
-    for (int k = 0; k < 3; k++) {
-      const double d1 = d.cm[k] - d.lo[k];
-      const double d2 = d.hi[k] - d.cm[k];
-      const double e = d1 > d2 ? d1 : d2;
-      r2 += e * e;
-    }
-    a.leaf_reach = round_up_f32(sqrt(r2));
-    a.leaf_soft = round_up_f32(leaf_soft);
-  }
-  a.pad = 0;
-  o.tnode[i] = a;
-  GravNode g;
-  g.cx = d.cm[0];
-  g.cy = d.cm[1];
-  g.cz = d.cm[2];
-  g.mass = d.mass;
-  g.soft = d.soft;
-  g.qxx = d.q[0];
-  g.qxy = d.q[1];
-  g.qxz = d.q[2];
-  g.qyy = d.q[3];
-  g.qyz = d.q[4];
-  g.qzz = d.q[5];
-  g.tr = 0.5 * (g.qxx + g.qyy + g.qzz);
-  o.gn[i] = g;
-  GravNode32 h;
-  h.cx = g.cx;
-  h.cy = g.cy;
-  h.cz = g.cz;
-  h.soft64 = g.soft;
-  h.mass = (float)g.mass;
-  h.soft = (float)g.soft;
-  h.qxx = (float)g.qxx;
-  h.qxy = (float)g.qxy;
-  h.qxz = (float)g.qxz;
-  h.qyy = (float)g.qyy;
-  h.qyz = (float)g.qyz;
-  h.qzz = (float)g.qzz;
-  o.gn32[i] = h;
-  if (a.type == PT_NODE_LEAF && a.count > 0) {
-    Bucket b;
-    b.lox = d.lo[0];
-    b.loy = d.lo[1];
-    b.loz = d.lo[2];
-    b.hix = d.hi[0];
-    b.hiy = d.hi[1];
-    b.hiz = d.hi[2];
-    b.cx = d.cm[0];
-    b.cy = d.cm[1];
-    b.cz = d.cm[2];
-    b.soft = d.soft;
-    b.pad0 = 0.0;
-    b.pad1 = 0.0;
-    b.node = (int32_t)i;
-    b.begin = a.begin;
-    b.count = a.count;
-    b.pad2 = 0;
-    o.bk[o.bucket_of[a.begin]] = b;
+__device__ __forceinline__ void quad_store(const PtTree& t, int64_t i, int l, const QuadNode& d,
+                                           double radius, double leaf_soft,
+                                           double* __restrict__ nd, const PtPackOut& o) {
+  const double qxx = pt_quad_f64<0x00>(d.qd), qyy = pt_quad_f64<0x55>(d.qd),
+               qzz = pt_quad_f64<0xAA>(d.qd);
+  double* r = nd + i * PT_ND_STRIDE;
+  r[l] = d.v;
+  r[4 + l] = l < 3 ? d.qd : d.mass;
+  r[8 + l] = l < 3 ? d.qo : radius;
+  r[12 + l] = l < 3 ? d.lo : 0.0;
+  r[16 + l] = l < 3 ? d.hi : 0.0;
+  const int32_t count = t.count[i], type = t.type[i], begin = t.begin[i];
+  const double d1 = d.v - d.lo, d2 = d.hi - d.v;
+  const double reach2 = quad_len2(d1 > d2 ? d1 : d2);
+  // TreeNode: {cx, cy, cz, radius} then {count, first_child} {type, begin}
+  // {leaf_reach, leaf_soft} {node_soft, pad}, one 8-byte piece per lane
+  double* a = reinterpret_cast<double*>(o.tnode + i);
+  a[l] = l < 3 ? d.v : radius;
+  int2 w;
+  if (l == 0) w = make_int2(count, t.first_child[i]);
+  if (l == 1) w = make_int2(type, begin);
+  const bool leaf = type == PT_NODE_LEAF;
+  const float ls = __int_as_float(
+      pt_quad_i32<0xFF>(__float_as_int(leaf ? round_up_f32(leaf_soft) : 0.f)));
+  if (l == 2)
+    w = make_int2(__float_as_int(leaf ? round_up_f32(sqrt(reach2)) : 0.f), __float_as_int(ls));
+  if (l == 3)
+    w = make_int2(__float_as_int(type == PT_NODE_INTERNAL ? round_up_f32(d.v) : 0.f), 0);
+  reinterpret_cast<int2*>(o.tnode + i)[4 + l] = w;
+  double* g = reinterpret_cast<double*>(o.gn + i);
+  g[l] = d.v;
+  g[4 + l] = l < 3 ? d.qd : d.mass;
+  g[8 + l] = l < 3 ? d.qo : 0.5 * (qxx + qyy + qzz);
+  // GravNode32: centre and softening, then {qxx qxy} {qyy qyz} {qzz qxz} {mass soft}
+  reinterpret_cast<double*>(o.gn32 + i)[l] = d.v;
+  reinterpret_cast<float2*>(o.gn32 + i)[4 + l] =
+      make_float2((float)(l < 3 ? d.qd : d.mass), (float)(l < 3 ? d.qo : d.v));
+  if (leaf && count > 0) {
+    double* b = reinterpret_cast<double*>(o.bk + o.bucket_of[begin]);
+    b[l] = l < 3 ? d.lo : 0.0;
+    b[4 + l] = l < 3 ? d.hi : 0.0;
+    b[8 + l] = d.v;
+    if (l < 2)
+      reinterpret_cast<int2*>(b + 12)[l] = l == 0 ? make_int2((int)i, begin) : make_int2(count, 0);
   }
 }
 
-// One particle of the CentroidData leaf constructor: moments, box, and the
-// largest softening.
-__device__ __forceinline__ void leaf_add(CData& d, double& smax, double px, double py, double pz,
-                                         double pm, double pe) {
-  smax = pe > smax ? pe : smax;
-  mom_add_particle(d, px, py, pz, pm, pe);
-  const double p[3] = {px, py, pz};
-  for (int k = 0; k < 3; k++) {
-    if (p[k] < d.lo[k]) d.lo[k] = p[k];
-    if (p[k] > d.hi[k]) d.hi[k] = p[k];
-  }
-}
+static_assert(sizeof(TreeNode) == 64 && sizeof(GravNode) == 96 && sizeof(GravNode32) == 64 &&
+                  sizeof(Bucket) == 128,
+              "record layouts written by quad_store");
 
-// One thread per node: a leaf runs the sequential particle recurrence of the
-// CentroidData leaf constructor in sorted particle order; an empty leaf stores
-// the default CentroidData; internal nodes are left to the upward pass.  The
-// node's walk/interaction records (and a leaf's bucket record) follow.
+// A quad per node: a leaf runs the sequential particle recurrence of the
+// CentroidData leaf constructor (examples/CentroidData.h:41-59) in sorted
+// particle order; an empty leaf stores the default CentroidData; internal
+// nodes are left to the upward pass.  Bound by the recurrence's chain of
+// dependent divides, one per particle; its inputs are loaded kPre particles
+// ahead.
 __global__ void __launch_bounds__(256)
 leaf_kernel(const PtTree t, int64_t nn, const double* __restrict__ x,
             const double* __restrict__ y, const double* __restrict__ z,
             const double* __restrict__ m, const double* __restrict__ e, double* __restrict__ nd,
             const PtPackOut o) {
-  const int64_t id = blockIdx.x * 256ll + threadIdx.x;
+  const int64_t id = blockIdx.x * 64ll + (threadIdx.x >> 2);
+  const int l = threadIdx.x & 3;
   if (id >= nn) return;
   const int ty = t.type[id];
   if (ty == PT_NODE_INTERNAL) return;
-  CData d;
-  cd_default(d);
-  double smax = 0.0;
+  const bool swap = l == 2;
+  QuadNode d = quad_default();
+  double radius = 0.0, smax = 0.0;
   if (ty == PT_NODE_LEAF) {
     const int64_t b = t.begin[id];
-    const int64_t n = t.count[id];
-    // the first kLeafPre particles' inputs are loaded together, then added
-    // in order (the same sequence as one at a time, without a memory round
-    // trip per particle)
-    constexpr int kLeafPre = 16;
-    double qx[kLeafPre], qy[kLeafPre], qz[kLeafPre], qm[kLeafPre], qe[kLeafPre];
+    const int32_t n = t.count[id];
+    const double* __restrict__ mine = l == 0 ? x : l == 1 ? y : l == 2 ? z : e;
+    constexpr int kPre = 8;
+    for (int32_t k0 = 0; k0 < n; k0 += kPre) {
+      double pv[kPre], pm[kPre];
 #pragma unroll
-    for (int k = 0; k < kLeafPre; k++) {
-      if (k < n) {
-        qx[k] = x[b + k];
-        qy[k] = y[b + k];
-        qz[k] = z[b + k];
-        qm[k] = m[b + k];
-        qe[k] = e[b + k];
+      for (int k = 0; k < kPre; k++) {
+        if (k0 + k < n) {
+          pv[k] = mine[b + k0 + k];
+          pm[k] = m[b + k0 + k];
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < kPre; k++) {
+        if (k0 + k < n) {
+          quad_add_particle(d, pm[k], pv[k], swap);
+          if (pv[k] < d.lo) d.lo = pv[k];
+          if (pv[k] > d.hi) d.hi = pv[k];
+          smax = pv[k] > smax ? pv[k] : smax;
+        }
       }
     }
-#pragma unroll
-    for (int k = 0; k < kLeafPre; k++) {
-      if (k < n) leaf_add(d, smax, qx[k], qy[k], qz[k], qm[k], qe[k]);
-    }
-    for (int64_t i = b + kLeafPre; i < b + n; i++) leaf_add(d, smax, x[i], y[i], z[i], m[i], e[i]);
-    d.count = n;
-    if (d.count > 1) {
-      d.radius = 0.5 * len3(d.hi[0] - d.lo[0], d.hi[1] - d.lo[1], d.hi[2] - d.lo[2]);
-    } else {
-      d.radius = 1.0;
-    }
+    // calculateRadiusBox (examples/MultipoleMoments.h:473-482)
+    radius = n > 1 ? 0.5 * sqrt(quad_len2(d.hi - d.lo)) : 1.0;
   }
-  cd_store(d, nd, nn, id);
-  pack_node(t, id, d, smax, o);
+  quad_store(t, id, l, d, radius, smax, nd, o);
 }
 
 __device__ __forceinline__ uint64_t left_align(uint64_t k) {
@@ -321,146 +225,164 @@ __device__ __forceinline__ uint64_t left_align(uint64_t k) {
   return k << (PT_KEY_BITS - (3 * depth + 1));
 }
 
-// One internal node (its children are final).  The children's pop order is
-// built in registers (fully unrolled loops over the 8 children, the order
-// packed as 8 nibbles) so nothing spills to scratch.
-// A child's CentroidData fields as the merge reads them: soft mass cm[3]
-// q[6] lo[3] hi[3] (its radius is not used: the merge recomputes it).
-constexpr int kUpFields = 17;
-constexpr int kUpThreads = 64;  // threads (= parents) per work-group of the upward pass
-
-// The thread's 8 children's fields are first loaded together into its LDS
-// slab (every load in flight at once), then merged from there.
-__device__ __forceinline__ void upward_node(const PtTree& t, int32_t p, double* __restrict__ nd,
-                                            int64_t nn, int32_t* __restrict__ ord_h,
-                                            uint64_t* __restrict__ ord_b,
-                                            double (*__restrict__ slab)[kUpFields],
-                                            const PtPackOut& o) {
-  const int32_t fc = t.first_child[p];
-  // every child's fields, type and order keys are loaded in one phase (an
-  // empty child's stored defaults and a leaf's order keys are not used)
-#pragma unroll
-  for (int c = 0; c < 8; c++) {
-    const int64_t ch = fc + c;
-    slab[c][0] = nd[PT_CD_SOFT * nn + ch];
-    slab[c][1] = nd[PT_CD_MASS * nn + ch];
-#pragma unroll
-    for (int k = 0; k < 3; k++) slab[c][2 + k] = nd[(PT_CD_CM + k) * nn + ch];
-#pragma unroll
-    for (int k = 0; k < 6; k++) slab[c][5 + k] = nd[(PT_CD_Q + k) * nn + ch];
-#pragma unroll
-    for (int k = 0; k < 3; k++) slab[c][11 + k] = nd[(PT_CD_LO + k) * nn + ch];
-#pragma unroll
-    for (int k = 0; k < 3; k++) slab[c][14 + k] = nd[(PT_CD_HI + k) * nn + ch];
-  }
-  int ctype[8];
-  int32_t h[8];
-  uint64_t b[8];
-  uint64_t ckey[8];
-  int n_leaf = 0, n_empty = 0;
-#pragma unroll
-  for (int c = 0; c < 8; c++) {
-    ctype[c] = t.type[fc + c];
-    ckey[c] = t.key[fc + c];
-    const int32_t hc = ord_h[fc + c];
-    const uint64_t bc = ord_b[fc + c];
-    h[c] = ctype[c] == PT_NODE_INTERNAL ? hc : -1;
-    b[c] = ctype[c] == PT_NODE_INTERNAL ? bc : 0;
-    n_leaf += ctype[c] == PT_NODE_LEAF;
-    n_empty += ctype[c] == PT_NODE_EMPTY;
-  }
-  // position of every child in the pop order: non-empty leaves, empty leaves
-  // (each in child order), then internal children ascending in (h, b)
-  uint32_t order = 0;
-  int32_t hmax = -1;
-  uint64_t bmax = 0;
-  int k_leaf = 0, k_empty = 0;
-#pragma unroll
-  for (int c = 0; c < 8; c++) {
-    int pos;
-    if (ctype[c] == PT_NODE_LEAF) {
-      pos = k_leaf++;
-    } else if (ctype[c] == PT_NODE_EMPTY) {
-      pos = n_leaf + k_empty++;
-    } else {
-      int rank = 0;
-#pragma unroll
-      for (int o = 0; o < 8; o++) {
-        const bool before = ctype[o] == PT_NODE_INTERNAL &&
-                            (h[o] < h[c] || (h[o] == h[c] && b[o] < b[c]));
-        rank += before ? 1 : 0;
-      }
-      pos = n_leaf + n_empty + rank;
-      if (h[c] > hmax || (h[c] == hmax && b[c] > bmax)) {
-        hmax = h[c];
-        bmax = b[c];
-      }
-    }
-    order |= (uint32_t)c << (4 * pos);
-  }
-  if (hmax < 0) {
-    // frontier node: h = 0, b = rank of the last-popped leaf child
-    uint64_t bl = 0;
-#pragma unroll
-    for (int c = 0; c < 8; c++) {
-      uint64_t r = left_align(ckey[c]) >> 1;
-      if (ctype[c] == PT_NODE_EMPTY) r |= (1ull << 63);
-      bl = r > bl ? r : bl;
-    }
-    ord_h[p] = 0;
-    ord_b[p] = bl;
-  } else {
-    ord_h[p] = hmax + 1;
-    ord_b[p] = bmax;
-  }
-  // the parent starts from the default CentroidData; an empty child is the
-  // default too and is not read
-  CData d;
-  cd_default(d);
-  for (int j = 0; j < 8; j++) {
-    const int c = (order >> (4 * j)) & 15;
-    CData cd;
-    cd_default(cd);
-    if (ctype[c] != PT_NODE_EMPTY) {
-      const double* f = slab[c];
-      cd.soft = f[0];
-      cd.mass = f[1];
-      for (int k = 0; k < 3; k++) cd.cm[k] = f[2 + k];
-      for (int k = 0; k < 6; k++) cd.q[k] = f[5 + k];
-      for (int k = 0; k < 3; k++) cd.lo[k] = f[11 + k];
-      for (int k = 0; k < 3; k++) cd.hi[k] = f[14 + k];
-      cd.count = t.count[fc + c];
-    }
-    cd_merge(d, cd);
-  }
-  cd_radius(d);
-  cd_store(d, nd, nn, p);
-  pack_node(t, p, d, 0.0, o);
+__device__ __forceinline__ unsigned quad_or(unsigned v) {
+  v |= (unsigned)pt_quad_i32<0xB1>((int)v);
+  return v | (unsigned)pt_quad_i32<0x4E>((int)v);
 }
 
-// One thread per internal node of one level (deepest level first).
+// The larger of (h, b) and the CTRL-permuted lane's, lexicographically.
+template <int CTRL>
+__device__ __forceinline__ void quad_max_hb(int32_t& h, uint64_t& b) {
+  const int32_t oh = pt_quad_i32<CTRL>(h);
+  const uint64_t ob = pt_quad_u64<CTRL>(b);
+  if (oh > h || (oh == h && ob > b)) {
+    h = oh;
+    b = ob;
+  }
+}
+
+// Children of child index O's lane among a lane's two: the internal ones that
+// come before (h, b) are counted into rank[].
+template <int O>
+__device__ __forceinline__ void quad_rank(const int32_t (&h)[2], const uint64_t (&b)[2],
+                                          int (&rank)[2]) {
+  constexpr int bc = (O >> 1) * 0x55;
+  const int32_t oh = pt_quad_i32<bc>(h[O & 1]);
+  const uint64_t ob = pt_quad_u64<bc>(b[O & 1]);
+#pragma unroll
+  for (int j = 0; j < 2; j++)
+    rank[j] += oh >= 0 && (oh < h[j] || (oh == h[j] && ob < b[j])) ? 1 : 0;
+}
+
+// One internal node per quad, its children final.  Lane l finds the pop
+// positions of children 2 l and 2 l + 1; then every lane loads its column of
+// the 8 children's records in pop order, all in flight at once, and merges
+// them in that order.
+__device__ __forceinline__ void upward_node(const PtTree& t, int32_t p, int l,
+                                            double* __restrict__ nd, int32_t* __restrict__ ord_h,
+                                            uint64_t* __restrict__ ord_b, const PtPackOut& o) {
+  const int64_t fc = t.first_child[p];
+  int ctype[2];
+  int32_t h[2];
+  uint64_t b[2], ckey[2];
+#pragma unroll
+  for (int j = 0; j < 2; j++) {
+    const int64_t ch = fc + 2 * l + j;
+    ctype[j] = t.type[ch];
+    ckey[j] = t.key[ch];
+    h[j] = ord_h[ch];
+    b[j] = ord_b[ch];
+  }
+  unsigned leafm = 0, emptym = 0;
+#pragma unroll
+  for (int j = 0; j < 2; j++) {
+    const bool inner = ctype[j] == PT_NODE_INTERNAL;
+    h[j] = inner ? h[j] : -1;
+    b[j] = inner ? b[j] : 0;
+    leafm |= (ctype[j] == PT_NODE_LEAF ? 1u : 0u) << (2 * l + j);
+    emptym |= (ctype[j] == PT_NODE_EMPTY ? 1u : 0u) << (2 * l + j);
+  }
+  leafm = quad_or(leafm);
+  emptym = quad_or(emptym);
+  const int n_leaf = __popc(leafm), n_first = n_leaf + __popc(emptym);
+  int rank[2] = {0, 0};
+  if (__ballot(n_first < 8) != 0ull) {
+    quad_rank<0>(h, b, rank);
+    quad_rank<1>(h, b, rank);
+    quad_rank<2>(h, b, rank);
+    quad_rank<3>(h, b, rank);
+    quad_rank<4>(h, b, rank);
+    quad_rank<5>(h, b, rank);
+    quad_rank<6>(h, b, rank);
+    quad_rank<7>(h, b, rank);
+  }
+  unsigned order = 0;
+  int32_t hmax = -1;
+  uint64_t bmax = 0, bleaf = 0;
+#pragma unroll
+  for (int j = 0; j < 2; j++) {
+    const int c = 2 * l + j;
+    const unsigned below = (1u << c) - 1u;
+    const int pos = ctype[j] == PT_NODE_LEAF    ? __popc(leafm & below)
+                    : ctype[j] == PT_NODE_EMPTY ? n_leaf + __popc(emptym & below)
+                                                : n_first + rank[j];
+    order |= (unsigned)c << (4 * pos);
+    if (h[j] > hmax || (h[j] == hmax && b[j] > bmax)) {
+      hmax = h[j];
+      bmax = b[j];
+    }
+    uint64_t r = left_align(ckey[j]) >> 1;
+    if (ctype[j] == PT_NODE_EMPTY) r |= 1ull << 63;
+    bleaf = r > bleaf ? r : bleaf;
+  }
+  order = quad_or(order);
+  if (n_first < 8) {
+    quad_max_hb<0xB1>(hmax, bmax);
+    quad_max_hb<0x4E>(hmax, bmax);
+    hmax++;
+  } else {
+    // frontier node: h = 0, b = rank of the last-popped leaf child
+    hmax = 0;
+    bmax = bleaf;
+    quad_max_hb<0xB1>(hmax, bmax);
+    quad_max_hb<0x4E>(hmax, bmax);
+  }
+  if (l == 0) {
+    ord_h[p] = hmax;
+    ord_b[p] = bmax;
+  }
+  double row[8][5];
+#pragma unroll
+  for (int j = 0; j < 8; j++) {
+    const double* r = nd + (fc + ((order >> (4 * j)) & 15u)) * PT_ND_STRIDE + l;
+#pragma unroll
+    for (int k = 0; k < 5; k++) row[j][k] = r[4 * k];
+  }
+  const bool swap = l == 2;
+  QuadNode d = quad_default();
+#pragma unroll
+  for (int j = 0; j < 8; j++) {
+    QuadNode c{row[j][0], row[j][1], row[j][2], row[j][3], row[j][4],
+               pt_quad_f64<0xFF>(row[j][1])};
+    quad_merge(d, c, swap);
+  }
+  // calculateRadiusFarthestCorner (examples/MultipoleMoments.h:458-469); an
+  // internal node holds more than one particle
+  const double d1 = d.v - d.lo, d2 = d.hi - d.v;
+  const double radius = sqrt(quad_len2(d1 > d2 ? d1 : d2));
+  quad_store(t, p, l, d, radius, 0.0, nd, o);
+}
+
+// A quad per internal node of one level (deepest level first).  Latency bound:
+// two dependent loads, then eight merges of one divide each, 7.5 us a level at
+// 1M particles.  One thread per node took 18 us on a level of any size (168
+// scattered 8-byte loads per thread, then 8 x 4 divides); with the leaves' 52
+// -> 41 us and the small levels' run 64 -> 23 us (1k particles) the evaluation
+// went from 3031 to 2950 us at 1M and from 337 to 271 at 1k.
+constexpr int kUpThreads = 64;
+
 __global__ void __launch_bounds__(kUpThreads)
 upward_kernel(const PtTree t, const int32_t* __restrict__ level_nodes, int32_t nl,
-              double* __restrict__ nd, int64_t nn, int32_t* __restrict__ ord_h,
-              uint64_t* __restrict__ ord_b, const PtPackOut o) {
-  __shared__ double slab[kUpThreads][8][kUpFields];
-  const int64_t li = (int64_t)blockIdx.x * kUpThreads + threadIdx.x;
+              double* __restrict__ nd, int32_t* __restrict__ ord_h, uint64_t* __restrict__ ord_b,
+              const PtPackOut o) {
+  const int64_t li = (int64_t)blockIdx.x * (kUpThreads / 4) + (threadIdx.x >> 2);
   if (li >= nl) return;
-  upward_node(t, level_nodes[li], nd, nn, ord_h, ord_b, slab[threadIdx.x], o);
+  upward_node(t, level_nodes[li], threadIdx.x & 3, nd, ord_h, ord_b, o);
 }
 
 // A run of consecutive small levels in one work-group, deepest first, with a
 // work-group barrier between levels (a level reads what the one below wrote;
 // all waves of the group share the CU's caches).
-__global__ void __launch_bounds__(kUpThreads)
+constexpr int kRunThreads = 1024;
+
+__global__ void __launch_bounds__(kRunThreads)
 upward_run_kernel(const PtTree t, const int32_t* __restrict__ level_nodes, PtLevelRun run,
-                  double* __restrict__ nd, int64_t nn, int32_t* __restrict__ ord_h,
+                  double* __restrict__ nd, int32_t* __restrict__ ord_h,
                   uint64_t* __restrict__ ord_b, const PtPackOut o) {
-  __shared__ double slab[kUpThreads][8][kUpFields];
   for (int k = 0; k < run.nlev; k++) {
     const int32_t off = run.off[k], cnt = run.cnt[k];
-    for (int32_t li = threadIdx.x; li < cnt; li += kUpThreads)
-      upward_node(t, level_nodes[off + li], nd, nn, ord_h, ord_b, slab[threadIdx.x], o);
+    for (int32_t li = threadIdx.x >> 2; li < cnt; li += blockDim.x / 4)
+      upward_node(t, level_nodes[off + li], threadIdx.x & 3, nd, ord_h, ord_b, o);
     __syncthreads();
   }
 }
@@ -510,9 +432,9 @@ hexa_leaf_kernel(const PtTree t, const int32_t* __restrict__ bucket_node, int64_
                  const double* __restrict__ nd, int64_t nn, double* __restrict__ raw) {
   const int64_t bi = blockIdx.x * 256ll + threadIdx.x;
   if (bi >= nb) return;
-  const int32_t id = bucket_node[bi];
-  const double cx = nd[(PT_CD_CM + 0) * nn + id], cy = nd[(PT_CD_CM + 1) * nn + id],
-               cz = nd[(PT_CD_CM + 2) * nn + id];
+  const int64_t id = bucket_node[bi];
+  const double cx = nd[id * PT_ND_STRIDE + PT_ND_CM + 0], cy = nd[id * PT_ND_STRIDE + PT_ND_CM + 1],
+               cz = nd[id * PT_ND_STRIDE + PT_ND_CM + 2];
   double r[PT_HEXA_RAW];
 #pragma unroll
   for (int k = 0; k < PT_HEXA_RAW; k++) r[k] = 0.0;
@@ -544,7 +466,7 @@ __device__ __forceinline__ double hx_child(const double* __restrict__ nd,
                                            int64_t ch, double mass, int i, int j, int k) {
   const int l = i + j + k;
   if (l == 0) return mass;
-  if (l == 2) return nd[(PT_CD_Q + hx_index(2, i, j)) * nn + ch];
+  if (l == 2) return nd[ch * PT_ND_STRIDE + PT_ND_Q(hx_index(2, i, j))];
   if (l == 3) return raw[hx_index(3, i, j) * nn + ch];
   return raw[(10 + hx_index(4, i, j)) * nn + ch];
 }
@@ -556,23 +478,23 @@ hexa_up_kernel(const PtTree t, const int32_t* __restrict__ level_nodes, int32_t 
                const double* __restrict__ nd, int64_t nn, double* __restrict__ raw) {
   const int64_t li = blockIdx.x * 256ll + threadIdx.x;
   if (li >= nl) return;
-  const int32_t p = level_nodes[li];
+  const int64_t p = level_nodes[li];
   double r[PT_HEXA_RAW];
 #pragma unroll
   for (int k = 0; k < PT_HEXA_RAW; k++) r[k] = 0.0;
-  const double pmass = nd[PT_CD_MASS * nn + p];
+  const double pmass = nd[p * PT_ND_STRIDE + PT_ND_MASS];
   if (pmass != 0.0) {
-    const double pc[3] = {nd[(PT_CD_CM + 0) * nn + p], nd[(PT_CD_CM + 1) * nn + p],
-                          nd[(PT_CD_CM + 2) * nn + p]};
+    const double pc[3] = {nd[p * PT_ND_STRIDE + PT_ND_CM + 0], nd[p * PT_ND_STRIDE + PT_ND_CM + 1],
+                          nd[p * PT_ND_STRIDE + PT_ND_CM + 2]};
     const int32_t fc = t.first_child[p];
     for (int c = 0; c < 8; c++) {
       const int64_t ch = fc + c;
-      const double cm = nd[PT_CD_MASS * nn + ch];
+      const double cm = nd[ch * PT_ND_STRIDE + PT_ND_MASS];
       if (cm == 0.0) continue;
       double px[5], py[5], pz[5];
-      hx_pow(nd[(PT_CD_CM + 0) * nn + ch] - pc[0], px);
-      hx_pow(nd[(PT_CD_CM + 1) * nn + ch] - pc[1], py);
-      hx_pow(nd[(PT_CD_CM + 2) * nn + ch] - pc[2], pz);
+      hx_pow(nd[ch * PT_ND_STRIDE + PT_ND_CM + 0] - pc[0], px);
+      hx_pow(nd[ch * PT_ND_STRIDE + PT_ND_CM + 1] - pc[1], py);
+      hx_pow(nd[ch * PT_ND_STRIDE + PT_ND_CM + 2] - pc[2], pz);
 #pragma unroll
       for (int l = 3; l <= 4; l++)
 #pragma unroll
@@ -612,7 +534,7 @@ hexa_pack_kernel(const PtTree t, const double* __restrict__ nd, const double* __
   for (int k = 0; k < PT_HEXA_RAW; k++) r[k] = ty == PT_NODE_EMPTY ? 0.0 : raw[k * nn + i];
   double q[6];
 #pragma unroll
-  for (int k = 0; k < 6; k++) q[k] = nd[(PT_CD_Q + k) * nn + i];
+  for (int k = 0; k < 6; k++) q[k] = nd[i * PT_ND_STRIDE + PT_ND_Q(k)];
 #define R3(a, b) r[hx_index(3, a, b)]
 #define R4(a, b) r[10 + hx_index(4, a, b)]
   const double tr = q[0] + q[3] + q[5];
@@ -627,11 +549,11 @@ hexa_pack_kernel(const PtTree t, const double* __restrict__ nd, const double* __
   const double tyz = R4(2, 1) + R4(0, 3) + R4(0, 1);
   const double ss = txx + tyy + tzz;
   HexNode h;
-  h.cx = nd[(PT_CD_CM + 0) * nn + i];
-  h.cy = nd[(PT_CD_CM + 1) * nn + i];
-  h.cz = nd[(PT_CD_CM + 2) * nn + i];
-  h.mass = nd[PT_CD_MASS * nn + i];
-  h.soft = nd[PT_CD_SOFT * nn + i];
+  h.cx = nd[i * PT_ND_STRIDE + PT_ND_CM + 0];
+  h.cy = nd[i * PT_ND_STRIDE + PT_ND_CM + 1];
+  h.cz = nd[i * PT_ND_STRIDE + PT_ND_CM + 2];
+  h.mass = nd[i * PT_ND_STRIDE + PT_ND_MASS];
+  h.soft = nd[i * PT_ND_STRIDE + PT_ND_SOFT];
   h.h[0] = q[0] - tr * (1.0 / 3.0);
   h.h[1] = q[3] - tr * (1.0 / 3.0);
   h.h[2] = q[1];
@@ -659,12 +581,12 @@ hexa_pack_kernel(const PtTree t, const double* __restrict__ nd, const double* __
   for (int k = 0; k < 6; k++) h.pad[k] = 0.0;
   hn[i] = h;
   HexOpen o;
-  o.lox = nd[(PT_CD_LO + 0) * nn + i];
-  o.loy = nd[(PT_CD_LO + 1) * nn + i];
-  o.loz = nd[(PT_CD_LO + 2) * nn + i];
-  o.hix = nd[(PT_CD_HI + 0) * nn + i];
-  o.hiy = nd[(PT_CD_HI + 1) * nn + i];
-  o.hiz = nd[(PT_CD_HI + 2) * nn + i];
+  o.lox = nd[i * PT_ND_STRIDE + PT_ND_LO + 0];
+  o.loy = nd[i * PT_ND_STRIDE + PT_ND_LO + 1];
+  o.loz = nd[i * PT_ND_STRIDE + PT_ND_LO + 2];
+  o.hix = nd[i * PT_ND_STRIDE + PT_ND_HI + 0];
+  o.hiy = nd[i * PT_ND_STRIDE + PT_ND_HI + 1];
+  o.hiz = nd[i * PT_ND_STRIDE + PT_ND_HI + 2];
   o.soft = h.soft;
   o.pad = 0.0;
   ho[i] = o;
@@ -678,24 +600,27 @@ int pt_launch_leaf_moments(const PtTree& t, int64_t nn, const double* x, const d
                            const double* z, const double* m, const double* e, double* nd,
                            const PtPackOut& o, hipStream_t s) {
   if (nn <= 0) return 0;
-  leaf_kernel<<<grid_for(nn), 256, 0, s>>>(t, nn, x, y, z, m, e, nd, o);
+  leaf_kernel<<<(unsigned)((nn + 63) / 64), 256, 0, s>>>(t, nn, x, y, z, m, e, nd, o);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
 int pt_launch_upward_run(const PtTree& t, const int32_t* level_nodes, const PtLevelRun& run,
-                         double* nd, int64_t nn, int32_t* ord_h, uint64_t* ord_b,
-                         const PtPackOut& o, hipStream_t s) {
+                         double* nd, int32_t* ord_h, uint64_t* ord_b, const PtPackOut& o,
+                         hipStream_t s) {
   if (run.nlev <= 0) return 0;
-  upward_run_kernel<<<1, kUpThreads, 0, s>>>(t, level_nodes, run, nd, nn, ord_h, ord_b, o);
+  int32_t most = 0;
+  for (int k = 0; k < run.nlev; k++) most = run.cnt[k] > most ? run.cnt[k] : most;
+  const int threads = most >= kRunThreads / 4 ? kRunThreads : (most * 4 + 63) / 64 * 64;
+  upward_run_kernel<<<1, threads, 0, s>>>(t, level_nodes, run, nd, ord_h, ord_b, o);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
 int pt_launch_upward_level(const PtTree& t, const int32_t* level_nodes, int32_t nl, double* nd,
-                           int64_t nn, int32_t* ord_h, uint64_t* ord_b, const PtPackOut& o,
-                           hipStream_t s) {
+                           int32_t* ord_h, uint64_t* ord_b, const PtPackOut& o, hipStream_t s) {
   if (nl <= 0) return 0;
-  upward_kernel<<<(unsigned)((nl + kUpThreads - 1) / kUpThreads), kUpThreads, 0, s>>>(
-      t, level_nodes, nl, nd, nn, ord_h, ord_b, o);
+  constexpr int per = kUpThreads / 4;
+  upward_kernel<<<(unsigned)((nl + per - 1) / per), kUpThreads, 0, s>>>(t, level_nodes, nl, nd,
+                                                                        ord_h, ord_b, o);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

@@ -3,13 +3,14 @@ of one wave chunk and of one wave tile give or take a particle, buckets of one
 particle and larger than the set, keys shared by more particles than a bucket
 holds, a chain of single-child levels (far more internal nodes than the tables
 first hold), and the last key cell.  Node set, ranges, links and buckets are
-equal, from the full sort and from a top-bits one."""
+equal, from the full sort and from a top-bits one, and so are the nodes'
+moments bit for bit, massless particles, leaves and subtrees included."""
 import numpy as np
 import pytest
 
 from oracle import oracle as O
 from paratreet_amd import ics
-from tests.helpers import rel_err
+from tests.helpers import bits, oracle_node_data, rel_err
 
 pytestmark = pytest.mark.gpu
 
@@ -46,7 +47,11 @@ def test_tree_matches_oracle(kind, n, bucket):
     from paratreet_amd.gravity import Configuration, Driver
     pos = {"plummer": lambda: ics.plummer(n, seed=70 + bucket)[0], "chain": lambda: _chain(n),
            "shared": lambda: _shared_keys(n), "corner": lambda: _corner(n)}[kind]()
-    m, e = np.full(n, 1.0 / n), np.full(n, 0.01)
+    rng = np.random.default_rng(n + bucket)
+    m, e = rng.uniform(0.5, 1.5, n) / n, rng.uniform(0.005, 0.02, n)
+    weight = m.copy()
+    if n > 60:
+        m[pos[:, 0] > np.quantile(pos[:, 0], 0.7)] = 0.0
     P = O.Pipeline(pos, m, e, bucket=bucket, theta=0.7)
     d = Driver(Configuration(max_particles_per_leaf=bucket))
     d.load(pos, m, e)
@@ -59,7 +64,7 @@ def test_tree_matches_oracle(kind, n, bucket):
             d.assign_keys()
             d.build_tree()
         else:
-            cnt = d.compute_forces(theta=0.7, precision=0)
+            d.compute_forces(theta=0.7, precision=0)
         g = d.nodes()
         at = np.array([onodes[int(k)] for k in g["key"]])
         assert len(at) == len(P.nodes) and len(np.unique(at)) == len(at)
@@ -75,6 +80,10 @@ def test_tree_matches_oracle(kind, n, bucket):
         sk, perm = d.sorted()
         assert np.array_equal(sk, P.sorted_keys)
         assert np.array_equal(perm.astype(np.int64), P.perm.astype(np.int64))
+        assert np.array_equal(bits(d.node_data()), bits(oracle_node_data(P)[at]))
+    P = O.Pipeline(pos, weight, e, bucket=bucket, theta=0.7)
+    d.load(pos, weight, e)
+    cnt = d.compute_forces(theta=0.7, precision=0)
     oacc, _, ocnt = P.gravity_unsorted()
     assert tuple(int(v) for v in cnt) == tuple(int(v) for v in ocnt)
     if n > 1:
