@@ -4,7 +4,6 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <array>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -91,6 +90,7 @@ struct pt_ctx {
   DBuf<HexNode> hn;
   DBuf<HexOpen> ho;
   double gm = 0.0;  // GravityVisitor::monopole_gravity_factor
+  DBuf<double> reptab;  // offsets of the periodic replicas
   DBuf<double> ewt;  // Ewald Fourier table (periodic build)
   DBuf<int32_t> ewcount;
   DBuf<unsigned long long> cpart;  // per-block counter partials
@@ -376,7 +376,7 @@ void pt_ctx_destroy(pt_ctx* c) {
   release(c->bucket_of); release(c->u32_total);
   release(c->tstat); release(c->tinternal); release(c->tmeta);
   release(c->prec);
-  release(c->ewt);
+  release(c->ewt); release(c->reptab);
   release(c->ewcount);
   release(c->hraw); release(c->hn); release(c->ho);
   release(c->bucket_node); release(c->nd); release(c->ord_h); release(c->ord_b);
@@ -740,7 +740,6 @@ pt_status pt_traverse(pt_ctx* c, double theta, const double offset[3], pt_counte
     PT_TRY_HIP(c, ensure(c->pc_off, nb + 1));
     PT_TRY_HIP(c, ensure(c->cpart, std::max<int64_t>(nblk, 1) * 4));
     if ((st = ensure_scratch(c, pt_scan_scratch_bytes(nb + 1)))) return st;
-    PT_TRY_LAUNCH(c, pt_launch_fill_u64(c->cpart.p, std::max<int64_t>(nblk, 1) * 4, 0ull, c->stream));
     PT_TRY_LAUNCH(c, pt_launch_fill_u32((uint32_t*)c->derr.p, 1, 0u, c->stream));
     const HexOpen* ho = c->cfg.hexadecapole ? c->ho.p : nullptr;
     PT_TRY_LAUNCH(c, pt_launch_traverse(false, c->tnode.p, ho, c->bk.p, nb, gf, c->gm, c->offset,
@@ -987,7 +986,7 @@ static pt_status gravity_fused(pt_ctx* c, double theta, const double offset[3],
   const bool grouped = cap > 0;
   const int64_t nblk = std::max<int64_t>(
       grouped ? pt_grouped_gravity_blocks(nb, c->n, cap)
-              : (hexa ? pt_hexa_gravity_blocks(nb) : pt_gravity_blocks(nb, (int)precision)),
+              : pt_gravity_blocks(nb, (int)precision, hexa),
       1);
   PT_TRY_HIP(c, ensure(c->cpart, nblk * 4));
   PT_TRY_HIP(c, ensure(c->wqueue, 8));
@@ -1009,14 +1008,20 @@ static pt_status gravity_fused(pt_ctx* c, double theta, const double offset[3],
   }
   // the visitor offsets: one, or the (2N+1)^3 period replicas in the order of
   // ExMain::traversalFn (examples/Gravity.C:35-46), each added to `offset`;
-  // every replica's traversal adds to the accelerations and the counters
-  std::vector<std::array<double, 3>> offs;
+  // every replica's traversal adds to the accelerations and the counters.  One
+  // launch walks for as many replicas as fit beside a node id in 30 bits.
   const int nr = c->cfg.periodic ? c->cfg.n_replicas : 0;
-  for (int X = -nr; X <= nr; X++)
-    for (int Y = -nr; Y <= nr; Y++)
-      for (int Z = -nr; Z <= nr; Z++)
-        offs.push_back({c->offset[0] + X * c->cfg.period[0], c->offset[1] + Y * c->cfg.period[1],
-                        c->offset[2] + Z * c->cfg.period[2]});
+  const int64_t n_rep = (int64_t)(2 * nr + 1) * (2 * nr + 1) * (2 * nr + 1);
+  const bool shifted =
+      n_rep > 1 || c->offset[0] != 0.0 || c->offset[1] != 0.0 || c->offset[2] != 0.0;
+  int bits = 4;
+  while (bits < 30 && (int64_t(1) << bits) < c->nn + 8) bits++;
+  const int64_t per_launch = std::min<int64_t>(n_rep, int64_t(1) << (30 - bits));
+  if (shifted) {
+    PT_TRY_HIP(c, ensure(c->reptab, 3 * n_rep));
+    PT_TRY_LAUNCH(c, pt_launch_replica_table(nr, c->offset, c->cfg.period, c->reptab.p,
+                                             c->stream));
+  }
   // examples/Gravity.C:30-33: with dual_tree, Subtree::startDual's traversal
   // first, then the down traversal adds to the same accelerations
   const bool dual = c->cfg.dual_tree != 0;
@@ -1029,39 +1034,32 @@ static pt_status gravity_fused(pt_ctx* c, double theta, const double offset[3],
   for (int attempt = 0; attempt < 2; attempt++) {
     PT_TRY_LAUNCH(c, pt_launch_fill_u32((uint32_t*)c->derr.p, 1, 0u, c->stream));
     if (dual && (st = launch_list_interact(c, precision))) return st;
-    for (size_t r = 0; r < offs.size(); r++) {
-      const bool acc = r > 0 || dual;
-      const double* off = offs[r].data();
-      PT_TRY_LAUNCH(c, pt_launch_fill_u64(c->cpart.p, nblk * 4, 0ull, c->stream));
+    for (int64_t r0 = 0; r0 < n_rep; r0 += per_launch) {
+      const bool acc = r0 > 0 || dual;
+      const PtReplicas reps{c->reptab.p + 3 * r0, bits,
+                            (int32_t)std::min<int64_t>(per_launch, n_rep - r0)};
+      const PtReplicas* rep = shifted ? &reps : nullptr;
+      const HexOpen* ho = hexa ? c->ho.p : nullptr;
+      const HexNode* hn = hexa ? c->hn.p : nullptr;
       {
         Timer t(c, PT_T_FORCE);
         if (grouped)
           PT_TRY_LAUNCH(c, pt_launch_grouped_gravity(
                                (int)precision, attempt == 1, c->bk.p, c->fg_first.p, c->fg_nb.p,
-                               c->fg_ng.p, nb, c->n, cap, c->tnode.p, c->gn.p, c->gn32.p,
-                               hexa ? c->ho.p : nullptr, hexa ? c->hn.p : nullptr, c->xs.p,
-                               c->ys.p, c->zs.p, c->ms.p, c->es.p, gf, c->gm, off, c->axs.p,
-                               c->ays.p, c->azs.p, c->pots.p, c->cpart.p, c->derr.p, acc,
-                               c->stream));
-        else if (hexa)
-          PT_TRY_LAUNCH(c, pt_launch_hexa_gravity((int)precision, attempt == 1, c->bk.p, nb,
-                                                  c->tnode.p, c->ho.p,
-                                                  c->hn.p, c->xs.p, c->ys.p, c->zs.p, c->ms.p,
-                                                  c->es.p, gf, c->gm, off, c->axs.p, c->ays.p,
-                                                  c->azs.p, c->pots.p, c->cpart.p, c->derr.p, acc,
-                                                  c->stream));
+                               c->fg_ng.p, nb, c->n, cap, c->tnode.p, c->gn.p, c->gn32.p, ho, hn,
+                               c->xs.p, c->ys.p, c->zs.p, c->ms.p, c->es.p, gf, c->gm, rep,
+                               c->axs.p, c->ays.p, c->azs.p, c->pots.p, c->cpart.p, c->derr.p,
+                               acc, c->stream));
         else
           PT_TRY_LAUNCH(c, pt_launch_gravity((int)precision, attempt == 1, c->bk.p, nb,
-                                             c->tnode.p, c->gn.p, c->gn32.p, c->xs.p, c->ys.p,
-                                             c->zs.p, c->ms.p, c->es.p, gf, off, c->axs.p,
-                                             c->ays.p, c->azs.p, c->pots.p, c->cpart.p,
+                                             c->tnode.p, c->gn.p, c->gn32.p, ho, hn, c->xs.p,
+                                             c->ys.p, c->zs.p, c->ms.p, c->es.p, gf, c->gm, rep,
+                                             c->axs.p, c->ays.p, c->azs.p, c->pots.p, c->cpart.p,
                                              c->derr.p, c->wqueue.p, acc, c->stream));
       }
-      if (r + 1 < offs.size())
+      if (r0 + per_launch < n_rep)
         PT_TRY_LAUNCH(c, pt_launch_reduce_counters(c->cpart.p, nblk, c->counters.p, c->derr.p,
-                                                   c->stream, acc));
-      else
-        break;
+                                                   c->stream, r0 > 0));
     }
     if (c->cfg.periodic) {
       // LeafEwaldFn after the replicas (examples/Gravity.C:47-50)
@@ -1082,7 +1080,7 @@ static pt_status gravity_fused(pt_ctx* c, double theta, const double offset[3],
     // the last replica's counters, the unsort to caller order and the one
     // read-back; a rerun (stack overflow, rare) repeats every replica
     int32_t herr = 0;
-    if ((st = finish_counters(c, nblk, &herr, true, offs.size() > 1))) return st;
+    if ((st = finish_counters(c, nblk, &herr, true, n_rep > per_launch))) return st;
     if (!herr) break;
     if (attempt == 1) return fail(c, PT_ERR_CAPACITY, "walk stack overflow at 1536 entries");
   }

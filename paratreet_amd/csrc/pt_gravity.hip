@@ -59,6 +59,8 @@ constexpr int kGroupMax = PT_WAVE;  // targets per pass (one per lane at most)
 // FP32 work-group at 6 per CU in LDS (26.5 KiB each).
 constexpr int kSmallStack = 192;
 constexpr int kBigStack = 1536;
+// Several replicas walked at once start with up to 64 roots on the stack.
+constexpr int kRepStack = 384;
 
 // ---------------------------------------------------------------------------
 // arithmetic
@@ -153,8 +155,22 @@ constexpr double kNullPos = 1.0e6;
 // Per-wave LDS working set: the staged chunk (also the final reduction area),
 // the walk stack and the pending closed-node / leaf-source buffers (a step
 // adds at most 64 entries to a buffer holding fewer than 64).
-template <bool F32, int STACK>
-struct __align__(16) WaveLds {
+// The walk entries of the buffered leaf sources (their replica), kept when a
+// walk serves several replicas.
+struct NoEntries {
+  __device__ __forceinline__ int32_t entry(int) const { return 0; }
+  __device__ __forceinline__ void set_entry(int, int32_t) {}
+};
+struct LeafEntries {
+  int32_t ppent[2 * PT_WAVE];
+  __device__ __forceinline__ int32_t entry(int k) const { return ppent[k]; }
+  __device__ __forceinline__ void set_entry(int k, int32_t e) { ppent[k] = e; }
+};
+template <bool REP>
+using EntriesIf = typename std::conditional<REP, LeafEntries, NoEntries>::type;
+
+template <bool F32, int STACK, bool REP = false>
+struct __align__(16) WaveLds : EntriesIf<REP> {
   static constexpr int kStage = kSlots * (F32 ? sizeof(SrcC32) : sizeof(SrcC64));
   static_assert(64 * 4 * sizeof(double) <= kStage, "reduction area");
   unsigned char stage[kStage];
@@ -300,11 +316,6 @@ __device__ __forceinline__ bool node_far_dsq(double dsq, float nsoft, const Buck
 // A closed node's id with the far flag of node_far_dsq in bit 30.
 constexpr int32_t kFarNode = 1 << 30;
 
-__device__ __forceinline__ float frame32(double v, double o, double cc) {
-  return (float)((v + o) - cc);
-}
-
-
 struct Group {
   int ng;      // targets in this pass
   int S;       // source slots = 64 / ng
@@ -387,11 +398,11 @@ __device__ __forceinline__ SrcC<F32> node_record(int32_t id, bool far,
                                                  const GravNode* __restrict__ gn,
                                                  const GravNode32* __restrict__ gn32,
                                                  const Bucket& b, const BucketF& bf, float emax,
-                                                 double ox, double oy, double oz, double ccx,
-                                                 double ccy, double ccz, bool& near) {
+                                                 const Off3& o, double ccx, double ccy,
+                                                 double ccz, bool& near) {
   if constexpr (F32) {
     const GravNode32 h = gn32[id];
-    const double cx = h.cx + ox, cy = h.cy + oy, cz = h.cz + oz;
+    const double cx = h.cx + o.x, cy = h.cy + o.y, cz = h.cz + o.z;
     const double soft = h.soft64;
     SrcC32 r;
     r.cx = (float)(cx - ccx);
@@ -416,12 +427,12 @@ __device__ __forceinline__ SrcC<F32> node_record(int32_t id, bool far,
     return r;
   } else {
     const GravNode s = gn[id];
-    const double cx = s.cx + ox, cy = s.cy + oy, cz = s.cz + oz;
+    const double cx = s.cx + o.x, cy = s.cy + o.y, cz = s.cz + o.z;
     const double soft = s.soft;
     SrcC64 r;
-    r.cx = s.cx;
-    r.cy = s.cy;
-    r.cz = s.cz;
+    r.cx = cx;
+    r.cy = cy;
+    r.cz = cz;
     r.mass = s.mass;
     bool mono = false;
     near = false;
@@ -463,14 +474,14 @@ __device__ __forceinline__ SrcP<F32> particle_record(int64_t j, const double* __
                                                      const double* __restrict__ pz,
                                                      const double* __restrict__ pm,
                                                      const double* __restrict__ pe,
-                                                     const BucketF& bf, float emax, double ox,
-                                                     double oy, double oz, double ccx, double ccy,
-                                                     double ccz, bool& near) {
+                                                     const BucketF& bf, float emax, const Off3& o,
+                                                     double ccx, double ccy, double ccz,
+                                                     bool& near) {
   if constexpr (F32) {
     SrcP32 r;
-    r.x = (float)((px[j] + ox) - ccx);
-    r.y = (float)((py[j] + oy) - ccy);
-    r.z = (float)((pz[j] + oz) - ccz);
+    r.x = (float)((px[j] + o.x) - ccx);
+    r.y = (float)((py[j] + o.y) - ccy);
+    r.z = (float)((pz[j] + o.z) - ccz);
     r.m = (float)pm[j];
     r.e = (float)pe[j];
     r.pad0 = r.pad1 = r.pad2 = 0.f;
@@ -478,14 +489,13 @@ __device__ __forceinline__ SrcP<F32> particle_record(int64_t j, const double* __
     return r;
   } else {
     SrcP64 r;
-    r.x = px[j];
-    r.y = py[j];
-    r.z = pz[j];
+    r.x = px[j] + o.x;
+    r.y = py[j] + o.y;
+    r.z = pz[j] + o.z;
     r.m = pm[j];
     r.e = pe[j];
     r.pad = 0.0;
-    near = near32(frame32(r.x, ox, ccx), frame32(r.y, oy, ccy), frame32(r.z, oz, ccz), (float)r.e,
-                  bf, emax);
+    near = near32((float)(r.x - ccx), (float)(r.y - ccy), (float)(r.z - ccz), (float)r.e, bf, emax);
     return r;
   }
 }
@@ -530,8 +540,7 @@ __device__ __forceinline__ void node_pair(const SrcC<F32>& s, const Lanes<F32>& 
                                           typename std::conditional<F32, float, double>::type& px,
                                           typename std::conditional<F32, float, double>::type& py,
                                           typename std::conditional<F32, float, double>::type& pz,
-                                          typename std::conditional<F32, float, double>::type& pp,
-                                          double ox, double oy, double oz) {
+                                          typename std::conditional<F32, float, double>::type& pp) {
   if constexpr (F32) {
     if (s.soft < 0.f) {
       // addGravity: unsoftened monopole, no potential
@@ -576,7 +585,7 @@ __device__ __forceinline__ void node_pair(const SrcC<F32>& s, const Lanes<F32>& 
     }
   } else {
     if (s.soft < 0.0) {
-      const double dx = (s.cx + ox) - L.tx, dy = (s.cy + oy) - L.ty, dz = (s.cz + oz) - L.tz;
+      const double dx = s.cx - L.tx, dy = s.cy - L.ty, dz = s.cz - L.tz;
       const double rsq = fma(dx, dx, fma(dy, dy, dz * dz));
       const double ir = pt_rsqrt64(rsq);
       double f = s.mass * (ir * ir * ir);
@@ -585,7 +594,7 @@ __device__ __forceinline__ void node_pair(const SrcC<F32>& s, const Lanes<F32>& 
       py = fma(dy, f, py);
       pz = fma(dz, f, pz);
     } else {
-      const double rx = (L.tx - s.cx) - ox, ry = (L.ty - s.cy) - oy, rz = (L.tz - s.cz) - oz;
+      const double rx = L.tx - s.cx, ry = L.ty - s.cy, rz = L.tz - s.cz;
       const double rsq = fma(rx, rx, fma(ry, ry, rz * rz));
       const double dir = pt_rsqrt64(rsq);
       double a, bb, c, d;
@@ -611,7 +620,7 @@ __device__ __forceinline__ void node_pair_far(
     typename std::conditional<F32, float, double>::type& py,
     typename std::conditional<F32, float, double>::type& pz,
     typename std::conditional<F32, float, double>::type& pp,
-    typename std::conditional<F32, float, double>::type& pq, double ox, double oy, double oz) {
+    typename std::conditional<F32, float, double>::type& pq) {
   if constexpr (F32) {
     // The unsoftened branch of SPLINEQ (a = 1/r, b = 1/r^3, c = 3/r^5,
     // d = 15/r^7) regrouped over the staged 3Q and 3 tr: with u = 1/r^2,
@@ -636,7 +645,7 @@ __device__ __forceinline__ void node_pair_far(
     pp = fmaf(-s.mass, v, pp);
     pq = fmaf(b, fmaf(-1.5f, k, s.tr), pq);
   } else {
-    const double rx = (L.tx - s.cx) - ox, ry = (L.ty - s.cy) - oy, rz = (L.tz - s.cz) - oz;
+    const double rx = L.tx - s.cx, ry = L.ty - s.cy, rz = L.tz - s.cz;
     const double rsq = fma(rx, rx, fma(ry, ry, rz * rz));
     const double a = pt_rsqrt64(rsq);
     const double bb = a * a * a;
@@ -656,14 +665,14 @@ __device__ __forceinline__ void node_pair_far(
 
 template <bool F32, typename W_t>
 __device__ __forceinline__ void eval_nodes(const W_t& W, const Group& g, Lanes<F32>& L, int kfar,
-                                           int kend, double ox, double oy, double oz) {
+                                           int kend) {
   const SrcC<F32>* src = reinterpret_cast<const SrcC<F32>*>(W.stage);
   if constexpr (F32) {
     float px = 0.f, py = 0.f, pz = 0.f, pp = 0.f, pq = 0.f;
-    for (int k = 0; k < kfar; k++) node_pair<true>(src[g.s + k * g.S], L, px, py, pz, pp, ox, oy, oz);
+    for (int k = 0; k < kfar; k++) node_pair<true>(src[g.s + k * g.S], L, px, py, pz, pp);
 #pragma unroll 2
     for (int k = kfar; k < kend; k++)
-      node_pair_far<true>(src[g.s + k * g.S], L, px, py, pz, pp, pq, ox, oy, oz);
+      node_pair_far<true>(src[g.s + k * g.S], L, px, py, pz, pp, pq);
     pp = fmaf(1.0f / 3.0f, pq, pp);
     kahan_add(L.ax, L.cx, px);
     kahan_add(L.ay, L.cy, py);
@@ -671,16 +680,15 @@ __device__ __forceinline__ void eval_nodes(const W_t& W, const Group& g, Lanes<F
     kahan_add(L.ap, L.cp, pp);
   } else {
     for (int k = 0; k < kfar; k++)
-      node_pair<false>(src[g.s + k * g.S], L, L.ax, L.ay, L.az, L.ap, ox, oy, oz);
+      node_pair<false>(src[g.s + k * g.S], L, L.ax, L.ay, L.az, L.ap);
     for (int k = kfar; k < kend; k++)
-      node_pair_far<false>(src[g.s + k * g.S], L, L.ax, L.ay, L.az, L.ap, L.ap, ox, oy, oz);
+      node_pair_far<false>(src[g.s + k * g.S], L, L.ax, L.ay, L.az, L.ap, L.ap);
   }
 }
 
 template <bool F32, typename W_t>
 __device__ __forceinline__ void eval_particles(const W_t& W, const Group& g, Lanes<F32>& L,
-                                               int kfar, int kend, double ox, double oy,
-                                               double oz) {
+                                               int kfar, int kend) {
   if constexpr (F32) {
     float px = 0.f, py = 0.f, pz = 0.f;
     const SrcP32* src = reinterpret_cast<const SrcP32*>(W.stage);
@@ -728,7 +736,7 @@ __device__ __forceinline__ void eval_particles(const W_t& W, const Group& g, Lan
     const SrcP64* src = reinterpret_cast<const SrcP64*>(W.stage);
     for (int k = 0; k < kfar; k++) {
       const SrcP64 s = src[g.s + k * g.S];
-      const double dx = (s.x + ox) - L.tx, dy = (s.y + oy) - L.ty, dz = (s.z + oz) - L.tz;
+      const double dx = s.x - L.tx, dy = s.y - L.ty, dz = s.z - L.tz;
       const double rsq = fma(dx, dx, fma(dy, dy, dz * dz));
       double f = spline_b64(rsq, s.e + L.te) * s.m;
       f = rsq != 0 ? f : 0.0;
@@ -738,7 +746,7 @@ __device__ __forceinline__ void eval_particles(const W_t& W, const Group& g, Lan
     }
     for (int k = kfar; k < kend; k++) {
       const SrcP64 s = src[g.s + k * g.S];
-      const double dx = (s.x + ox) - L.tx, dy = (s.y + oy) - L.ty, dz = (s.z + oz) - L.tz;
+      const double dx = s.x - L.tx, dy = s.y - L.ty, dz = s.z - L.tz;
       const double rsq = fma(dx, dx, fma(dy, dy, dz * dz));
       const double a = pt_rsqrt64(rsq);
       const double f = (a * a * a) * s.m;
@@ -749,22 +757,22 @@ __device__ __forceinline__ void eval_particles(const W_t& W, const Group& g, Lan
   }
 }
 
-// Flattens up to 64 leaf sources (begin and flagged count, leaf_entry, in
-// the calling lane; count 0 = none) into particles and evaluates them 64 at a
+// Flattens up to 64 leaf sources (begin, flagged count, leaf_entry, and walk
+// entry in the calling lane; count 0 = none) into particles and evaluates them 64 at a
 // time.  Leaves not flagged far come first, so each window holds its near
 // particles in its first slots and the rest take the branch-free loop.  Each
 // window marks the slot where every leaf starts (the leaf's lane in LDS, a
 // bit in a ballot); a slot's leaf is the mark at the highest start bit at or
 // below it, or the previous window's last leaf when there is none.
-template <bool F32, typename W_t>
-__device__ __forceinline__ void do_leaves(W_t& W, int32_t beg, int32_t cntf, const Group& g,
-                                          Lanes<F32>& L, const double* __restrict__ px,
+template <bool F32, typename W_t, typename Sh>
+__device__ __forceinline__ void do_leaves(W_t& W, int32_t beg, int32_t cntf, int32_t ent,
+                                          const Group& g, Lanes<F32>& L,
+                                          const double* __restrict__ px,
                                           const double* __restrict__ py,
                                           const double* __restrict__ pz,
                                           const double* __restrict__ pm,
                                           const double* __restrict__ pe, const BucketF& bf,
-                                          double ox, double oy, double oz, double ccx, double ccy,
-                                          double ccz) {
+                                          const Sh& sh, double ccx, double ccy, double ccz) {
   const int lane = __lane_id();
   const bool far = (cntf & kFarLeaf) != 0;
   const int cnt = cntf & ~kFarLeaf;
@@ -789,12 +797,13 @@ __device__ __forceinline__ void do_leaves(W_t& W, int32_t beg, int32_t cntf, con
     carry = __builtin_amdgcn_readlane(leaf, cw - 1);
     const int lbeg = __shfl(beg, leaf, PT_WAVE);
     const int lexc = __shfl(exc, leaf, PT_WAVE);
+    const int lent = Sh::kRep ? __shfl(ent, leaf, PT_WAVE) : 0;
     const int slot = s0 + lane;
     if (lane < cw && slot < total) {
       const int64_t j = (int64_t)lbeg + (slot - lexc);
       bool nr;
       reinterpret_cast<SrcP<F32>*>(W.stage)[lane] = particle_record<F32>(
-          j, px, py, pz, pm, pe, bf, L.emax, ox, oy, oz, ccx, ccy, ccz, nr);
+          j, px, py, pz, pm, pe, bf, L.emax, sh.at(lent), ccx, ccy, ccz, nr);
     }
     const int nsrc = (total - s0) < cw ? (total - s0) : cw;
     const int nn = near_total - s0;
@@ -802,23 +811,23 @@ __device__ __forceinline__ void do_leaves(W_t& W, int32_t beg, int32_t cntf, con
     pad_chunk<F32, false, W_t>(W, nsrc, g);
     __builtin_amdgcn_wave_barrier();
     eval_particles<F32, W_t>(W, g, L, uniform_if<!F32>(ceil_div_s(nnear, g)),
-                             uniform_if<!F32>(ceil_div_s(nsrc, g)), ox, oy, oz);
+                             uniform_if<!F32>(ceil_div_s(nsrc, g)));
     __builtin_amdgcn_wave_barrier();
   }
 }
 
-template <bool F32, typename W_t>
-__device__ __forceinline__ void do_nodes(W_t& W, int32_t id, int nsrc, const Group& g,
+template <bool F32, typename W_t, typename Sh>
+__device__ __forceinline__ void do_nodes(W_t& W, int32_t ent, int nsrc, const Group& g,
                                          Lanes<F32>& L, const GravNode* __restrict__ gn,
                                          const GravNode32* __restrict__ gn32, const Bucket& b,
-                                         const BucketF& bf, double ox, double oy, double oz,
-                                         double ccx, double ccy, double ccz) {
+                                         const BucketF& bf, const Sh& sh, double ccx, double ccy,
+                                         double ccz) {
   const bool act = (int)__lane_id() < nsrc;
   bool nr = false;
   SrcC<F32> r{};
   if (act)
-    r = node_record<F32>(id & ~kFarNode, (id & kFarNode) != 0, gn, gn32, b, bf, L.emax, ox, oy,
-                         oz, ccx, ccy, ccz, nr);
+    r = node_record<F32>(sh.id(ent & ~kFarNode), (ent & kFarNode) != 0, gn, gn32, b, bf, L.emax,
+                         sh.at(ent & ~kFarNode), ccx, ccy, ccz, nr);
   // near (monopole or possibly softened) nodes first, then far ones
   const unsigned long long mn = pt_ballot(act && nr), mf = pt_ballot(act && !nr);
   const int nnear = __popcll(mn);
@@ -826,7 +835,7 @@ __device__ __forceinline__ void do_nodes(W_t& W, int32_t id, int nsrc, const Gro
   pad_chunk<F32, true, W_t>(W, nsrc, g);
   __builtin_amdgcn_wave_barrier();
   eval_nodes<F32, W_t>(W, g, L, uniform_if<!F32>(ceil_div_s(nnear, g)),
-                       uniform_if<!F32>(ceil_div_s(nsrc, g)), ox, oy, oz);
+                       uniform_if<!F32>(ceil_div_s(nsrc, g)));
   __builtin_amdgcn_wave_barrier();
 }
 
@@ -909,6 +918,7 @@ interact_kernel(const Bucket* __restrict__ bk, int64_t nb, const TreeNode* __res
   const BucketF bf = bucket_frame(b, ccx, ccy, ccz);
   const int64_t pc0 = pc_off[bi], pc1 = pc_off[bi + 1];
   const int64_t pp0 = pp_off[bi], pp1 = pp_off[bi + 1];
+  const OneShift sh{ox, oy, oz};
   for (int g0 = 0; g0 < b.count; g0 += kGroupMax) {
     const Group g = make_group(b, g0);
     Lanes<F32> L;
@@ -916,7 +926,7 @@ interact_kernel(const Bucket* __restrict__ bk, int64_t nb, const TreeNode* __res
     for (int64_t e0 = pc0; e0 < pc1; e0 += PT_WAVE) {
       const int nsrc = (pc1 - e0) < PT_WAVE ? (int)(pc1 - e0) : PT_WAVE;
       const int32_t id = lane < nsrc ? pc[e0 + lane] : 0;
-      do_nodes<F32, W_t>(W, id, nsrc, g, L, gn, gn32, b, bf, ox, oy, oz, ccx, ccy, ccz);
+      do_nodes<F32, W_t>(W, id, nsrc, g, L, gn, gn32, b, bf, sh, ccx, ccy, ccz);
     }
     for (int64_t l0 = pp0; l0 < pp1; l0 += PT_WAVE) {
       int32_t beg = 0, cnt = 0;
@@ -926,7 +936,7 @@ interact_kernel(const Bucket* __restrict__ bk, int64_t nb, const TreeNode* __res
         cnt = leaf_entry(nd.count, nd.cx, nd.cy, nd.cz, nd.leaf_reach, nd.leaf_soft, bf, L.emax,
                          ox, oy, oz, ccx, ccy, ccz);
       }
-      do_leaves<F32, W_t>(W, beg, cnt, g, L, px, py, pz, pm, pe, bf, ox, oy, oz, ccx, ccy, ccz);
+      do_leaves<F32, W_t>(W, beg, cnt, 0, g, L, px, py, pz, pm, pe, bf, sh, ccx, ccy, ccz);
     }
     finish_group<F32, W_t>(W, g, L, ax, ay, az, pot);
   }
@@ -1040,11 +1050,10 @@ __device__ __forceinline__ void hexa_eval(const R* __restrict__ h, R m, R rx, R 
   gz = fma_r(c2, v2z, fma_r(c3, v3z, fma_r(c4, v4z, -rz * g)));
 }
 
-__device__ __forceinline__ void hexa_pair(const SrcH& s, Lanes<false>& L, double ox, double oy,
-                                          double oz) {
+__device__ __forceinline__ void hexa_pair(const SrcH& s, Lanes<false>& L) {
   if (s.mono != 0.0) {
     // addGravity: unsoftened monopole, no potential
-    const double dx = (s.cx + ox) - L.tx, dy = (s.cy + oy) - L.ty, dz = (s.cz + oz) - L.tz;
+    const double dx = s.cx - L.tx, dy = s.cy - L.ty, dz = s.cz - L.tz;
     const double rsq = dx * dx + dy * dy + dz * dz;
     const double ir = pt_rsqrt64(rsq);
     double f = s.mass * (ir * ir * ir);
@@ -1053,7 +1062,7 @@ __device__ __forceinline__ void hexa_pair(const SrcH& s, Lanes<false>& L, double
     L.ay += dy * f;
     L.az += dz * f;
   } else {
-    const double rx = (L.tx - s.cx) - ox, ry = (L.ty - s.cy) - oy, rz = (L.tz - s.cz) - oz;
+    const double rx = L.tx - s.cx, ry = L.ty - s.cy, rz = L.tz - s.cz;
     double p, gx, gy, gz;
     hexa_eval<double>(s.h, s.mass, rx, ry, rz, p, gx, gy, gz);
     L.ap += p;
@@ -1068,22 +1077,23 @@ __device__ __forceinline__ void hexa_pair(const SrcH& s, Lanes<false>& L, double
 // and evaluates them for the group's targets (slot s of a lane takes sources
 // s, s + S, ... of each part; the S partial sums are combined in
 // finish_group).
-template <typename W_t>
-__device__ __forceinline__ void do_nodes_hexa(W_t& W, int32_t id, int nsrc, const Group& g,
+template <typename W_t, typename Sh>
+__device__ __forceinline__ void do_nodes_hexa(W_t& W, int32_t ent, int nsrc, const Group& g,
                                               Lanes<false>& L, const HexNode* __restrict__ hn,
-                                              const Bucket& b, double ox, double oy, double oz) {
+                                              const Bucket& b, const Sh& sh) {
   const int lane = __lane_id();
   SrcH* st = reinterpret_cast<SrcH*>(W.stage);
   for (int h = 0; h < nsrc; h += kHexaStage) {
     if (lane >= h && lane < h + kHexaStage && lane < nsrc) {
-      const bool far = (id & kFarNode) != 0;
-      const HexNode& s = hn[id & ~kFarNode];
+      const bool far = (ent & kFarNode) != 0;
+      const HexNode& s = hn[sh.id(ent & ~kFarNode)];
+      const Off3 o = sh.at(ent & ~kFarNode);
       SrcH r;
-      r.cx = s.cx;
-      r.cy = s.cy;
-      r.cz = s.cz;
+      r.cx = s.cx + o.x;
+      r.cy = s.cy + o.y;
+      r.cz = s.cz + o.z;
       r.mass = s.mass;
-      r.mono = !far && pt_open_softening(s.cx + ox, s.cy + oy, s.cz + oz, s.soft, b) ? 1.0 : 0.0;
+      r.mono = !far && pt_open_softening(r.cx, r.cy, r.cz, s.soft, b) ? 1.0 : 0.0;
 #pragma unroll
       for (int k = 0; k < PT_HEXA_MOMS; k++) r.h[k] = s.h[k];
       st[lane - h] = r;
@@ -1093,7 +1103,7 @@ __device__ __forceinline__ void do_nodes_hexa(W_t& W, int32_t id, int nsrc, cons
     const int kend = ceil_div_s(n, g);
     for (int k = 0; k < kend; k++) {
       const int i = g.s + k * g.S;
-      if (i < n) hexa_pair(st[i], L, ox, oy, oz);
+      if (i < n) hexa_pair(st[i], L);
     }
     __builtin_amdgcn_wave_barrier();
   }
@@ -1126,17 +1136,18 @@ __device__ __forceinline__ void hexa_pair32(const SrcH32& s, const Lanes<true>& 
 // once (centres shifted to the bucket frame in FP64, the openSoftening
 // decision in FP64), each chunk's FP32 partial sums added to the Kahan
 // accumulators.
-template <typename W_t>
-__device__ __forceinline__ void do_nodes_hexa32(W_t& W, int32_t id, int nsrc, const Group& g,
+template <typename W_t, typename Sh>
+__device__ __forceinline__ void do_nodes_hexa32(W_t& W, int32_t ent, int nsrc, const Group& g,
                                                 Lanes<true>& L, const HexNode* __restrict__ hn,
-                                                const Bucket& b, double ox, double oy, double oz,
-                                                double ccx, double ccy, double ccz) {
+                                                const Bucket& b, const Sh& sh, double ccx,
+                                                double ccy, double ccz) {
   const int lane = __lane_id();
   SrcH32* st = reinterpret_cast<SrcH32*>(W.stage);
   if (lane < nsrc) {
-    const bool far = (id & kFarNode) != 0;
-    const HexNode& s = hn[id & ~kFarNode];
-    const double cx = s.cx + ox, cy = s.cy + oy, cz = s.cz + oz;
+    const bool far = (ent & kFarNode) != 0;
+    const HexNode& s = hn[sh.id(ent & ~kFarNode)];
+    const Off3 o = sh.at(ent & ~kFarNode);
+    const double cx = s.cx + o.x, cy = s.cy + o.y, cz = s.cz + o.z;
     SrcH32 r;
     r.cx = (float)(cx - ccx);
     r.cy = (float)(cy - ccy);
@@ -1183,6 +1194,7 @@ interact_hexa_kernel(const Bucket* __restrict__ bk, int64_t nb,
   const BucketF bf = bucket_frame(b, ccx, ccy, ccz);
   const int64_t pc0 = pc_off[bi], pc1 = pc_off[bi + 1];
   const int64_t pp0 = pp_off[bi], pp1 = pp_off[bi + 1];
+  const OneShift sh{ox, oy, oz};
   for (int g0 = 0; g0 < b.count; g0 += kGroupMax) {
     const Group g = make_group(b, g0);
     Lanes<false> L;
@@ -1190,7 +1202,7 @@ interact_hexa_kernel(const Bucket* __restrict__ bk, int64_t nb,
     for (int64_t e0 = pc0; e0 < pc1; e0 += PT_WAVE) {
       const int nsrc = (pc1 - e0) < PT_WAVE ? (int)(pc1 - e0) : PT_WAVE;
       const int32_t id = lane < nsrc ? pc[e0 + lane] : 0;
-      do_nodes_hexa<HexaLds>(W, id, nsrc, g, L, hn, b, ox, oy, oz);
+      do_nodes_hexa<HexaLds>(W, id, nsrc, g, L, hn, b, sh);
     }
     for (int64_t l0 = pp0; l0 < pp1; l0 += PT_WAVE) {
       int32_t beg = 0, cnt = 0;
@@ -1200,18 +1212,15 @@ interact_hexa_kernel(const Bucket* __restrict__ bk, int64_t nb,
         cnt = leaf_entry(nd.count, nd.cx, nd.cy, nd.cz, nd.leaf_reach, nd.leaf_soft, bf, L.emax,
                          ox, oy, oz, ccx, ccy, ccz);
       }
-      do_leaves<false, HexaLds>(W, beg, cnt, g, L, px, py, pz, pm, pe, bf, ox, oy, oz, ccx, ccy,
-                                ccz);
+      do_leaves<false, HexaLds>(W, beg, cnt, 0, g, L, px, py, pz, pm, pe, bf, sh, ccx, ccy, ccz);
     }
     finish_group<false, HexaLds>(W, g, L, ax, ay, az, pot);
   }
 }
 
-// Fused walk + interactions of the HEXADECAPOLE build (FP64): the walk with
-// the hexadecapole open(), closed nodes evaluated with the reduced moments,
-// leaves with leaf(); one wave per bucket, chunks evaluated as they fill.
-template <int STACK>
-struct __align__(16) HexaFusedLds {
+// LDS working set of a fused wave of the HEXADECAPOLE build.
+template <int STACK, bool REP>
+struct __align__(16) HexaFusedLds : EntriesIf<REP> {
   static constexpr int kStage = HexaLds::kStage;
   static_assert(PT_WAVE * sizeof(SrcH32) <= kStage, "FP32 node chunk");
   unsigned char stage[kStage];
@@ -1222,166 +1231,33 @@ struct __align__(16) HexaFusedLds {
   int32_t fl_mark[PT_WAVE];
 };
 
-template <int STACK, bool F32>
-__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(STACK == kSmallStack ? (F32 ? kHexaWaves32 : kHexaWaves) : 1, 8)))
-hexa_gravity_kernel(const Bucket* __restrict__ bk, int64_t nb, const TreeNode* __restrict__ nodes,
-                    const HexOpen* __restrict__ ho, const HexNode* __restrict__ hn,
-                    const double* __restrict__ px, const double* __restrict__ py,
-                    const double* __restrict__ pz, const double* __restrict__ pm,
-                    const double* __restrict__ pe, double gf, double gm, double ox, double oy,
-                    double oz, double* __restrict__ ax, double* __restrict__ ay,
-                    double* __restrict__ az, double* __restrict__ pot,
-                    unsigned long long* __restrict__ partials, int32_t* __restrict__ err, int acc) {
-  using W_t = HexaFusedLds<STACK>;
-  __shared__ W_t lds[kWaves];
-  __shared__ unsigned long long s_cnt[kWaves][4];
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PT_WAVE);
-  const int lane = threadIdx.x & (PT_WAVE - 1);
-  W_t& W = lds[wave];
-  unsigned long long c_node = 0, c_part = 0, c_open = 0, c_close = 0;
-  bool overflow = false;
-  const int64_t bi = pt_xcd_block(blockIdx.x, gridDim.x) * kWaves + wave;
-  if (bi < nb) {
-    const Bucket b = bk[bi];
-    const int64_t nt = b.count;
-    const double ccx = (b.lox + b.hix) * 0.5, ccy = (b.loy + b.hiy) * 0.5,
-                 ccz = (b.loz + b.hiz) * 0.5;
-    const BucketF bf = bucket_frame(b, ccx, ccy, ccz);
-    for (int g0 = 0; g0 < b.count; g0 += kGroupMax) {
-      const Group g = make_group(b, g0);
-      const bool count = g0 == 0;  // the walk repeats per target group; count once
-      Lanes<F32> L;
-      load_targets<F32>(L, g, px, py, pz, pe, ccx, ccy, ccz);
-      int sp = 0;
-      int npc = 0, npp = 0;
-      WalkCounts wc;
-      {
-        const WalkLane r = pt_walk_root<true>(nodes, b, gf, ox, oy, oz, W.stack, sp, wc, ho, gm);
-        if (r.is_closed) {
-          if (lane == 0) W.pcbuf[0] = 0;
-          npc = 1;
-        } else if (r.is_leaf) {
-          if (lane == 0) {
-            W.ppbeg[0] = r.begin;
-            W.ppcnt[0] = r.count;
-          }
-          npp = 1;
-        }
-        if (count) {
-          c_open += wc.n_open;
-          c_close += wc.n_close;
-          c_node += (unsigned long long)wc.n_close * nt;
-          c_part += (unsigned long long)wc.leaf_parts * nt;
-        }
-      }
-      __builtin_amdgcn_wave_barrier();
-      while (sp > 0) {
-        unsigned long long leafm, closem;
-        const WalkLane r = pt_walk_step<STACK, true>(nodes, b, gf, ox, oy, oz, W.stack, sp,
-                                                     overflow, wc, leafm, closem, ho, gm);
-        if (count) {
-          c_open += wc.n_open;
-          c_close += wc.n_close;
-          c_node += (unsigned long long)wc.n_close * nt;
-          c_part += (unsigned long long)wc.leaf_parts * nt;
-        }
-        if (r.is_closed) W.pcbuf[npc + pt_rank_in(closem)] = r.node;
-        if (r.is_leaf) {
-          const int k = npp + pt_rank_in(leafm);
-          W.ppbeg[k] = r.begin;
-          W.ppcnt[k] = leaf_far_dsq(r.dsq, r.leaf_reach, r.leaf_soft, bf, L.emax)
-                           ? (r.count | kFarLeaf)
-                           : r.count;
-        }
-        npc += __popcll(closem);
-        npp += __popcll(leafm);
-        __builtin_amdgcn_wave_barrier();
-        if (npc >= PT_WAVE) {
-          if constexpr (F32)
-            do_nodes_hexa32<W_t>(W, W.pcbuf[lane], PT_WAVE, g, L, hn, b, ox, oy, oz, ccx, ccy,
-                                 ccz);
-          else
-            do_nodes_hexa<W_t>(W, W.pcbuf[lane], PT_WAVE, g, L, hn, b, ox, oy, oz);
-          const int rest = npc - PT_WAVE;
-          const int32_t v = lane < rest ? W.pcbuf[PT_WAVE + lane] : 0;
-          __builtin_amdgcn_wave_barrier();
-          if (lane < rest) W.pcbuf[lane] = v;
-          npc = rest;
-          __builtin_amdgcn_wave_barrier();
-        }
-        if (npp >= PT_WAVE) {
-          do_leaves<F32, W_t>(W, W.ppbeg[lane], W.ppcnt[lane], g, L, px, py, pz, pm, pe, bf, ox,
-                                oy, oz, ccx, ccy, ccz);
-          const int rest = npp - PT_WAVE;
-          const int32_t vb = lane < rest ? W.ppbeg[PT_WAVE + lane] : 0;
-          const int32_t vc = lane < rest ? W.ppcnt[PT_WAVE + lane] : 0;
-          __builtin_amdgcn_wave_barrier();
-          if (lane < rest) {
-            W.ppbeg[lane] = vb;
-            W.ppcnt[lane] = vc;
-          }
-          npp = rest;
-          __builtin_amdgcn_wave_barrier();
-        }
-      }
-      if (npc > 0) {
-        const int32_t id = lane < npc ? W.pcbuf[lane] : 0;
-        if constexpr (F32)
-          do_nodes_hexa32<W_t>(W, id, npc, g, L, hn, b, ox, oy, oz, ccx, ccy, ccz);
-        else
-          do_nodes_hexa<W_t>(W, id, npc, g, L, hn, b, ox, oy, oz);
-      }
-      if (npp > 0) {
-        const int32_t beg = lane < npp ? W.ppbeg[lane] : 0;
-        const int32_t cnt = lane < npp ? W.ppcnt[lane] : 0;
-        do_leaves<F32, W_t>(W, beg, cnt, g, L, px, py, pz, pm, pe, bf, ox, oy, oz, ccx, ccy,
-                              ccz);
-      }
-      finish_group<F32, W_t>(W, g, L, ax, ay, az, pot, acc != 0);
-    }
-  }
-  if (lane == 0) {
-    if (overflow) atomicExch(err, 1);
-    s_cnt[wave][0] = c_node;
-    s_cnt[wave][1] = c_part;
-    s_cnt[wave][2] = c_open;
-    s_cnt[wave][3] = c_close;
-  }
-  __syncthreads();
-  if (threadIdx.x < 4) {
-    unsigned long long v = 0;
-    for (int w = 0; w < kWaves; w++) v += s_cnt[w][threadIdx.x];
-    partials[(int64_t)blockIdx.x * 4 + threadIdx.x] = v;
-  }
-}
-
 // The LDS working set of a fused wave: the quadrupole build's, or the
 // HEXADECAPOLE build's (larger node records).
-template <bool F32, int STACK, bool HEXA>
+template <bool F32, int STACK, bool HEXA, typename Sh>
 struct FusedLdsOf {
-  using type = WaveLds<F32, STACK>;
+  using type = WaveLds<F32, STACK, Sh::kRep>;
 };
-template <bool F32, int STACK>
-struct FusedLdsOf<F32, STACK, true> {
-  using type = HexaFusedLds<STACK>;
+template <bool F32, int STACK, typename Sh>
+struct FusedLdsOf<F32, STACK, true, Sh> {
+  using type = HexaFusedLds<STACK, Sh::kRep>;
 };
 
 // Stages and evaluates up to one chunk of closed nodes (node id, with the
 // kFarNode flag, in the calling lane) in the build's form.
-template <bool F32, bool HEXA, typename W_t>
+template <bool F32, bool HEXA, typename W_t, typename Sh>
 __device__ __forceinline__ void stage_nodes(W_t& W, int32_t id, int nsrc, const Group& g,
                                             Lanes<F32>& L, const GravNode* __restrict__ gn,
                                             const GravNode32* __restrict__ gn32,
                                             const HexNode* __restrict__ hn, const Bucket& b,
-                                            const BucketF& bf, double ox, double oy, double oz,
+                                            const BucketF& bf, const Sh& sh,
                                             double ccx, double ccy, double ccz) {
   if constexpr (HEXA) {
     if constexpr (F32)
-      do_nodes_hexa32<W_t>(W, id, nsrc, g, L, hn, b, ox, oy, oz, ccx, ccy, ccz);
+      do_nodes_hexa32<W_t>(W, id, nsrc, g, L, hn, b, sh, ccx, ccy, ccz);
     else
-      do_nodes_hexa<W_t>(W, id, nsrc, g, L, hn, b, ox, oy, oz);
+      do_nodes_hexa<W_t>(W, id, nsrc, g, L, hn, b, sh);
   } else {
-    do_nodes<F32, W_t>(W, id, nsrc, g, L, gn, gn32, b, bf, ox, oy, oz, ccx, ccy, ccz);
+    do_nodes<F32, W_t>(W, id, nsrc, g, L, gn, gn32, b, bf, sh, ccx, ccy, ccz);
   }
 }
 
@@ -1389,7 +1265,7 @@ __device__ __forceinline__ void stage_nodes(W_t& W, int32_t id, int nsrc, const 
 // leaf sources (64 at a time).  A walk step starts with npc < cw and
 // npp < 64 and adds at most 64 to each, so the buffers (128 entries) never
 // overflow and each rest (< 64) fits one move.
-template <bool F32, bool HEXA, typename W_t>
+template <bool F32, bool HEXA, typename W_t, typename Sh>
 __device__ __forceinline__ void drain_full(W_t& W, int& npc, int& npp, const Group& g,
                                            Lanes<F32>& L, const GravNode* __restrict__ gn,
                                            const GravNode32* __restrict__ gn32,
@@ -1398,13 +1274,12 @@ __device__ __forceinline__ void drain_full(W_t& W, int& npc, int& npp, const Gro
                                            const double* __restrict__ py,
                                            const double* __restrict__ pz,
                                            const double* __restrict__ pm,
-                                           const double* __restrict__ pe, double ox, double oy,
-                                           double oz, double ccx, double ccy, double ccz) {
+                                           const double* __restrict__ pe, const Sh& sh, double ccx, double ccy, double ccz) {
   const int lane = __lane_id();
   const int cw = (F32 || HEXA) ? PT_WAVE : g.cw;
   while (npc >= cw) {
     stage_nodes<F32, HEXA, W_t>(W, lane < cw ? W.pcbuf[lane] : 0, cw, g, L, gn, gn32, hn, b, bf,
-                                ox, oy, oz, ccx, ccy, ccz);
+                                sh, ccx, ccy, ccz);
     const int rest = npc - cw;
     const int32_t v = lane < rest ? W.pcbuf[cw + lane] : 0;
     __builtin_amdgcn_wave_barrier();
@@ -1413,15 +1288,17 @@ __device__ __forceinline__ void drain_full(W_t& W, int& npc, int& npp, const Gro
     __builtin_amdgcn_wave_barrier();
   }
   if (npp >= PT_WAVE) {
-    do_leaves<F32, W_t>(W, W.ppbeg[lane], W.ppcnt[lane], g, L, px, py, pz, pm, pe, bf, ox, oy, oz,
-                        ccx, ccy, ccz);
+    do_leaves<F32, W_t>(W, W.ppbeg[lane], W.ppcnt[lane], W.entry(lane), g, L, px, py, pz,
+                        pm, pe, bf, sh, ccx, ccy, ccz);
     const int rest = npp - PT_WAVE;
     const int32_t vb = lane < rest ? W.ppbeg[PT_WAVE + lane] : 0;
     const int32_t vc = lane < rest ? W.ppcnt[PT_WAVE + lane] : 0;
+    const int32_t ve = lane < rest ? W.entry(PT_WAVE + lane) : 0;
     __builtin_amdgcn_wave_barrier();
     if (lane < rest) {
       W.ppbeg[lane] = vb;
       W.ppcnt[lane] = vc;
+      W.set_entry(lane, ve);
     }
     npp = rest;
     __builtin_amdgcn_wave_barrier();
@@ -1429,7 +1306,7 @@ __device__ __forceinline__ void drain_full(W_t& W, int& npc, int& npp, const Gro
 }
 
 // Evaluates what is left in the buffers.
-template <bool F32, bool HEXA, typename W_t>
+template <bool F32, bool HEXA, typename W_t, typename Sh>
 __device__ __forceinline__ void drain_rest(W_t& W, int npc, int npp, const Group& g,
                                            Lanes<F32>& L, const GravNode* __restrict__ gn,
                                            const GravNode32* __restrict__ gn32,
@@ -1438,76 +1315,84 @@ __device__ __forceinline__ void drain_rest(W_t& W, int npc, int npp, const Group
                                            const double* __restrict__ py,
                                            const double* __restrict__ pz,
                                            const double* __restrict__ pm,
-                                           const double* __restrict__ pe, double ox, double oy,
-                                           double oz, double ccx, double ccy, double ccz) {
+                                           const double* __restrict__ pe, const Sh& sh, double ccx, double ccy, double ccz) {
   const int lane = __lane_id();
   if (npc > 0) {
     const int32_t id = lane < npc ? W.pcbuf[lane] : 0;
-    stage_nodes<F32, HEXA, W_t>(W, id, npc, g, L, gn, gn32, hn, b, bf, ox, oy, oz, ccx, ccy, ccz);
+    stage_nodes<F32, HEXA, W_t>(W, id, npc, g, L, gn, gn32, hn, b, bf, sh, ccx, ccy, ccz);
   }
   if (npp > 0) {
     const int32_t beg = lane < npp ? W.ppbeg[lane] : 0;
     const int32_t cnt = lane < npp ? W.ppcnt[lane] : 0;
-    do_leaves<F32, W_t>(W, beg, cnt, g, L, px, py, pz, pm, pe, bf, ox, oy, oz, ccx, ccy, ccz);
+    const int32_t ent = lane < npp ? W.entry(lane) : 0;
+    do_leaves<F32, W_t>(W, beg, cnt, ent, g, L, px, py, pz, pm, pe, bf, sh, ccx, ccy, ccz);
   }
+}
+
+// Buffers what a walk visit found: closed nodes and leaf sources, each with
+// its far flag.
+template <bool F32, typename W_t>
+__device__ __forceinline__ void buffer_lane(W_t& W, const WalkLane& r, unsigned long long leafm,
+                                            unsigned long long closem, const BucketF& bf,
+                                            const Lanes<F32>& L, int& npc, int& npp) {
+  if (r.is_closed)
+    W.pcbuf[npc + pt_rank_in(closem)] =
+        node_far_dsq(r.dsq, r.node_soft, bf, L.emax) ? (r.node | kFarNode) : r.node;
+  if (r.is_leaf) {
+    const int k = npp + pt_rank_in(leafm);
+    W.ppbeg[k] = r.begin;
+    W.ppcnt[k] = leaf_far_dsq(r.dsq, r.leaf_reach, r.leaf_soft, bf, L.emax)
+                     ? (r.count | kFarLeaf)
+                     : r.count;
+    W.set_entry(k, r.node);
+  }
+  npc += __popcll(closem);
+  npp += __popcll(leafm);
+  __builtin_amdgcn_wave_barrier();
 }
 
 // The walk of one bucket below the opened nodes on the stack ([0, sp); the
 // entries from `limit` up are kept), its chunks evaluated as they fill.
 // w_open / w_close: this walk's open() outcomes; lane_leaf_parts: the
 // source-leaf particles this lane visited.
-template <bool F32, int STACK, bool HEXA>
+template <bool F32, int STACK, bool HEXA, typename Sh>
 __device__ __forceinline__ void walk_below(
-    typename FusedLdsOf<F32, STACK, HEXA>::type& W, int& sp, int& npc, int& npp, int limit, const Bucket& b,
+    typename FusedLdsOf<F32, STACK, HEXA, Sh>::type& W, int& sp, int& npc, int& npp, int limit, const Bucket& b,
     const BucketF& bf, const Group& g, Lanes<F32>& L, const TreeNode* __restrict__ nodes,
     const GravNode* __restrict__ gn, const GravNode32* __restrict__ gn32,
     const HexOpen* __restrict__ ho, const HexNode* __restrict__ hn, double gm,
     const double* __restrict__ px, const double* __restrict__ py, const double* __restrict__ pz,
-    const double* __restrict__ pm, const double* __restrict__ pe, double gf, double ox,
-    double oy, double oz, double ccx, double ccy, double ccz, int& w_open, int& w_close,
+    const double* __restrict__ pm, const double* __restrict__ pe, double gf, const Sh& sh, double ccx, double ccy, double ccz, int& w_open, int& w_close,
     int& lane_leaf_parts, bool& overflow) {
-  using W_t = typename FusedLdsOf<F32, STACK, HEXA>::type;
+  using W_t = typename FusedLdsOf<F32, STACK, HEXA, Sh>::type;
   WalkCounts wc;
   while (sp > 0) {
     unsigned long long leafm, closem;
-    const WalkLane r = pt_walk_step<STACK, HEXA, false>(nodes, b, gf, ox, oy, oz, W.stack, sp,
-                                                        overflow, wc, leafm, closem, ho, gm, limit);
+    const WalkLane r = pt_walk_step<HEXA, false>(nodes, b, gf, sh, W.stack, sp, overflow, wc,
+                                                 leafm, closem, ho, gm, limit);
     w_open += wc.n_open;
     w_close += wc.n_close;
     lane_leaf_parts += r.is_leaf ? r.count : 0;
-    if (r.is_closed)
-      W.pcbuf[npc + pt_rank_in(closem)] =
-          node_far_dsq(r.dsq, r.node_soft, bf, L.emax) ? (r.node | kFarNode) : r.node;
-    if (r.is_leaf) {
-      const int k = npp + pt_rank_in(leafm);
-      W.ppbeg[k] = r.begin;
-      W.ppcnt[k] = leaf_far_dsq(r.dsq, r.leaf_reach, r.leaf_soft, bf, L.emax)
-                       ? (r.count | kFarLeaf)
-                       : r.count;
-    }
-    npc += __popcll(closem);
-    npp += __popcll(leafm);
-    __builtin_amdgcn_wave_barrier();
-    drain_full<F32, HEXA, W_t>(W, npc, npp, g, L, gn, gn32, hn, b, bf, px, py, pz, pm, pe, ox, oy, oz, ccx,
+    buffer_lane<F32, W_t>(W, r, leafm, closem, bf, L, npc, npp);
+    drain_full<F32, HEXA, W_t>(W, npc, npp, g, L, gn, gn32, hn, b, bf, px, py, pz, pm, pe, sh, ccx,
                          ccy, ccz);
   }
 }
 
 // One target bucket of the fused kernel: the walk for the bucket box with
 // the bucket's chunks evaluated as they fill, counters added to the wave's.
-template <bool F32, int STACK, bool HEXA>
+template <bool F32, int STACK, bool HEXA, typename Sh>
 __device__ __forceinline__ void gravity_bucket(
-    typename FusedLdsOf<F32, STACK, HEXA>::type& W, int64_t bi, const Bucket* __restrict__ bk,
+    typename FusedLdsOf<F32, STACK, HEXA, Sh>::type& W, int64_t bi, const Bucket* __restrict__ bk,
     const TreeNode* __restrict__ nodes, const GravNode* __restrict__ gn,
     const GravNode32* __restrict__ gn32,
     const HexOpen* __restrict__ ho, const HexNode* __restrict__ hn, double gm, const double* __restrict__ px,
     const double* __restrict__ py, const double* __restrict__ pz, const double* __restrict__ pm,
-    const double* __restrict__ pe, double gf, double ox, double oy, double oz,
+    const double* __restrict__ pe, double gf, const Sh& sh,
     double* __restrict__ ax, double* __restrict__ ay, double* __restrict__ az,
     double* __restrict__ pot, unsigned long long& c_node, unsigned long long& c_part,
     unsigned long long& c_open, unsigned long long& c_close, bool& overflow, bool acc) {
-  using W_t = typename FusedLdsOf<F32, STACK, HEXA>::type;
-  const int lane = threadIdx.x & (PT_WAVE - 1);
+  using W_t = typename FusedLdsOf<F32, STACK, HEXA, Sh>::type;
   const Bucket b = bk[bi];
   const int64_t nt = b.count;
   const double ccx = (b.lox + b.hix) * 0.5, ccy = (b.loy + b.hiy) * 0.5,
@@ -1522,28 +1407,26 @@ __device__ __forceinline__ void gravity_bucket(
     int npc = 0, npp = 0;
     int w_open = 0, w_close = 0;
     int lane_leaf_parts = 0;
-    {
+    // the replicas' roots 64 at a time, each batch walked to the end
+    for (int r0 = 0; r0 < sh.roots(); r0 += PT_WAVE) {
+      const bool active = r0 + (int)__lane_id() < sh.roots();
+      const int32_t e = sh.root(active ? r0 + (int)__lane_id() : r0);
       WalkCounts wc;
-      const WalkLane r = pt_walk_root<HEXA>(nodes, b, gf, ox, oy, oz, W.stack, sp, wc, ho, gm);
-      if (r.is_closed) {
-        if (lane == 0) W.pcbuf[0] = 0;
-        npc = 1;
-      } else if (r.is_leaf) {
-        if (lane == 0) {
-          W.ppbeg[0] = r.begin;
-          W.ppcnt[0] = r.count;
-        }
-        npp = 1;
-      }
-      w_open = wc.n_open;
-      w_close = wc.n_close;
-      lane_leaf_parts = lane == 0 ? wc.leaf_parts : 0;
+      unsigned long long leafm, closem;
+      const WalkLane r = pt_walk_visit<HEXA, false>(nodes, b, gf, sh, active, e, W.stack, sp,
+                                                    overflow, wc, leafm, closem, ho, gm, STACK);
+      w_open += wc.n_open;
+      w_close += wc.n_close;
+      lane_leaf_parts += r.is_leaf ? r.count : 0;
+      buffer_lane<F32, W_t>(W, r, leafm, closem, bf, L, npc, npp);
+      if constexpr (Sh::kRep)
+        drain_full<F32, HEXA, W_t>(W, npc, npp, g, L, gn, gn32, hn, b, bf, px, py, pz, pm, pe, sh,
+                                   ccx, ccy, ccz);
+      walk_below<F32, STACK, HEXA>(W, sp, npc, npp, STACK, b, bf, g, L, nodes, gn, gn32, ho, hn,
+                                   gm, px, py, pz, pm, pe, gf, sh, ccx, ccy, ccz, w_open, w_close,
+                                   lane_leaf_parts, overflow);
     }
-    __builtin_amdgcn_wave_barrier();
-    walk_below<F32, STACK, HEXA>(W, sp, npc, npp, STACK, b, bf, g, L, nodes, gn, gn32, ho, hn, gm, px, py, pz, pm,
-                           pe, gf, ox, oy, oz, ccx, ccy, ccz, w_open, w_close, lane_leaf_parts,
-                           overflow);
-    drain_rest<F32, HEXA, W_t>(W, npc, npp, g, L, gn, gn32, hn, b, bf, px, py, pz, pm, pe, ox, oy, oz, ccx,
+    drain_rest<F32, HEXA, W_t>(W, npc, npp, g, L, gn, gn32, hn, b, bf, px, py, pz, pm, pe, sh, ccx,
                          ccy, ccz);
     if (count) {
       c_open += (unsigned)w_open;
@@ -1656,17 +1539,18 @@ constexpr int kSubTargets = 16;
 // growing down from res_top (anything else).  used_top: entries above
 // res_top held by enclosing residual lists.  Returns false, writing nothing,
 // when the entries would not fit with kMemberReserve to spare.
-template <bool F32, int STACK, bool HEXA>
+template <bool F32, int STACK, bool HEXA, typename Sh>
 __device__ __forceinline__ bool shared_visit(
-    typename FusedLdsOf<F32, STACK, HEXA>::type& W, int32_t node, bool active, const TreeNode* __restrict__ nodes,
+    typename FusedLdsOf<F32, STACK, HEXA, Sh>::type& W, int32_t node, bool active, const TreeNode* __restrict__ nodes,
     const Bucket* __restrict__ mb, int mG, const Bucket& ub, const BucketF& ubf, float emax,
-    double gf, const HexOpen* __restrict__ ho, double gm, double ox, double oy, double oz,
+    double gf, const HexOpen* __restrict__ ho, double gm, const Sh& sh,
     int& sp, int& npc, int& npp, int& nres,
     int res_top, int& sh_open, int& sh_close, int& lane_leaf_parts) {
-  const TreeNode nd = nodes[node];
+  const TreeNode nd = nodes[sh.id(node)];
+  const Off3 o = sh.at(node);
   const bool leaf = active && nd.type == PT_NODE_LEAF;
   const bool internal = active && nd.type == PT_NODE_INTERNAL;
-  const double cx = nd.cx + ox, cy = nd.cy + oy, cz = nd.cz + oz;
+  const double cx = nd.cx + o.x, cy = nd.cy + o.y, cz = nd.cz + o.z;
   const double dsq = pt_box_point_dsq(ub, cx, cy, cz);
   bool op = false, cl = false;
   if (internal) {
@@ -1689,11 +1573,12 @@ __device__ __forceinline__ bool shared_visit(
       } else {
         bool any_open = false, any_closed = false;
         for (int k = 0; k < mG; k++) {
-          bool o;
-          if constexpr (HEXA) o = pt_gv_open_hexa(nd, ho[node], mb[k], gf, gm, ox, oy, oz);
-          else o = pt_box_point_dsq(mb[k], cx, cy, cz) <= rsq;
-          any_open |= o;
-          any_closed |= !o;
+          bool mo;
+          if constexpr (HEXA)
+            mo = pt_gv_open_hexa(nd, ho[sh.id(node)], mb[k], gf, gm, o.x, o.y, o.z);
+          else mo = pt_box_point_dsq(mb[k], cx, cy, cz) <= rsq;
+          any_open |= mo;
+          any_closed |= !mo;
         }
         op = !any_closed;
         cl = !any_open;
@@ -1708,7 +1593,7 @@ __device__ __forceinline__ bool shared_visit(
   const int held = STACK - res_top + nres + n_res;  // residual entries after this visit
   if (sp + n_open + held > STACK || held > STACK - kMemberReserve) return false;
   __builtin_amdgcn_wave_barrier();
-  if (op) W.stack[sp + pt_rank_in(openm)] = nd.first_child;
+  if (op) W.stack[sp + pt_rank_in(openm)] = sh.with(node, nd.first_child);
   if (res) W.stack[res_top - 1 - (nres + pt_rank_in(resm))] = node;
   if (shared_close) W.pcbuf[npc + pt_rank_in(closem)] = node | kFarNode;
   if (leaf) {
@@ -1716,6 +1601,7 @@ __device__ __forceinline__ bool shared_visit(
     W.ppbeg[k] = nd.begin;
     W.ppcnt[k] = leaf_far_dsq(dsq, nd.leaf_reach, nd.leaf_soft, ubf, emax) ? (nd.count | kFarLeaf)
                                                                             : nd.count;
+    W.set_entry(k, node);
   }
   lane_leaf_parts += leaf ? nd.count : 0;
   sp += n_open;
@@ -1736,19 +1622,18 @@ __device__ __forceinline__ bool shared_visit(
 // added by the lanes base + t that wrote the group's sums (base >= 0), and
 // the counters take every member's shared calls.  Returns false with nothing
 // written or counted when the lists overflow.
-template <bool F32, int STACK, bool HEXA>
+template <bool F32, int STACK, bool HEXA, typename Sh>
 __device__ __forceinline__ bool shared_walk(
-    typename FusedLdsOf<F32, STACK, HEXA>::type& W, const Bucket* __restrict__ bk, int64_t mb0, int mG, int seed_top,
+    typename FusedLdsOf<F32, STACK, HEXA, Sh>::type& W, const Bucket* __restrict__ bk, int64_t mb0, int mG, int seed_top,
     int nseed, int res_top, int& nres, int base, const TreeNode* __restrict__ nodes,
     const GravNode* __restrict__ gn, const GravNode32* __restrict__ gn32,
     const HexOpen* __restrict__ ho, const HexNode* __restrict__ hn, double gm,
     const double* __restrict__ px, const double* __restrict__ py, const double* __restrict__ pz,
-    const double* __restrict__ pm, const double* __restrict__ pe, double gf, double ox,
-    double oy, double oz, double* __restrict__ ax, double* __restrict__ ay,
+    const double* __restrict__ pm, const double* __restrict__ pe, double gf, const Sh& sh, double* __restrict__ ax, double* __restrict__ ay,
     double* __restrict__ az, double* __restrict__ pot, unsigned long long& c_node,
     unsigned long long& c_part, unsigned long long& c_open, unsigned long long& c_close,
     bool acc) {
-  using W_t = typename FusedLdsOf<F32, STACK, HEXA>::type;
+  using W_t = typename FusedLdsOf<F32, STACK, HEXA, Sh>::type;
   const int lane = threadIdx.x & (PT_WAVE - 1);
   const Bucket* mb = bk + mb0;
   Bucket ub = mb[0];
@@ -1773,33 +1658,30 @@ __device__ __forceinline__ bool shared_walk(
   int sp = 0, npc = 0, npp = 0;
   int sh_open = 0, sh_close = 0, lane_leaf_parts = 0;
   nres = 0;
-  // seeds 64 at a time (the root alone from the top), each batch walked to
-  // the end
-  const int nbatch = nseed < 0 ? 1 : nseed;
+  // seeds (the replicas' roots from the top) 64 at a time, each batch walked
+  // to the end
+  const int nbatch = nseed < 0 ? sh.roots() : nseed;
   for (int r0 = 0; r0 < nbatch; r0 += PT_WAVE) {
-    const bool active = nseed < 0 ? lane == 0 : r0 + lane < nseed;
-    const int32_t node = nseed < 0 ? 0 : W.stack[seed_top - 1 - (active ? r0 + lane : r0)];
-    if (!shared_visit<F32, STACK, HEXA>(W, node, active, nodes, mb, mG, ub, ubf, L.emax, gf, ho, gm, ox, oy, oz,
-                                  sp, npc, npp, nres, res_top, sh_open, sh_close,
+    const bool active = r0 + lane < nbatch;
+    const int k0 = active ? r0 + lane : r0;
+    const int32_t node = nseed < 0 ? sh.root(k0) : W.stack[seed_top - 1 - k0];
+    if (!shared_visit<F32, STACK, HEXA>(W, node, active, nodes, mb, mG, ub, ubf, L.emax, gf, ho, gm, sh, sp, npc, npp, nres, res_top, sh_open, sh_close,
                                   lane_leaf_parts))
       return false;
-    drain_full<F32, HEXA, W_t>(W, npc, npp, g, L, gn, gn32, hn, ub, ubf, px, py, pz, pm, pe, ox, oy, oz,
-                         gcx, gcy, gcz);
+    drain_full<F32, HEXA, W_t>(W, npc, npp, g, L, gn, gn32, hn, ub, ubf, px, py, pz, pm, pe, sh, gcx, gcy, gcz);
     while (sp > 0) {
       const int k = sp < 8 ? sp : 8;
       sp -= k;
       const int slot = lane >> 3;
       const bool act = slot < k;
       const int32_t child = W.stack[sp + (act ? slot : 0)] + (lane & 7);
-      if (!shared_visit<F32, STACK, HEXA>(W, child, act, nodes, mb, mG, ub, ubf, L.emax, gf, ho, gm, ox, oy,
-                                    oz, sp, npc, npp, nres, res_top, sh_open, sh_close,
+      if (!shared_visit<F32, STACK, HEXA>(W, child, act, nodes, mb, mG, ub, ubf, L.emax, gf, ho, gm, sh, sp, npc, npp, nres, res_top, sh_open, sh_close,
                                     lane_leaf_parts))
         return false;
-      drain_full<F32, HEXA, W_t>(W, npc, npp, g, L, gn, gn32, hn, ub, ubf, px, py, pz, pm, pe, ox, oy, oz,
-                           gcx, gcy, gcz);
+      drain_full<F32, HEXA, W_t>(W, npc, npp, g, L, gn, gn32, hn, ub, ubf, px, py, pz, pm, pe, sh, gcx, gcy, gcz);
     }
   }
-  drain_rest<F32, HEXA, W_t>(W, npc, npp, g, L, gn, gn32, hn, ub, ubf, px, py, pz, pm, pe, ox, oy, oz, gcx,
+  drain_rest<F32, HEXA, W_t>(W, npc, npp, g, L, gn, gn32, hn, ub, ubf, px, py, pz, pm, pe, sh, gcx,
                        gcy, gcz);
   // every member made each shared call
   c_open += (unsigned long long)sh_open * mG;
@@ -1819,23 +1701,23 @@ __device__ __forceinline__ bool shared_walk(
 // its shared walk gave up).  Returns false, having written nothing and
 // counted nothing, when the group's shared walk gives up; the caller then
 // walks each member on its own.
-template <bool F32, int STACK, bool HEXA>
+template <bool F32, int STACK, bool HEXA, typename Sh>
 __device__ __forceinline__ bool gravity_group(
-    typename FusedLdsOf<F32, STACK, HEXA>::type& W, int64_t b0, int G, const Bucket* __restrict__ bk,
+    typename FusedLdsOf<F32, STACK, HEXA, Sh>::type& W, int64_t b0, int G, const Bucket* __restrict__ bk,
     const TreeNode* __restrict__ nodes, const GravNode* __restrict__ gn,
     const GravNode32* __restrict__ gn32,
     const HexOpen* __restrict__ ho, const HexNode* __restrict__ hn, double gm, const double* __restrict__ px,
     const double* __restrict__ py, const double* __restrict__ pz, const double* __restrict__ pm,
-    const double* __restrict__ pe, double gf, double ox, double oy, double oz,
+    const double* __restrict__ pe, double gf, const Sh& sh,
     double* __restrict__ ax, double* __restrict__ ay, double* __restrict__ az,
     double* __restrict__ pot, unsigned long long& c_node, unsigned long long& c_part,
     unsigned long long& c_open, unsigned long long& c_close, bool& overflow, bool acc) {
-  using W_t = typename FusedLdsOf<F32, STACK, HEXA>::type;
+  using W_t = typename FusedLdsOf<F32, STACK, HEXA, Sh>::type;
   const int lane = threadIdx.x & (PT_WAVE - 1);
   const int64_t first = bk[b0].begin;
   int nres = 0;
   if (!shared_walk<F32, STACK, HEXA>(W, bk, b0, G, STACK, -1, STACK, nres, -1, nodes, gn, gn32, ho, hn, gm, px, py,
-                               pz, pm, pe, gf, ox, oy, oz, ax, ay, az, pot, c_node, c_part, c_open,
+                               pz, pm, pe, gf, sh, ax, ay, az, pot, c_node, c_part, c_open,
                                c_close, acc))
     return false;
   if (nres == 0) return true;
@@ -1849,7 +1731,7 @@ __device__ __forceinline__ bool gravity_group(
       int nres2 = 0;
       if (shared_walk<F32, STACK, HEXA>(W, bk, b0 + k0, k1 - k0, STACK, nres, STACK - nres, nres2,
                                   (int)(bk[b0 + k0].begin - first), nodes, gn, gn32, ho, hn, gm, px, py, pz,
-                                  pm, pe, gf, ox, oy, oz, ax, ay, az, pot, c_node, c_part, c_open,
+                                  pm, pe, gf, sh, ax, ay, az, pot, c_node, c_part, c_open,
                                   c_close, acc)) {
         seed_top = STACK - nres;
         nseed = nres2;
@@ -1873,16 +1755,18 @@ __device__ __forceinline__ bool gravity_group(
       for (int r0 = 0; r0 < nseed; r0 += PT_WAVE) {
         const bool active = r0 + lane < nseed;
         const int32_t node = W.stack[seed_top - 1 - (active ? r0 + lane : r0)];
-        const TreeNode nd = nodes[node];
-        const double dsq = pt_box_point_dsq(b, nd.cx + ox, nd.cy + oy, nd.cz + oz);
+        const TreeNode nd = nodes[sh.id(node)];
+        const Off3 o = sh.at(node);
+        const double dsq = pt_box_point_dsq(b, nd.cx + o.x, nd.cy + o.y, nd.cz + o.z);
         bool op;
-        if constexpr (HEXA) op = active && pt_gv_open_hexa(nd, ho[node], b, gf, gm, ox, oy, oz);
+        if constexpr (HEXA)
+          op = active && pt_gv_open_hexa(nd, ho[sh.id(node)], b, gf, gm, o.x, o.y, o.z);
         else op = active && pt_gv_open_dsq(nd, gf, dsq);
         const bool cl = active && !op;
         const unsigned long long openm = __ballot(op), closem = __ballot(cl);
         const int n_open = __popcll(openm);
         __builtin_amdgcn_wave_barrier();
-        if (op) W.stack[pt_rank_in(openm)] = nd.first_child;
+        if (op) W.stack[pt_rank_in(openm)] = sh.with(node, nd.first_child);
         if (cl)
           W.pcbuf[npc + pt_rank_in(closem)] =
               node_far_dsq(dsq, nd.node_soft, bf, L.emax) ? (node | kFarNode) : node;
@@ -1891,15 +1775,13 @@ __device__ __forceinline__ bool gravity_group(
         w_open += n_open;
         w_close += __popcll(closem);
         __builtin_amdgcn_wave_barrier();
-        drain_full<F32, HEXA, W_t>(W, npc, npp, g, L, gn, gn32, hn, b, bf, px, py, pz, pm, pe, ox, oy, oz,
-                             ccx, ccy, ccz);
+        drain_full<F32, HEXA, W_t>(W, npc, npp, g, L, gn, gn32, hn, b, bf, px, py, pz, pm, pe, sh, ccx, ccy, ccz);
         walk_below<F32, STACK, HEXA>(W, sp, npc, npp, limit, b, bf, g, L, nodes, gn, gn32, ho, hn, gm, px, py, pz,
-                               pm, pe, gf, ox, oy, oz, ccx, ccy, ccz, w_open, w_close,
+                               pm, pe, gf, sh, ccx, ccy, ccz, w_open, w_close,
                                lane_leaf_parts, overflow);
         if (overflow) return true;
       }
-      drain_rest<F32, HEXA, W_t>(W, npc, npp, g, L, gn, gn32, hn, b, bf, px, py, pz, pm, pe, ox, oy, oz,
-                           ccx, ccy, ccz);
+      drain_rest<F32, HEXA, W_t>(W, npc, npp, g, L, gn, gn32, hn, b, bf, px, py, pz, pm, pe, sh, ccx, ccy, ccz);
       const int64_t nt = b.count;
       c_open += (unsigned)w_open;
       c_close += (unsigned)w_close;
@@ -1921,35 +1803,39 @@ __device__ __forceinline__ bool gravity_group(
 // fewer resident waves; the FP64 kernel gains from the dynamic balance.)
 // The FP32C kernel is compiled for six waves per SIMD (80 VGPRs, a 40-byte
 // spill): 3.79 ms against 3.95 ms at five on the 1M Plummer.
-template <bool F32, int STACK, bool OFF>
-__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(F32 && STACK == kSmallStack ? 6 : 1, 8)))
+// HEXADECAPOLE: one work-group per 4 buckets in both forms.
+template <bool F32, int STACK, bool HEXA>
+constexpr int bucket_waves_per_eu() {
+  if (STACK != kSmallStack) return 1;
+  return HEXA ? (F32 ? kHexaWaves32 : kHexaWaves) : (F32 ? 6 : 1);
+}
+
+template <bool F32, int STACK, bool HEXA, typename Sh>
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(bucket_waves_per_eu<F32, STACK, HEXA>(), 8)))
 gravity_kernel(const Bucket* __restrict__ bk, int64_t nb, const TreeNode* __restrict__ nodes,
                const GravNode* __restrict__ gn, const GravNode32* __restrict__ gn32,
+               const HexOpen* __restrict__ ho, const HexNode* __restrict__ hn,
                const double* __restrict__ px,
                const double* __restrict__ py, const double* __restrict__ pz,
-               const double* __restrict__ pm, const double* __restrict__ pe, double gf,
-               double ox_in, double oy_in, double oz_in, double* __restrict__ ax,
+               const double* __restrict__ pm, const double* __restrict__ pe, double gf, double gm,
+               Sh sh, double* __restrict__ ax,
                double* __restrict__ ay, double* __restrict__ az, double* __restrict__ pot,
                unsigned long long* __restrict__ partials, int32_t* __restrict__ err,
                unsigned long long* __restrict__ queue, int acc) {
-  using W_t = WaveLds<F32, STACK>;
+  using W_t = typename FusedLdsOf<F32, STACK, HEXA, Sh>::type;
   __shared__ W_t lds[kWaves];
   __shared__ unsigned long long s_cnt[kWaves][4];
-  // without a replica offset the offset is -0.0, which every v + offset
-  // folds away exactly (v + -0.0 == v for every v, -0.0 included)
-  const double ox = OFF ? ox_in : -0.0, oy = OFF ? oy_in : -0.0, oz = OFF ? oz_in : -0.0;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PT_WAVE);
   const int lane = threadIdx.x & (PT_WAVE - 1);
   W_t& W = lds[wave];
   unsigned long long c_node = 0, c_part = 0, c_open = 0, c_close = 0;
   bool overflow = false;
-  if constexpr (F32) {
+  if constexpr (F32 || HEXA) {
     const int64_t bi = pt_xcd_block(blockIdx.x, gridDim.x) * kWaves + wave;
     if (bi < nb)
-      gravity_bucket<F32, STACK, false>(W, bi, bk, nodes, gn, gn32, nullptr, nullptr, 0.0, px, py,
-                                        pz, pm, pe, gf, ox, oy, oz,
-                                 ax, ay, az, pot, c_node, c_part, c_open, c_close, overflow,
-                                 acc != 0);
+      gravity_bucket<F32, STACK, HEXA>(W, bi, bk, nodes, gn, gn32, ho, hn, gm, px, py, pz, pm, pe,
+                                       gf, sh, ax, ay, az, pot, c_node, c_part, c_open, c_close,
+                                       overflow, acc != 0);
   } else {
     const int xcd = blockIdx.x % 8;
     const int64_t b_lo = nb * xcd / 8, b_hi = nb * (xcd + 1) / 8;
@@ -1959,10 +1845,9 @@ gravity_kernel(const Bucket* __restrict__ bk, int64_t nb, const TreeNode* __rest
       // the next index is fetched now and used after this bucket
       unsigned long long next = 0;
       if (lane == 0) next = atomicAdd(&queue[xcd], 1ull);
-      gravity_bucket<F32, STACK, false>(W, bi, bk, nodes, gn, gn32, nullptr, nullptr, 0.0, px, py,
-                                        pz, pm, pe, gf, ox, oy, oz,
-                                 ax, ay, az, pot, c_node, c_part, c_open, c_close, overflow,
-                                 acc != 0);
+      gravity_bucket<F32, STACK, HEXA>(W, bi, bk, nodes, gn, gn32, ho, hn, gm, px, py, pz, pm, pe,
+                                       gf, sh, ax, ay, az, pot, c_node, c_part, c_open, c_close,
+                                       overflow, acc != 0);
       bi = b_lo + (int64_t)__shfl(next, 0, PT_WAVE);
     }
   }
@@ -1998,7 +1883,7 @@ constexpr int kGroupStack32 = 512;
 constexpr int kGroupStack64 = 384;
 constexpr int kGroupStackHexa = 384;  // the HEXADECAPOLE build, both forms
 
-template <bool F32, int STACK, bool OFF, bool HEXA>
+template <bool F32, int STACK, bool HEXA, typename Sh>
 __global__ void __launch_bounds__(kGWaves * PT_WAVE)
 grouped_gravity_kernel(const Bucket* __restrict__ bk, const int32_t* __restrict__ gfirst,
                        const int32_t* __restrict__ gnb, const uint32_t* __restrict__ ngroups,
@@ -2007,14 +1892,13 @@ grouped_gravity_kernel(const Bucket* __restrict__ bk, const int32_t* __restrict_
                        const HexNode* __restrict__ hn, const double* __restrict__ px,
                        const double* __restrict__ py, const double* __restrict__ pz,
                        const double* __restrict__ pm, const double* __restrict__ pe, double gf,
-                       double gm, double ox_in, double oy_in, double oz_in, double* __restrict__ ax,
+                       double gm, Sh sh, double* __restrict__ ax,
                        double* __restrict__ ay, double* __restrict__ az, double* __restrict__ pot,
                        unsigned long long* __restrict__ partials, int32_t* __restrict__ err,
                        int acc) {
-  using W_t = typename FusedLdsOf<F32, STACK, HEXA>::type;
+  using W_t = typename FusedLdsOf<F32, STACK, HEXA, Sh>::type;
   __shared__ W_t lds[kGWaves];
   __shared__ unsigned long long s_cnt[kGWaves][4];
-  const double ox = OFF ? ox_in : -0.0, oy = OFF ? oy_in : -0.0, oz = OFF ? oz_in : -0.0;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PT_WAVE);
   const int lane = threadIdx.x & (PT_WAVE - 1);
   W_t& W = lds[wave];
@@ -2031,13 +1915,13 @@ grouped_gravity_kernel(const Bucket* __restrict__ bk, const int32_t* __restrict_
     // walk per bucket
     const bool done =
         G > 1 && gravity_group<F32, STACK, HEXA>(W, b0, G, bk, nodes, gn, gn32, ho, hn, gm, px,
-                                                 py, pz, pm, pe, gf, ox, oy, oz, ax, ay, az, pot,
+                                                 py, pz, pm, pe, gf, sh, ax, ay, az, pot,
                                                  c_node, c_part, c_open, c_close, overflow,
                                                  acc != 0);
     if (!done) {
       for (int k = 0; k < G; k++)
         gravity_bucket<F32, STACK, HEXA>(W, b0 + k, bk, nodes, gn, gn32, ho, hn, gm, px, py, pz,
-                                         pm, pe, gf, ox, oy, oz, ax, ay, az, pot, c_node, c_part,
+                                         pm, pe, gf, sh, ax, ay, az, pot, c_node, c_part,
                                          c_open, c_close, overflow, acc != 0);
     }
   }
@@ -2120,9 +2004,9 @@ inline unsigned grid_for(int64_t nb) { return (unsigned)((nb + kWaves - 1) / kWa
 // resident grid, 8 per CU (at least what fits on a CU; work-groups that do
 // not fit start as others finish -- none waits on another), a multiple of 8
 // (one share per XCD), capped by the bucket count.
-int64_t pt_gravity_blocks(int64_t nb, int precision) {
+int64_t pt_gravity_blocks(int64_t nb, int precision, bool hexa) {
   const int64_t need = (nb + kWaves - 1) / kWaves;
-  if (precision != 0) return need;
+  if (precision != 0 || hexa) return need;
   static int64_t cap = 0;
   if (cap == 0) {
     int dev = 0, cus = 0;
@@ -2166,61 +2050,45 @@ int pt_launch_interact_hexa(const Bucket* bk, int64_t nb, const TreeNode* nodes,
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-// Fused HEXADECAPOLE evaluation: one work-group per 4 buckets.
-int64_t pt_hexa_gravity_blocks(int64_t nb) { return (nb + kWaves - 1) / kWaves; }
-
-int pt_launch_hexa_gravity(int precision, bool big_stack, const Bucket* bk, int64_t nb,
-                           const TreeNode* nodes, const HexOpen* ho, const HexNode* hn,
-                           const double* x, const double* y, const double* z, const double* m,
-                           const double* e, double gf, double gm, const double off[3],
-                           double* ax, double* ay, double* az, double* pot,
-                           unsigned long long* partials, int32_t* err, bool accumulate,
-                           hipStream_t s) {
-  if (nb <= 0) return 0;
-  const unsigned grid = (unsigned)pt_hexa_gravity_blocks(nb);
-#define PT_HEXA_LAUNCH(STACK, F32)                                                               \
-  hexa_gravity_kernel<STACK, F32><<<grid, kThreads, 0, s>>>(                                   \
-      bk, nb, nodes, ho, hn, x, y, z, m, e, gf, gm, off[0], off[1], off[2], ax, ay, az, pot,    \
-      partials, err, accumulate ? 1 : 0)
-  if (precision == 0) {
-    if (big_stack) PT_HEXA_LAUNCH(kBigStack, false);
-    else PT_HEXA_LAUNCH(kSmallStack, false);
-  } else {
-    if (big_stack) PT_HEXA_LAUNCH(kBigStack, true);
-    else PT_HEXA_LAUNCH(kSmallStack, true);
-  }
-#undef PT_HEXA_LAUNCH
-  return hipGetLastError() == hipSuccess ? 0 : -1;
-}
-
 // big_stack selects the kBigStack-entry walk stack (used after a walk with
 // the small stack reported an overflow; 1536 entries keep the FP64
 // work-group under 64 KiB of LDS).
 int pt_launch_gravity(int precision, bool big_stack, const Bucket* bk, int64_t nb,
                       const TreeNode* nodes, const GravNode* gn, const GravNode32* gn32,
-                      const double* x, const double* y, const double* z, const double* m,
-                      const double* e, double gf, const double off[3], double* ax, double* ay, double* az,
-                      double* pot, unsigned long long* partials, int32_t* err,
-                      unsigned long long* queue, bool accumulate, hipStream_t s) {
+                      const HexOpen* ho, const HexNode* hn, const double* x, const double* y,
+                      const double* z, const double* m, const double* e, double gf, double gm,
+                      const PtReplicas* rep, double* ax, double* ay, double* az, double* pot,
+                      unsigned long long* partials, int32_t* err, unsigned long long* queue,
+                      bool accumulate, hipStream_t s) {
   if (nb <= 0) return 0;
+  const bool hexa = ho != nullptr;
   if (pt_launch_fill_u64(queue, 8, 0ull, s) != 0) return -1;
-  const unsigned grid = (unsigned)pt_gravity_blocks(nb, precision);
-  const bool has_off = off[0] != 0.0 || off[1] != 0.0 || off[2] != 0.0;
-#define PT_GRAVITY_LAUNCH(F32, STACK, OFF)                                                     \
-  gravity_kernel<F32, STACK, OFF><<<grid, kThreads, 0, s>>>(                                   \
-      bk, nb, nodes, gn, gn32, x, y, z, m, e, gf, off[0], off[1], off[2], ax, ay, az, pot,      \
-      partials, err, queue, accumulate ? 1 : 0)
-#define PT_GRAVITY_LAUNCH_OFF(F32, STACK)   \
-  if (has_off) PT_GRAVITY_LAUNCH(F32, STACK, true); \
-  else PT_GRAVITY_LAUNCH(F32, STACK, false)
-  if (precision == 0) {
-    if (big_stack) PT_GRAVITY_LAUNCH_OFF(false, kBigStack);
-    else PT_GRAVITY_LAUNCH_OFF(false, kSmallStack);
-  } else {
-    if (big_stack) PT_GRAVITY_LAUNCH_OFF(true, kBigStack);
-    else PT_GRAVITY_LAUNCH_OFF(true, kSmallStack);
+  const unsigned grid = (unsigned)pt_gravity_blocks(nb, precision, hexa);
+#define PT_GRAVITY_LAUNCH(F32, STACK, HEXA, SH)                                              \
+  gravity_kernel<F32, STACK, HEXA><<<grid, kThreads, 0, s>>>(                                \
+      bk, nb, nodes, gn, gn32, ho, hn, x, y, z, m, e, gf, gm, SH, ax, ay, az, pot, partials, \
+      err, queue, accumulate ? 1 : 0)
+#define PT_GRAVITY_LAUNCH_REP(F32, HEXA)                                                     \
+  if (rep) {                                                                                 \
+    const RepShift sh{rep->tab, rep->bits, rep->n};                                          \
+    if (big_stack) PT_GRAVITY_LAUNCH(F32, kBigStack, HEXA, sh);                              \
+    else PT_GRAVITY_LAUNCH(F32, kRepStack, HEXA, sh);                                        \
+  } else {                                                                                   \
+    if (big_stack) PT_GRAVITY_LAUNCH(F32, kBigStack, HEXA, NoShift{});                       \
+    else PT_GRAVITY_LAUNCH(F32, kSmallStack, HEXA, NoShift{});                               \
   }
-#undef PT_GRAVITY_LAUNCH_OFF
+  if (hexa) {
+    if (precision == 0) {
+      PT_GRAVITY_LAUNCH_REP(false, true)
+    } else {
+      PT_GRAVITY_LAUNCH_REP(true, true)
+    }
+  } else if (precision == 0) {
+    PT_GRAVITY_LAUNCH_REP(false, false)
+  } else {
+    PT_GRAVITY_LAUNCH_REP(true, false)
+  }
+#undef PT_GRAVITY_LAUNCH_REP
 #undef PT_GRAVITY_LAUNCH
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
@@ -2259,36 +2127,61 @@ int pt_launch_grouped_gravity(int precision, bool big_stack, const Bucket* bk,
                               const GravNode* gn, const GravNode32* gn32, const HexOpen* ho,
                               const HexNode* hn, const double* x, const double* y,
                               const double* z, const double* m, const double* e, double gf,
-                              double gm, const double off[3], double* ax, double* ay, double* az,
+                              double gm, const PtReplicas* rep, double* ax, double* ay, double* az,
                               double* pot, unsigned long long* partials, int32_t* err,
                               bool accumulate, hipStream_t s) {
   if (nb <= 0) return 0;
   const unsigned grid = (unsigned)pt_grouped_gravity_blocks(nb, n, cap);
-  const bool has_off = off[0] != 0.0 || off[1] != 0.0 || off[2] != 0.0;
   const bool hexa = ho != nullptr;
-#define PT_GROUPED_LAUNCH(F32, STACK, OFF, HEXA)                                               \
-  grouped_gravity_kernel<F32, STACK, OFF, HEXA><<<grid, kGWaves * PT_WAVE, 0, s>>>(            \
-      bk, gfirst, gnb, ngroups, nodes, gn, gn32, ho, hn, x, y, z, m, e, gf, gm, off[0], off[1], \
-      off[2], ax, ay, az, pot, partials, err, accumulate ? 1 : 0)
-#define PT_GROUPED_LAUNCH_OFF(F32, STACK, HEXA)               \
-  if (has_off) PT_GROUPED_LAUNCH(F32, STACK, true, HEXA);     \
-  else PT_GROUPED_LAUNCH(F32, STACK, false, HEXA)
+#define PT_GROUPED_LAUNCH(F32, STACK, HEXA, SH)                                                \
+  grouped_gravity_kernel<F32, STACK, HEXA><<<grid, kGWaves * PT_WAVE, 0, s>>>(                 \
+      bk, gfirst, gnb, ngroups, nodes, gn, gn32, ho, hn, x, y, z, m, e, gf, gm, SH, ax, ay, az, \
+      pot, partials, err, accumulate ? 1 : 0)
+#define PT_GROUPED_LAUNCH_REP(F32, STACK, HEXA)                    \
+  if (rep) {                                                       \
+    const RepShift sh{rep->tab, rep->bits, rep->n};                \
+    if (big_stack) PT_GROUPED_LAUNCH(F32, kBigStack, HEXA, sh);    \
+    else PT_GROUPED_LAUNCH(F32, STACK, HEXA, sh);                  \
+  } else {                                                         \
+    if (big_stack) PT_GROUPED_LAUNCH(F32, kBigStack, HEXA, NoShift{}); \
+    else PT_GROUPED_LAUNCH(F32, STACK, HEXA, NoShift{});           \
+  }
   if (hexa) {
     if (precision == 0) {
-      if (big_stack) PT_GROUPED_LAUNCH_OFF(false, kBigStack, true);
-      else PT_GROUPED_LAUNCH_OFF(false, kGroupStackHexa, true);
+      PT_GROUPED_LAUNCH_REP(false, kGroupStackHexa, true)
     } else {
-      if (big_stack) PT_GROUPED_LAUNCH_OFF(true, kBigStack, true);
-      else PT_GROUPED_LAUNCH_OFF(true, kGroupStackHexa, true);
+      PT_GROUPED_LAUNCH_REP(true, kGroupStackHexa, true)
     }
   } else if (precision == 0) {
-    if (big_stack) PT_GROUPED_LAUNCH_OFF(false, kBigStack, false);
-    else PT_GROUPED_LAUNCH_OFF(false, kGroupStack64, false);
+    PT_GROUPED_LAUNCH_REP(false, kGroupStack64, false)
   } else {
-    if (big_stack) PT_GROUPED_LAUNCH_OFF(true, kBigStack, false);
-    else PT_GROUPED_LAUNCH_OFF(true, kGroupStack32, false);
+    PT_GROUPED_LAUNCH_REP(true, kGroupStack32, false)
   }
-#undef PT_GROUPED_LAUNCH_OFF
+#undef PT_GROUPED_LAUNCH_REP
 #undef PT_GROUPED_LAUNCH
+  return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
+namespace {
+
+// The offsets of the periodic replicas in the order of ExMain::traversalFn
+// (examples/Gravity.C:35-46): X outermost, then Y, then Z, each added to off.
+__global__ void __launch_bounds__(256)
+replica_table_kernel(int nr, Off3 off, Off3 period, double* __restrict__ tab) {
+  const int side = 2 * nr + 1;
+  const int r = blockIdx.x * 256 + threadIdx.x;
+  if (r >= side * side * side) return;
+  tab[3 * r] = off.x + (r / (side * side) - nr) * period.x;
+  tab[3 * r + 1] = off.y + (r / side % side - nr) * period.y;
+  tab[3 * r + 2] = off.z + (r % side - nr) * period.z;
+}
+
+}  // namespace
+
+int pt_launch_replica_table(int nr, const double off[3], const double period[3], double* tab,
+                            hipStream_t s) {
+  const int side = 2 * nr + 1;
+  replica_table_kernel<<<(unsigned)((side * side * side + 255) / 256), 256, 0, s>>>(
+      nr, Off3{off[0], off[1], off[2]}, Off3{period[0], period[1], period[2]}, tab);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }

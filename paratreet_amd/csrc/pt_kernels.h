@@ -130,24 +130,25 @@ int pt_launch_interact_hexa(const Bucket* bk, int64_t nb, const TreeNode* nodes,
                             const int32_t* pp, const int64_t* pc_off, const int32_t* pc,
                             const double off[3], double* ax, double* ay, double* az, double* pot,
                             hipStream_t s);
-// Fused walk + interactions of the HEXADECAPOLE build (FP64), counters as
-// partials of pt_hexa_gravity_blocks(nb) work-groups.
-int64_t pt_hexa_gravity_blocks(int64_t nb);
-// precision 0: FP64; otherwise the compensated-FP32 form of node() and leaf().
-int pt_launch_hexa_gravity(int precision, bool big_stack, const Bucket* bk, int64_t nb,
-                           const TreeNode* nodes, const HexOpen* ho, const HexNode* hn,
-                           const double* x, const double* y, const double* z, const double* m,
-                           const double* e, double gf, double gm, const double off[3],
-                           double* ax, double* ay, double* az, double* pot,
-                           unsigned long long* partials, int32_t* err, bool accumulate,
-                           hipStream_t s);
-int64_t pt_gravity_blocks(int64_t nb, int precision);
+// Offsets of one fused launch: n of them at tab[3 r] (device), walk entries
+// holding a replica's number above `bits` bits of node id, in 30 bits.
+struct PtReplicas {
+  const double* tab;
+  int32_t bits, n;
+};
+int pt_launch_replica_table(int nr, const double off[3], const double period[3], double* tab,
+                            hipStream_t s);
+// One walk per bucket: precision 0 FP64, otherwise the compensated-FP32 form;
+// ho != nullptr: the HEXADECAPOLE build; rep == nullptr: no offset.
+// Counters as partials of pt_gravity_blocks work-groups.
+int64_t pt_gravity_blocks(int64_t nb, int precision, bool hexa);
 int pt_launch_gravity(int precision, bool big_stack, const Bucket* bk, int64_t nb,
                       const TreeNode* nodes, const GravNode* gn, const GravNode32* gn32,
-                      const double* x, const double* y, const double* z, const double* m,
-                      const double* e, double gf, const double off[3], double* ax, double* ay, double* az,
-                      double* pot, unsigned long long* partials, int32_t* err,
-                      unsigned long long* queue, bool accumulate, hipStream_t s);
+                      const HexOpen* ho, const HexNode* hn, const double* x, const double* y,
+                      const double* z, const double* m, const double* e, double gf, double gm,
+                      const PtReplicas* rep, double* ax, double* ay, double* az, double* pot,
+                      unsigned long long* partials, int32_t* err, unsigned long long* queue,
+                      bool accumulate, hipStream_t s);
 
 // Bucket groups of the grouped fused kernel: runs of consecutive buckets of
 // at most cap (2..64) particles in all (a larger bucket alone), formed inside
@@ -172,7 +173,7 @@ int pt_launch_grouped_gravity(int precision, bool big_stack, const Bucket* bk,
                               const GravNode* gn, const GravNode32* gn32, const HexOpen* ho,
                               const HexNode* hn, const double* x, const double* y,
                               const double* z, const double* m, const double* e, double gf,
-                              double gm, const double off[3], double* ax, double* ay, double* az,
+                              double gm, const PtReplicas* rep, double* ax, double* ay, double* az,
                               double* pot, unsigned long long* partials, int32_t* err,
                               bool accumulate, hipStream_t s);
 

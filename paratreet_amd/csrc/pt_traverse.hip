@@ -46,26 +46,20 @@ traverse_kernel(const TreeNode* __restrict__ nodes, const HexOpen* __restrict__ 
   int32_t* ppw = FILL ? pp + pp_off[bi] : nullptr;
   int32_t* pcw = FILL ? pc + pc_off[bi] : nullptr;
   if (live) {
-    WalkCounts wc;
-    const WalkLane r = pt_walk_root<HEXA>(nodes, b, gf, ox, oy, oz, st, sp, wc, ho, gm);
-    if (r.is_leaf) {
-      if (FILL && lane == 0) ppw[0] = 0;
-      npp = 1;
-    } else if (r.is_closed) {
-      if (FILL && lane == 0) pcw[0] = 0;
-      npc = 1;
-    }
-    c_open += wc.n_open;
-    c_close += wc.n_close;
-    c_node += (unsigned long long)wc.n_close * nt;
-    c_part += (unsigned long long)wc.leaf_parts * nt;
-    while (sp > 0) {
+    const OneShift sh{ox, oy, oz};
+    bool first = true;  // the root, then its subtree
+    while (first || sp > 0) {
+      WalkCounts wc;
       unsigned long long leafm, closem;
-      const WalkLane r2 = pt_walk_step<PT_WALK_STACK, HEXA>(nodes, b, gf, ox, oy, oz, st, sp,
-                                                            overflow, wc, leafm, closem, ho, gm);
+      const WalkLane r =
+          first ? pt_walk_visit<HEXA, true>(nodes, b, gf, sh, lane == 0, 0, st, sp, overflow, wc,
+                                            leafm, closem, ho, gm, PT_WALK_STACK)
+                : pt_walk_step<HEXA, true>(nodes, b, gf, sh, st, sp, overflow, wc, leafm, closem,
+                                           ho, gm, PT_WALK_STACK);
+      first = false;
       if (FILL) {
-        if (r2.is_leaf) ppw[npp + pt_rank_in(leafm)] = r2.node;
-        if (r2.is_closed) pcw[npc + pt_rank_in(closem)] = r2.node;
+        if (r.is_leaf) ppw[npp + pt_rank_in(leafm)] = r.node;
+        if (r.is_closed) pcw[npc + pt_rank_in(closem)] = r.node;
       }
       npp += __popcll(leafm);
       npc += __popcll(closem);

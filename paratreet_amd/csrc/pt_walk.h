@@ -155,17 +155,66 @@ __device__ __forceinline__ bool pt_open_any(const TreeNode& s, int32_t id,
   }
 }
 
+// What a walk adds to the sources' positions (GravityVisitor's offset).  A
+// stack or buffer entry is a node id, with the replica's number above `bits`
+// bits in RepShift; flag bits (kFarNode) lie above both.
+struct Off3 {
+  double x, y, z;
+};
+
+// No offset: -0.0, which every v + offset folds away exactly (v + -0.0 == v
+// for every v, -0.0 included).
+struct NoShift {
+  static constexpr bool kRep = false;
+  __device__ __forceinline__ int32_t id(int32_t e) const { return e; }
+  __device__ __forceinline__ Off3 at(int32_t) const { return Off3{-0.0, -0.0, -0.0}; }
+  __device__ __forceinline__ int32_t with(int32_t, int32_t node) const { return node; }
+  __device__ __forceinline__ int32_t roots() const { return 1; }
+  __device__ __forceinline__ int32_t root(int32_t) const { return 0; }
+};
+
+// One offset for every entry.
+struct OneShift {
+  static constexpr bool kRep = false;
+  double x, y, z;
+  __device__ __forceinline__ int32_t id(int32_t e) const { return e; }
+  __device__ __forceinline__ Off3 at(int32_t) const { return Off3{x, y, z}; }
+  __device__ __forceinline__ int32_t with(int32_t, int32_t node) const { return node; }
+  __device__ __forceinline__ int32_t roots() const { return 1; }
+  __device__ __forceinline__ int32_t root(int32_t) const { return 0; }
+};
+
+// Several offsets in one walk, each with its own visit of the tree: replica r
+// of the n at tab[3 r].  One launch per replica left every launch to the
+// latency of its ~10 k short walks (27 launches of 234 us for 50k particles);
+// together the replicas fill the walk's steps and the 64-source chunks, and a
+// bucket's sums are reduced once: 7235 -> 747 us for the whole evaluation.
+struct RepShift {
+  static constexpr bool kRep = true;
+  const double* tab;
+  int32_t bits, n;
+  __device__ __forceinline__ int32_t id(int32_t e) const { return e & ((1 << bits) - 1); }
+  __device__ __forceinline__ Off3 at(int32_t e) const {
+    const double* o = tab + 3 * (e >> bits);
+    return Off3{o[0], o[1], o[2]};
+  }
+  __device__ __forceinline__ int32_t with(int32_t e, int32_t node) const {
+    return ((e >> bits) << bits) | node;
+  }
+  __device__ __forceinline__ int32_t roots() const { return n; }
+  __device__ __forceinline__ int32_t root(int32_t r) const { return r << bits; }
+};
+
 // Result of one walk step for the calling lane.
 struct WalkLane {
-  int32_t node;      // visited node id (valid if active)
+  int32_t node;      // visited entry (valid if active)
   int32_t count;     // its particle count
   int32_t begin;     // its first particle
   bool is_leaf;      // -> leaf() (P-P)
   bool is_closed;    // -> node() (P-C)
-  double cx, cy, cz;        // its centre of mass
   float leaf_reach, leaf_soft;  // leaf bounds (TreeNode)
   float node_soft;              // internal nodes' softening bound (TreeNode)
-  double dsq;                   // squared distance of cx + offset from the bucket box
+  double dsq;                   // squared distance of its centre + offset from the bucket box
 };
 
 // Wave-uniform per-step counts for the interaction counters.
@@ -175,87 +224,40 @@ struct WalkCounts {
   int leaf_parts; // sum of source-leaf particle counts (leaf() calls)
 };
 
-// Visits the root (node 0): pushes its first child when it is opened.  sp and
-// the counts are wave-uniform; lane 0 owns the stack write.
-template <bool HEXA = false>
-__device__ __forceinline__ WalkLane pt_walk_root(const TreeNode* __restrict__ nodes,
-                                                 const Bucket& b, double gf, double ox,
-                                                 double oy, double oz,
-                                                 int32_t* __restrict__ stack, int& sp,
-                                                 WalkCounts& wc,
-                                                 const HexOpen* __restrict__ ho = nullptr,
-                                                 double gm = 0.0) {
-  WalkLane r{0, 0, 0, false, false, 0.0, 0.0, 0.0, 0.f, 0.f, 0.f, 0.0};
-  wc = WalkCounts{0, 0, 0};
-  const TreeNode root = nodes[0];
-  r.count = root.count;
-  r.begin = root.begin;
-  r.cx = root.cx;
-  r.cy = root.cy;
-  r.cz = root.cz;
-  r.leaf_reach = root.leaf_reach;
-  r.leaf_soft = root.leaf_soft;
-  r.node_soft = root.node_soft;
-  r.dsq = pt_box_point_dsq(b, root.cx + ox, root.cy + oy, root.cz + oz);
-  if (root.type == PT_NODE_LEAF) {
-    r.is_leaf = true;
-    wc.leaf_parts = root.count;
-  } else if (root.type == PT_NODE_INTERNAL) {
-    if (pt_open_any<HEXA>(root, 0, ho, b, gf, gm, ox, oy, oz)) {
-      if (__lane_id() == 0) stack[0] = root.first_child;
-      sp = 1;
-      wc.n_open = 1;
-    } else {
-      r.is_closed = true;
-      wc.n_close = 1;
-    }
-  }
-  return r;
-}
-
-// One step: pops up to 8 opened nodes and tests their 64 children.  Returns
-// this lane's child and its classification; pushes opened children.  A push
-// beyond `limit` (<= STACK) entries sets overflow and ends the walk (the
-// caller reports it; nothing is silently dropped).  With SUM_LEAVES false wc.leaf_parts is
-// left 0 and the caller sums the leaf lanes' counts itself.
-template <int STACK, bool HEXA = false, bool SUM_LEAVES = true>
-__device__ __forceinline__ WalkLane pt_walk_step(const TreeNode* __restrict__ nodes,
-                                                 const Bucket& b, double gf, double ox,
-                                                 double oy, double oz,
-                                                 int32_t* __restrict__ stack, int& sp,
-                                                 bool& overflow, WalkCounts& wc,
-                                                 unsigned long long& leafm,
-                                                 unsigned long long& closem,
-                                                 const HexOpen* __restrict__ ho = nullptr,
-                                                 double gm = 0.0, int limit = STACK) {
-  const int lane = __lane_id();
-  const int k = sp < 8 ? sp : 8;
-  sp -= k;
-  const int slot = lane >> 3;
-  const bool active = slot < k;
-  // lanes beyond the k popped entries read the first one's children again
-  // (k >= 1 while the walk runs) and are masked out of every outcome: the
-  // loads need no branch and the lane state no defaults
+// Visits entry e in every active lane (at least one; the other lanes repeat an
+// active lane's entry and are masked out of every outcome, so the loads need
+// no branch and the lane state no defaults) and pushes the first children of
+// the opened nodes.  A push beyond `limit` entries sets overflow and ends the
+// walk (the caller reports it; nothing is silently dropped).  With SUM_LEAVES
+// false wc.leaf_parts is left 0 and the caller sums the leaf lanes' counts
+// itself.  sp and the counts are wave-uniform.
+template <bool HEXA, bool SUM_LEAVES, typename Sh>
+__device__ __forceinline__ WalkLane pt_walk_visit(const TreeNode* __restrict__ nodes,
+                                                  const Bucket& b, double gf, const Sh& sh,
+                                                  bool active, int32_t e,
+                                                  int32_t* __restrict__ stack, int& sp,
+                                                  bool& overflow, WalkCounts& wc,
+                                                  unsigned long long& leafm,
+                                                  unsigned long long& closem,
+                                                  const HexOpen* __restrict__ ho, double gm,
+                                                  int limit) {
   WalkLane r;
-  r.node = stack[sp + (active ? slot : 0)] + (lane & 7);
-  const TreeNode nd = nodes[r.node];
+  r.node = e;
+  const TreeNode nd = nodes[sh.id(e)];
+  const Off3 o = sh.at(e);
   r.count = nd.count;
   r.begin = nd.begin;
-  r.cx = nd.cx;
-  r.cy = nd.cy;
-  r.cz = nd.cz;
   r.leaf_reach = nd.leaf_reach;
   r.leaf_soft = nd.leaf_soft;
   r.node_soft = nd.node_soft;
-  const int32_t fc = nd.first_child;
   r.is_leaf = active && nd.type == PT_NODE_LEAF;
   const bool internal = active && nd.type == PT_NODE_INTERNAL;
   // every lane's box distance: the opening test's for internal nodes, the
   // near / far classification's for leaves and closed nodes
-  r.dsq = pt_box_point_dsq(b, nd.cx + ox, nd.cy + oy, nd.cz + oz);
+  r.dsq = pt_box_point_dsq(b, nd.cx + o.x, nd.cy + o.y, nd.cz + o.z);
   bool op = false;
   if constexpr (HEXA) {
-    if (internal) op = pt_open_any<HEXA>(nd, r.node, ho, b, gf, gm, ox, oy, oz);
+    if (internal) op = pt_open_any<HEXA>(nd, sh.id(e), ho, b, gf, gm, o.x, o.y, o.z);
   } else {
     op = internal && pt_gv_open_dsq(nd, gf, r.dsq);
   }
@@ -273,7 +275,7 @@ __device__ __forceinline__ WalkLane pt_walk_step(const TreeNode* __restrict__ no
     return r;
   }
   __builtin_amdgcn_wave_barrier();
-  if (op) stack[sp + pt_rank_in(openm)] = fc;
+  if (op) stack[sp + pt_rank_in(openm)] = sh.with(e, nd.first_child);
   __builtin_amdgcn_wave_barrier();
   sp += n_open;
   wc.n_open = n_open;
@@ -281,6 +283,27 @@ __device__ __forceinline__ WalkLane pt_walk_step(const TreeNode* __restrict__ no
   if constexpr (SUM_LEAVES) wc.leaf_parts = pt_wave_sum_int(r.is_leaf ? r.count : 0);
   else wc.leaf_parts = 0;
   return r;
+}
+
+// One step: pops up to 8 opened nodes and visits their 64 children (k >= 1
+// while the walk runs).
+template <bool HEXA, bool SUM_LEAVES, typename Sh>
+__device__ __forceinline__ WalkLane pt_walk_step(const TreeNode* __restrict__ nodes,
+                                                 const Bucket& b, double gf, const Sh& sh,
+                                                 int32_t* __restrict__ stack, int& sp,
+                                                 bool& overflow, WalkCounts& wc,
+                                                 unsigned long long& leafm,
+                                                 unsigned long long& closem,
+                                                 const HexOpen* __restrict__ ho, double gm,
+                                                 int limit) {
+  const int lane = __lane_id();
+  const int k = sp < 8 ? sp : 8;
+  sp -= k;
+  const int slot = lane >> 3;
+  const bool active = slot < k;
+  const int32_t e = stack[sp + (active ? slot : 0)] + (lane & 7);
+  return pt_walk_visit<HEXA, SUM_LEAVES>(nodes, b, gf, sh, active, e, stack, sp, overflow, wc,
+                                         leafm, closem, ho, gm, limit);
 }
 
 // XCD-aware bucket order: work-groups are dispatched round-robin over the 8
