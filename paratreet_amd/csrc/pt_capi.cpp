@@ -94,7 +94,6 @@ struct pt_ctx {
   DBuf<double> ewt;  // Ewald Fourier table (periodic build)
   DBuf<int32_t> ewcount;
   DBuf<unsigned long long> cpart;  // per-block counter partials
-  DBuf<unsigned long long> wqueue;  // per-XCD work counters of the fused kernel
   // bucket groups of the grouped fused kernel (pt_set_fused_grouping): 0 one
   // walk per bucket, 1 automatic, 2..64 the groups' particle cap
   int32_t fused_grouping = 1;
@@ -381,7 +380,6 @@ void pt_ctx_destroy(pt_ctx* c) {
   release(c->hraw); release(c->hn); release(c->ho);
   release(c->bucket_node); release(c->nd); release(c->ord_h); release(c->ord_b);
   release(c->tnode); release(c->gn); release(c->gn32); release(c->bk); release(c->cpart);
-  release(c->wqueue);
   release(c->fg_tfirst); release(c->fg_tnb); release(c->fg_first); release(c->fg_nb);
   release(c->fg_wcount); release(c->fg_woff); release(c->fg_ng);
   release(c->pp_cnt); release(c->pc_cnt); release(c->pp); release(c->pc);
@@ -945,16 +943,21 @@ pt_status pt_start_dual(pt_ctx* c, double theta, const double offset[3], uint64_
   return PT_OK;
 }
 
-// Fused walk + interactions (no lists), with a large-stack rerun if the
-// small walk stack (192 entries) overflowed for some bucket.
-// The particle cap of the grouped walk's bucket groups, 0 for one walk per
-// bucket.  Automatic: the largest of 64, 32 and 16 that still gives every
-// resident wave slot (four per SIMD) about six groups, 16 for smaller sets
-// down to one group per slot, and one walk per bucket below that (larger
-// groups share more of the walk, more groups keep the device busy to the
-// end).  Measured on 100k, 256k and 1M Plummer spheres and the 16M halo
-// mixture, this picks the fastest of those caps in each case.
-static int group_cap(pt_ctx* c) {
+// The particle cap of the bucket groups, 0 for one walk per bucket.
+// Automatic: larger groups share more of the walk, more groups keep the device
+// busy to the end, so the cap grows with the particles per resident wave slot
+// (four waves per SIMD).  Whole evaluations, us, at caps 0 / 8 / 16 / 32 / 64
+// (Plummer, buckets of 12 or 16):
+//   FP32C   20k  435 /  470 /  561 /  722       100k  764 /  724 /  766 /  877
+//          200k 1144 / 1068 / 1011 / 1090       524k 2215 / 2015 / 1860 / 1835
+//            1M 3786 / 3361 / 3038 / 2963 / 3162
+//   FP64    10k  310 /  348 /  403               20k  446 /  438 /  525
+//          100k  900 /  830 /  868 / 1045       200k 1420 / 1262 / 1262 / 1376
+//          524k 3129 / 2877 / 2780 / 2831         1M 5711 / 5131 / 4938 / 4973 / 5176
+// (the HEXADECAPOLE build's lie at the same sizes), and at 16M the cap of 64.
+// A walk of 27 replicas has the work of a larger set: 50k 633 / 650 / 730,
+// 200k 1648 / 1526 / 1483.
+static int group_cap(pt_ctx* c, pt_precision precision, int64_t n_rep) {
   if (c->fused_grouping == 0) return 0;
   if (c->fused_grouping >= 2) return c->fused_grouping;
   if (c->n_cus == 0) {
@@ -965,12 +968,16 @@ static int group_cap(pt_ctx* c) {
       cus = 256;
     c->n_cus = cus;
   }
-  const int64_t slots = (int64_t)c->n_cus * 16;
-  for (int cap = 64; cap >= 32; cap /= 2)
-    if (c->n >= 6 * cap * slots) return cap;
-  return c->n >= 16 * slots ? 16 : 0;
+  const int64_t per_slot = c->n / ((int64_t)c->n_cus * 16);
+  const bool f32 = precision != PT_FP64;
+  if (per_slot >= 384) return 64;
+  if (per_slot >= (f32 ? 96 : 160)) return 32;
+  if (per_slot >= 40) return 16;
+  return per_slot >= (n_rep > 1 ? 16 : f32 ? 8 : 4) ? 8 : 0;
 }
 
+// Fused walk + interactions (no lists), with a large-stack rerun if the walk
+// stack overflowed for some bucket.
 static pt_status gravity_fused(pt_ctx* c, double theta, const double offset[3],
                                pt_precision precision, pt_counters* counters) {
   pt_status st = check_ctx(c);
@@ -982,14 +989,13 @@ static pt_status gravity_fused(pt_ctx* c, double theta, const double offset[3],
   if (precision != PT_FP64 && (st = check_fp32c_range(c))) return st;
   const int64_t nb = c->nb;
   const bool hexa = c->cfg.hexadecapole != 0;
-  const int cap = group_cap(c);
+  // (2N+1)^3 period replicas
+  const int nr = c->cfg.periodic ? c->cfg.n_replicas : 0;
+  const int64_t n_rep = (int64_t)(2 * nr + 1) * (2 * nr + 1) * (2 * nr + 1);
+  const int cap = group_cap(c, precision, n_rep);
   const bool grouped = cap > 0;
-  const int64_t nblk = std::max<int64_t>(
-      grouped ? pt_grouped_gravity_blocks(nb, c->n, cap)
-              : pt_gravity_blocks(nb, (int)precision, hexa),
-      1);
+  const int64_t nblk = pt_gravity_blocks(nb, c->n, cap);
   PT_TRY_HIP(c, ensure(c->cpart, nblk * 4));
-  PT_TRY_HIP(c, ensure(c->wqueue, 8));
   if (grouped) {
     // the bucket groups of this tree (every replica walks with them)
     const int64_t nw = pt_fgroup_windows(nb);
@@ -1010,8 +1016,6 @@ static pt_status gravity_fused(pt_ctx* c, double theta, const double offset[3],
   // ExMain::traversalFn (examples/Gravity.C:35-46), each added to `offset`;
   // every replica's traversal adds to the accelerations and the counters.  One
   // launch walks for as many replicas as fit beside a node id in 30 bits.
-  const int nr = c->cfg.periodic ? c->cfg.n_replicas : 0;
-  const int64_t n_rep = (int64_t)(2 * nr + 1) * (2 * nr + 1) * (2 * nr + 1);
   const bool shifted =
       n_rep > 1 || c->offset[0] != 0.0 || c->offset[1] != 0.0 || c->offset[2] != 0.0;
   int bits = 4;
@@ -1043,19 +1047,13 @@ static pt_status gravity_fused(pt_ctx* c, double theta, const double offset[3],
       const HexNode* hn = hexa ? c->hn.p : nullptr;
       {
         Timer t(c, PT_T_FORCE);
-        if (grouped)
-          PT_TRY_LAUNCH(c, pt_launch_grouped_gravity(
-                               (int)precision, attempt == 1, c->bk.p, c->fg_first.p, c->fg_nb.p,
-                               c->fg_ng.p, nb, c->n, cap, c->tnode.p, c->gn.p, c->gn32.p, ho, hn,
-                               c->xs.p, c->ys.p, c->zs.p, c->ms.p, c->es.p, gf, c->gm, rep,
-                               c->axs.p, c->ays.p, c->azs.p, c->pots.p, c->cpart.p, c->derr.p,
-                               acc, c->stream));
-        else
-          PT_TRY_LAUNCH(c, pt_launch_gravity((int)precision, attempt == 1, c->bk.p, nb,
-                                             c->tnode.p, c->gn.p, c->gn32.p, ho, hn, c->xs.p,
-                                             c->ys.p, c->zs.p, c->ms.p, c->es.p, gf, c->gm, rep,
-                                             c->axs.p, c->ays.p, c->azs.p, c->pots.p, c->cpart.p,
-                                             c->derr.p, c->wqueue.p, acc, c->stream));
+        PT_TRY_LAUNCH(c, pt_launch_gravity(
+                             (int)precision, attempt == 1, c->bk.p,
+                             grouped ? c->fg_first.p : nullptr, grouped ? c->fg_nb.p : nullptr,
+                             c->fg_ng.p, nb, c->n, cap, c->tnode.p, c->gn.p, c->gn32.p, ho, hn,
+                             c->xs.p, c->ys.p, c->zs.p, c->ms.p, c->es.p, gf, c->gm, rep, c->axs.p,
+                             c->ays.p, c->azs.p, c->pots.p, c->cpart.p, c->derr.p, acc,
+                             c->stream));
       }
       if (r0 + per_launch < n_rep)
         PT_TRY_LAUNCH(c, pt_launch_reduce_counters(c->cpart.p, nblk, c->counters.p, c->derr.p,

@@ -51,16 +51,11 @@ namespace {
 constexpr int kWaves = 4;
 constexpr int kThreads = kWaves * PT_WAVE;
 constexpr int kGroupMax = PT_WAVE;  // targets per pass (one per lane at most)
-// Walk stack entries per wave.  The deepest walks measured on the workloads
-// here (a CPU replay of this walk order over 4000 sampled buckets: Plummer
-// 1M, theta 0.7: 57 entries; 64-halo mixture 4M, theta 0.5, bucket 32: 114)
-// fit the small stack with room to spare; a bucket that overflows it makes
-// the whole evaluation rerun with the big one.  The small stack keeps the
-// FP32 work-group at 6 per CU in LDS (26.5 KiB each).
-constexpr int kSmallStack = 192;
+// Walk stack entries after an overflow of the kernel's usual stack (the
+// deepest walks measured, a CPU replay of this walk order over 4000 sampled
+// buckets: Plummer 1M, theta 0.7: 57 entries; 64-halo mixture 4M, theta 0.5,
+// bucket 32: 114).
 constexpr int kBigStack = 1536;
-// Several replicas walked at once start with up to 64 roots on the stack.
-constexpr int kRepStack = 384;
 
 // ---------------------------------------------------------------------------
 // arithmetic
@@ -149,6 +144,7 @@ struct SrcP32 {  // source particle, FP32, bucket frame
 // reads beyond them hold null sources (zero mass and moments, far away), so
 // the evaluation loops need no bounds tests.  With S = 64 / nt the walk reads
 // S * ceil(n / S) <= 84 slots for n <= 64 (nt = 3, n = 64).
+// FP64 takes its chunks in multiples of S (Group::cw), at most 64 slots.
 constexpr int kSlots = 84;
 constexpr double kNullPos = 1.0e6;
 
@@ -171,7 +167,7 @@ using EntriesIf = typename std::conditional<REP, LeafEntries, NoEntries>::type;
 
 template <bool F32, int STACK, bool REP = false>
 struct __align__(16) WaveLds : EntriesIf<REP> {
-  static constexpr int kStage = kSlots * (F32 ? sizeof(SrcC32) : sizeof(SrcC64));
+  static constexpr int kStage = F32 ? kSlots * sizeof(SrcC32) : PT_WAVE * sizeof(SrcC64);
   static_assert(64 * 4 * sizeof(double) <= kStage, "reduction area");
   unsigned char stage[kStage];
   int32_t stack[STACK];
@@ -923,8 +919,9 @@ interact_kernel(const Bucket* __restrict__ bk, int64_t nb, const TreeNode* __res
     const Group g = make_group(b, g0);
     Lanes<F32> L;
     load_targets<F32>(L, g, px, py, pz, pe, ccx, ccy, ccz);
-    for (int64_t e0 = pc0; e0 < pc1; e0 += PT_WAVE) {
-      const int nsrc = (pc1 - e0) < PT_WAVE ? (int)(pc1 - e0) : PT_WAVE;
+    const int cw = F32 ? PT_WAVE : g.cw;
+    for (int64_t e0 = pc0; e0 < pc1; e0 += cw) {
+      const int nsrc = (pc1 - e0) < cw ? (int)(pc1 - e0) : cw;
       const int32_t id = lane < nsrc ? pc[e0 + lane] : 0;
       do_nodes<F32, W_t>(W, id, nsrc, g, L, gn, gn32, b, bf, sh, ccx, ccy, ccz);
     }
@@ -962,14 +959,10 @@ struct SrcH32 {
   float h[PT_HEXA_MOMS];
 };
 
-// Closed nodes are staged kHexaStage at a time (half a chunk), which keeps a
-// wave's LDS near 9 KiB, and the fused kernel is held to kHexaWaves waves per
-// SIMD (168 VGPRs, a small spill): 1M Plummer, theta 0.7, 13.8 ms against
-// 17.7 ms with a 64-entry stage at two waves per SIMD (four waves spill 264
-// bytes per lane and take 21.5 ms).
+// Closed nodes are staged kHexaStage at a time (half a chunk) in FP64, which
+// keeps a wave's LDS near 9 KiB (1M Plummer, theta 0.7: 13.8 ms against 17.7 ms
+// with a 64-entry stage).
 constexpr int kHexaStage = 32;
-constexpr int kHexaWaves = 3;
-constexpr int kHexaWaves32 = 4;  // the compensated-FP32 form (LDS allows four)
 
 struct __align__(16) HexaLds {
   static constexpr int kStage = kHexaStage * sizeof(SrcH);
@@ -1793,99 +1786,30 @@ __device__ __forceinline__ bool gravity_group(
   return true;
 }
 
-// Fused walk + interactions, one wave per target bucket.  FP32C: one
-// work-group per 4 buckets, mapped XCD-aware (pt_xcd_block).  FP64: a
-// resident grid (a multiple of 8 work-groups, dispatched round-robin over the
-// 8 XCDs) where XCD x owns the contiguous eighth [b_lo, b_hi) of the buckets
-// and its waves take the next one from the XCD's counter (queue[x], zero at
-// launch); every wave leaves once the counter has passed the range.  (The
-// loop form needs more registers, which the FP32C kernel pays for with
-// fewer resident waves; the FP64 kernel gains from the dynamic balance.)
-// The FP32C kernel is compiled for six waves per SIMD (80 VGPRs, a 40-byte
-// spill): 3.79 ms against 3.95 ms at five on the 1M Plummer.
-// HEXADECAPOLE: one work-group per 4 buckets in both forms.
-template <bool F32, int STACK, bool HEXA>
-constexpr int bucket_waves_per_eu() {
-  if (STACK != kSmallStack) return 1;
-  return HEXA ? (F32 ? kHexaWaves32 : kHexaWaves) : (F32 ? 6 : 1);
-}
-
-template <bool F32, int STACK, bool HEXA, typename Sh>
-__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(bucket_waves_per_eu<F32, STACK, HEXA>(), 8)))
-gravity_kernel(const Bucket* __restrict__ bk, int64_t nb, const TreeNode* __restrict__ nodes,
-               const GravNode* __restrict__ gn, const GravNode32* __restrict__ gn32,
-               const HexOpen* __restrict__ ho, const HexNode* __restrict__ hn,
-               const double* __restrict__ px,
-               const double* __restrict__ py, const double* __restrict__ pz,
-               const double* __restrict__ pm, const double* __restrict__ pe, double gf, double gm,
-               Sh sh, double* __restrict__ ax,
-               double* __restrict__ ay, double* __restrict__ az, double* __restrict__ pot,
-               unsigned long long* __restrict__ partials, int32_t* __restrict__ err,
-               unsigned long long* __restrict__ queue, int acc) {
-  using W_t = typename FusedLdsOf<F32, STACK, HEXA, Sh>::type;
-  __shared__ W_t lds[kWaves];
-  __shared__ unsigned long long s_cnt[kWaves][4];
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PT_WAVE);
-  const int lane = threadIdx.x & (PT_WAVE - 1);
-  W_t& W = lds[wave];
-  unsigned long long c_node = 0, c_part = 0, c_open = 0, c_close = 0;
-  bool overflow = false;
-  if constexpr (F32 || HEXA) {
-    const int64_t bi = pt_xcd_block(blockIdx.x, gridDim.x) * kWaves + wave;
-    if (bi < nb)
-      gravity_bucket<F32, STACK, HEXA>(W, bi, bk, nodes, gn, gn32, ho, hn, gm, px, py, pz, pm, pe,
-                                       gf, sh, ax, ay, az, pot, c_node, c_part, c_open, c_close,
-                                       overflow, acc != 0);
-  } else {
-    const int xcd = blockIdx.x % 8;
-    const int64_t b_lo = nb * xcd / 8, b_hi = nb * (xcd + 1) / 8;
-    unsigned long long first = 0;
-    if (lane == 0) first = atomicAdd(&queue[xcd], 1ull);
-    for (int64_t bi = b_lo + (int64_t)__shfl(first, 0, PT_WAVE); bi < b_hi;) {
-      // the next index is fetched now and used after this bucket
-      unsigned long long next = 0;
-      if (lane == 0) next = atomicAdd(&queue[xcd], 1ull);
-      gravity_bucket<F32, STACK, HEXA>(W, bi, bk, nodes, gn, gn32, ho, hn, gm, px, py, pz, pm, pe,
-                                       gf, sh, ax, ay, az, pot, c_node, c_part, c_open, c_close,
-                                       overflow, acc != 0);
-      bi = b_lo + (int64_t)__shfl(next, 0, PT_WAVE);
-    }
-  }
-  if (lane == 0) {
-    if (overflow) atomicExch(err, 1);
-    s_cnt[wave][0] = c_node;
-    s_cnt[wave][1] = c_part;
-    s_cnt[wave][2] = c_open;
-    s_cnt[wave][3] = c_close;
-  }
-  __syncthreads();
-  if (threadIdx.x < 4) {
-    unsigned long long v = 0;
-    for (int w = 0; w < kWaves; w++) v += s_cnt[w][threadIdx.x];
-    partials[(int64_t)blockIdx.x * 4 + threadIdx.x] = v;
-  }
-}
-
-// The grouped form of gravity_kernel: one wave per bucket group (gfirst /
-// gnb, *ngroups of them), gravity_group for a group of two or more buckets,
-// gravity_bucket for a group of one.  Work-group i runs on XCD i % 8, which
-// takes the contiguous eighth [ng x / 8, ng (x + 1) / 8) of the groups in
-// order (neighbouring groups share most sources in its L2); the grid is sized
-// for an upper bound of the group count and the surplus waves find no group.
-// Waves per work-group of the grouped kernel, and its walk stack (pending
-// entries and, from the top, the residual list) per precision.  FP32C: 512
-// entries (7.9 KiB of LDS per one-wave work-group, five per SIMD would fit);
-// the kernel's ~105 VGPRs keep four waves per SIMD without spilling, which
-// measured 3.5% faster than a five-wave register budget (95 VGPRs and a
-// spill).  FP64: 384.
-constexpr int kGWaves = 1;
+// The fused kernel: one wave per bucket group (gfirst / gnb, *ngroups of
+// them), gravity_group for a group of two or more buckets, gravity_bucket for
+// a group of one; without gfirst one wave per bucket (nb of them).
+// Work-group i runs on XCD i % 8, which takes the contiguous eighth
+// [ng x / 8, ng (x + 1) / 8) of the groups in order (neighbouring groups share
+// most sources in its L2); the grid is sized for an upper bound of the group
+// count and the surplus waves find no group.
+// One wave per work-group, so a wave's slot is free as soon as it ends: four
+// waves per work-group, taking buckets from a queue, took 356 against 216 us
+// for one walk per bucket of 20k particles in FP64.  The walk stack (pending
+// entries and, from the top, the residual list) is sized per precision so that
+// the registers and not the LDS bound the waves per SIMD.  FP32C: 512 entries
+// (7.9 KiB of LDS, five waves per SIMD would fit); the kernel's ~105 VGPRs keep
+// four waves per SIMD without spilling, which measured 3.5% faster than a
+// five-wave register budget (95 VGPRs and a spill).  FP64: 384 (9.3 KiB, four
+// waves at 124 VGPRs).
 constexpr int kGroupStack32 = 512;
 constexpr int kGroupStack64 = 384;
 constexpr int kGroupStackHexa = 384;  // the HEXADECAPOLE build, both forms
 
 template <bool F32, int STACK, bool HEXA, typename Sh>
-__global__ void __launch_bounds__(kGWaves * PT_WAVE)
-grouped_gravity_kernel(const Bucket* __restrict__ bk, const int32_t* __restrict__ gfirst,
+__global__ void __launch_bounds__(PT_WAVE)
+grouped_gravity_kernel(const Bucket* __restrict__ bk, int64_t nb,
+                       const int32_t* __restrict__ gfirst,
                        const int32_t* __restrict__ gnb, const uint32_t* __restrict__ ngroups,
                        const TreeNode* __restrict__ nodes, const GravNode* __restrict__ gn,
                        const GravNode32* __restrict__ gn32, const HexOpen* __restrict__ ho,
@@ -1897,20 +1821,17 @@ grouped_gravity_kernel(const Bucket* __restrict__ bk, const int32_t* __restrict_
                        unsigned long long* __restrict__ partials, int32_t* __restrict__ err,
                        int acc) {
   using W_t = typename FusedLdsOf<F32, STACK, HEXA, Sh>::type;
-  __shared__ W_t lds[kGWaves];
-  __shared__ unsigned long long s_cnt[kGWaves][4];
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PT_WAVE);
-  const int lane = threadIdx.x & (PT_WAVE - 1);
-  W_t& W = lds[wave];
+  __shared__ W_t W;
+  const int lane = threadIdx.x;
   unsigned long long c_node = 0, c_part = 0, c_open = 0, c_close = 0;
   bool overflow = false;
-  const int64_t ng = (int64_t)ngroups[0];
+  const int64_t ng = gfirst ? (int64_t)ngroups[0] : nb;
   const int xcd = blockIdx.x % 8;
   const int64_t g_lo = ng * xcd / 8, g_hi = ng * (xcd + 1) / 8;
-  const int64_t gi = g_lo + (int64_t)(blockIdx.x / 8) * kGWaves + wave;
+  const int64_t gi = g_lo + (int64_t)(blockIdx.x / 8);
   if (gi < g_hi) {
-    const int G = gnb[gi];
-    const int64_t b0 = gfirst[gi];
+    const int G = gfirst ? gnb[gi] : 1;
+    const int64_t b0 = gfirst ? gfirst[gi] : gi;
     // a group of one bucket, or a group whose residual list overflowed: one
     // walk per bucket
     const bool done =
@@ -1927,16 +1848,11 @@ grouped_gravity_kernel(const Bucket* __restrict__ bk, const int32_t* __restrict_
   }
   if (lane == 0) {
     if (overflow) atomicExch(err, 1);
-    s_cnt[wave][0] = c_node;
-    s_cnt[wave][1] = c_part;
-    s_cnt[wave][2] = c_open;
-    s_cnt[wave][3] = c_close;
-  }
-  __syncthreads();
-  if (threadIdx.x < 4) {
-    unsigned long long v = 0;
-    for (int w = 0; w < kGWaves; w++) v += s_cnt[w][threadIdx.x];
-    partials[(int64_t)blockIdx.x * 4 + threadIdx.x] = v;
+    unsigned long long* out = partials + (int64_t)blockIdx.x * 4;
+    out[0] = c_node;
+    out[1] = c_part;
+    out[2] = c_open;
+    out[3] = c_close;
   }
 }
 
@@ -2000,25 +1916,6 @@ inline unsigned grid_for(int64_t nb) { return (unsigned)((nb + kWaves - 1) / kWa
 
 }  // namespace
 
-// Work-groups of the fused kernel: FP32C one per 4 buckets; FP64 the
-// resident grid, 8 per CU (at least what fits on a CU; work-groups that do
-// not fit start as others finish -- none waits on another), a multiple of 8
-// (one share per XCD), capped by the bucket count.
-int64_t pt_gravity_blocks(int64_t nb, int precision, bool hexa) {
-  const int64_t need = (nb + kWaves - 1) / kWaves;
-  if (precision != 0 || hexa) return need;
-  static int64_t cap = 0;
-  if (cap == 0) {
-    int dev = 0, cus = 0;
-    (void)hipGetDevice(&dev);
-    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    cap = (int64_t)(cus > 0 ? cus : 8) * 8;
-  }
-  int64_t g = need < cap ? need : cap;
-  g = ((g + 7) / 8) * 8;
-  return g < 8 ? 8 : g;
-}
-
 int pt_launch_interact(int precision, const Bucket* bk, int64_t nb, const TreeNode* nodes,
                        const GravNode* gn, const GravNode32* gn32, const double* x, const double* y, const double* z,
                        const double* m, const double* e, const int64_t* pp_off, const int32_t* pp,
@@ -2050,49 +1947,6 @@ int pt_launch_interact_hexa(const Bucket* bk, int64_t nb, const TreeNode* nodes,
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-// big_stack selects the kBigStack-entry walk stack (used after a walk with
-// the small stack reported an overflow; 1536 entries keep the FP64
-// work-group under 64 KiB of LDS).
-int pt_launch_gravity(int precision, bool big_stack, const Bucket* bk, int64_t nb,
-                      const TreeNode* nodes, const GravNode* gn, const GravNode32* gn32,
-                      const HexOpen* ho, const HexNode* hn, const double* x, const double* y,
-                      const double* z, const double* m, const double* e, double gf, double gm,
-                      const PtReplicas* rep, double* ax, double* ay, double* az, double* pot,
-                      unsigned long long* partials, int32_t* err, unsigned long long* queue,
-                      bool accumulate, hipStream_t s) {
-  if (nb <= 0) return 0;
-  const bool hexa = ho != nullptr;
-  if (pt_launch_fill_u64(queue, 8, 0ull, s) != 0) return -1;
-  const unsigned grid = (unsigned)pt_gravity_blocks(nb, precision, hexa);
-#define PT_GRAVITY_LAUNCH(F32, STACK, HEXA, SH)                                              \
-  gravity_kernel<F32, STACK, HEXA><<<grid, kThreads, 0, s>>>(                                \
-      bk, nb, nodes, gn, gn32, ho, hn, x, y, z, m, e, gf, gm, SH, ax, ay, az, pot, partials, \
-      err, queue, accumulate ? 1 : 0)
-#define PT_GRAVITY_LAUNCH_REP(F32, HEXA)                                                     \
-  if (rep) {                                                                                 \
-    const RepShift sh{rep->tab, rep->bits, rep->n};                                          \
-    if (big_stack) PT_GRAVITY_LAUNCH(F32, kBigStack, HEXA, sh);                              \
-    else PT_GRAVITY_LAUNCH(F32, kRepStack, HEXA, sh);                                        \
-  } else {                                                                                   \
-    if (big_stack) PT_GRAVITY_LAUNCH(F32, kBigStack, HEXA, NoShift{});                       \
-    else PT_GRAVITY_LAUNCH(F32, kSmallStack, HEXA, NoShift{});                               \
-  }
-  if (hexa) {
-    if (precision == 0) {
-      PT_GRAVITY_LAUNCH_REP(false, true)
-    } else {
-      PT_GRAVITY_LAUNCH_REP(true, true)
-    }
-  } else if (precision == 0) {
-    PT_GRAVITY_LAUNCH_REP(false, false)
-  } else {
-    PT_GRAVITY_LAUNCH_REP(true, false)
-  }
-#undef PT_GRAVITY_LAUNCH_REP
-#undef PT_GRAVITY_LAUNCH
-  return hipGetLastError() == hipSuccess ? 0 : -1;
-}
-
 int64_t pt_fgroup_windows(int64_t nb) { return (nb + kFgWindow - 1) / kFgWindow; }
 
 // Two consecutive groups of a window hold more than cap particles together,
@@ -2101,9 +1955,9 @@ int64_t pt_fgroup_max_groups(int64_t nb, int64_t n, int cap) {
   return pt_fgroup_windows(nb) + 2 * n / (cap + 1) + 1;
 }
 
-int64_t pt_grouped_gravity_blocks(int64_t nb, int64_t n, int cap) {
-  const int64_t per_xcd = (pt_fgroup_max_groups(nb, n, cap) + 7) / 8 + 1;
-  return 8 * ((per_xcd + kGWaves - 1) / kGWaves);
+int64_t pt_gravity_blocks(int64_t nb, int64_t n, int cap) {
+  const int64_t groups = cap > 0 ? pt_fgroup_max_groups(nb, n, cap) : nb;
+  return 8 * ((groups + 7) / 8 + 1);
 }
 
 int pt_launch_fgroups(const Bucket* bk, int64_t nb, int cap, int32_t* tfirst, int32_t* tnb,
@@ -2121,21 +1975,22 @@ int pt_launch_fgroups(const Bucket* bk, int64_t nb, int cap, int32_t* tfirst, in
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-int pt_launch_grouped_gravity(int precision, bool big_stack, const Bucket* bk,
-                              const int32_t* gfirst, const int32_t* gnb, const uint32_t* ngroups,
-                              int64_t nb, int64_t n, int cap, const TreeNode* nodes,
-                              const GravNode* gn, const GravNode32* gn32, const HexOpen* ho,
-                              const HexNode* hn, const double* x, const double* y,
-                              const double* z, const double* m, const double* e, double gf,
-                              double gm, const PtReplicas* rep, double* ax, double* ay, double* az,
-                              double* pot, unsigned long long* partials, int32_t* err,
-                              bool accumulate, hipStream_t s) {
+// big_stack selects the kBigStack-entry walk stack (used after a walk with
+// the small stack reported an overflow).
+int pt_launch_gravity(int precision, bool big_stack, const Bucket* bk, const int32_t* gfirst,
+                      const int32_t* gnb, const uint32_t* ngroups, int64_t nb, int64_t n, int cap,
+                      const TreeNode* nodes, const GravNode* gn, const GravNode32* gn32,
+                      const HexOpen* ho, const HexNode* hn, const double* x, const double* y,
+                      const double* z, const double* m, const double* e, double gf, double gm,
+                      const PtReplicas* rep, double* ax, double* ay, double* az, double* pot,
+                      unsigned long long* partials, int32_t* err, bool accumulate,
+                      hipStream_t s) {
   if (nb <= 0) return 0;
-  const unsigned grid = (unsigned)pt_grouped_gravity_blocks(nb, n, cap);
+  const unsigned grid = (unsigned)pt_gravity_blocks(nb, n, cap);
   const bool hexa = ho != nullptr;
 #define PT_GROUPED_LAUNCH(F32, STACK, HEXA, SH)                                                \
-  grouped_gravity_kernel<F32, STACK, HEXA><<<grid, kGWaves * PT_WAVE, 0, s>>>(                 \
-      bk, gfirst, gnb, ngroups, nodes, gn, gn32, ho, hn, x, y, z, m, e, gf, gm, SH, ax, ay, az, \
+  grouped_gravity_kernel<F32, STACK, HEXA><<<grid, PT_WAVE, 0, s>>>(                           \
+      bk, nb, gfirst, gnb, ngroups, nodes, gn, gn32, ho, hn, x, y, z, m, e, gf, gm, SH, ax, ay, az, \
       pot, partials, err, accumulate ? 1 : 0)
 #define PT_GROUPED_LAUNCH_REP(F32, STACK, HEXA)                    \
   if (rep) {                                                       \

@@ -138,18 +138,6 @@ struct PtReplicas {
 };
 int pt_launch_replica_table(int nr, const double off[3], const double period[3], double* tab,
                             hipStream_t s);
-// One walk per bucket: precision 0 FP64, otherwise the compensated-FP32 form;
-// ho != nullptr: the HEXADECAPOLE build; rep == nullptr: no offset.
-// Counters as partials of pt_gravity_blocks work-groups.
-int64_t pt_gravity_blocks(int64_t nb, int precision, bool hexa);
-int pt_launch_gravity(int precision, bool big_stack, const Bucket* bk, int64_t nb,
-                      const TreeNode* nodes, const GravNode* gn, const GravNode32* gn32,
-                      const HexOpen* ho, const HexNode* hn, const double* x, const double* y,
-                      const double* z, const double* m, const double* e, double gf, double gm,
-                      const PtReplicas* rep, double* ax, double* ay, double* az, double* pot,
-                      unsigned long long* partials, int32_t* err, unsigned long long* queue,
-                      bool accumulate, hipStream_t s);
-
 // Bucket groups of the grouped fused kernel: runs of consecutive buckets of
 // at most cap (2..64) particles in all (a larger bucket alone), formed inside
 // windows of 64 buckets and compacted in order into gfirst / gnb, their
@@ -161,21 +149,20 @@ int64_t pt_fgroup_max_groups(int64_t nb, int64_t n, int cap);
 int pt_launch_fgroups(const Bucket* bk, int64_t nb, int cap, int32_t* tfirst, int32_t* tnb,
                       uint32_t* wcount, uint32_t* woff, void* scratch, uint32_t* ngroups,
                       int32_t* gfirst, int32_t* gnb, hipStream_t s);
-// The fused walk + interactions with the shared walk per bucket group; the
-// same calls, counters and partials layout as pt_launch_gravity (partials:
-// pt_grouped_gravity_blocks(nb, n, cap) work-groups).  ho / hn non-null: the
-// HEXADECAPOLE build (open() with gm, node() from hn), else the quadrupole
-// build (gn / gn32).
-int64_t pt_grouped_gravity_blocks(int64_t nb, int64_t n, int cap);
-int pt_launch_grouped_gravity(int precision, bool big_stack, const Bucket* bk,
-                              const int32_t* gfirst, const int32_t* gnb, const uint32_t* ngroups,
-                              int64_t nb, int64_t n, int cap, const TreeNode* nodes,
-                              const GravNode* gn, const GravNode32* gn32, const HexOpen* ho,
-                              const HexNode* hn, const double* x, const double* y,
-                              const double* z, const double* m, const double* e, double gf,
-                              double gm, const PtReplicas* rep, double* ax, double* ay, double* az,
-                              double* pot, unsigned long long* partials, int32_t* err,
-                              bool accumulate, hipStream_t s);
+// The fused walk + interactions: a shared walk per bucket group, or with
+// gfirst null (cap 0) one walk per bucket; counters as partials of
+// pt_gravity_blocks(nb, n, cap) work-groups.  precision 0 FP64, otherwise the
+// compensated-FP32 form; ho / hn non-null: the HEXADECAPOLE build (open() with
+// gm, node() from hn), else the quadrupole build (gn / gn32); rep null: no
+// offset.
+int64_t pt_gravity_blocks(int64_t nb, int64_t n, int cap);
+int pt_launch_gravity(int precision, bool big_stack, const Bucket* bk, const int32_t* gfirst,
+                      const int32_t* gnb, const uint32_t* ngroups, int64_t nb, int64_t n, int cap,
+                      const TreeNode* nodes, const GravNode* gn, const GravNode32* gn32,
+                      const HexOpen* ho, const HexNode* hn, const double* x, const double* y,
+                      const double* z, const double* m, const double* e, double gf, double gm,
+                      const PtReplicas* rep, double* ax, double* ay, double* az, double* pot,
+                      unsigned long long* partials, int32_t* err, bool accumulate, hipStream_t s);
 
 // Ewald lattice correction of the periodic build (quadrupole form) from the
 // root's moments (node 0 of nd), added to the sorted results.  table holds
