@@ -39,8 +39,6 @@
 
 namespace {
 
-constexpr int kAdjWaves = 4;
-constexpr int kAdjThreads = kAdjWaves * PT_WAVE;
 constexpr int kANT = PT_GROUP_TARGETS;  // targets per pass over a group's lists
 constexpr int kNodeAdj = 11;  // node cotangent: cm(3), M, Q(6: xx xy xz yy yz zz), soft
 // Nodes of the top levels (ids < kHotNodes in level order) are in the lists
@@ -177,19 +175,60 @@ __device__ __forceinline__ bool leaf_far_pass(const double* __restrict__ f, doub
   return dsq > 1.0001 * reach * reach;
 }
 
+// The target gradients of a pass, in LDS: kAccCols partial sums per target and
+// component, one per lane of each half wave; lane l adds to column l % 32 of
+// row 3 t + component.  The odd stride spreads the rows over the banks for the
+// final sums.  In registers (96 per lane, and the loop over the targets
+// unrolled for their sake) they left one wave per SIMD, whose dependent FP64
+// chains kept 45% of the issue slots.
+constexpr int kAccCols = 32;
+constexpr int kAccStride = kAccCols + 1;
+
+__device__ __forceinline__ void lds_add(double* p, double v) {
+  __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// acc: the calling lane's column of row 0.
+__device__ __forceinline__ void tgt_add(double* __restrict__ acc, int t, double x, double y,
+                                        double z) {
+  double* a = acc + t * (3 * kAccStride);
+  lds_add(a, x);
+  lds_add(a + kAccStride, y);
+  lds_add(a + 2 * kAccStride, z);
+}
+
+// The column sums of the pass's ng targets (first + g0 = i0), into global
+// memory.
+__device__ __forceinline__ void tgt_flush(const double* __restrict__ s_acc, int ng, int64_t i0,
+                                          double* __restrict__ gx, double* __restrict__ gy,
+                                          double* __restrict__ gz) {
+  const int row = threadIdx.x;
+  if (row < 3 * ng) {
+    const double* a = s_acc + row * kAccStride;
+    double v = 0.0;
+    for (int k = 0; k < kAccCols; k++) v += a[k];
+    const int c = row % 3;
+    atomicAdd((c == 0 ? gx : (c == 1 ? gy : gz)) + i0 + row / 3, v);
+  }
+}
+
 // One node() list entry against the pass's targets (FP64): the target
-// gradients into tg, the node cotangent into lam; mono: the members for which
-// openSoftening sends the node to addGravity.
+// gradients into acc, the node cotangent into lam; mono: the members for which
+// openSoftening sends the node to addGravity.  FAR (wave-uniform): every pair
+// is a node() pair beyond its softening, b = 1/r^3, c = 3/r^5, d = 15/r^7 with
+// derivatives -c r, -d r, -7 d / r and none in the softening.
+template <bool FAR>
 __device__ __forceinline__ void node_entry_pairs(const GravNode& s, unsigned mask, unsigned mono,
                                                  const TgtA* __restrict__ st, int ng, double ox,
-                                                 double oy, double oz, double (&tg)[kANT][3],
+                                                 double oy, double oz, double* __restrict__ acc,
                                                  double (&lam)[kNodeAdj]) {
   const double cx = s.cx + ox, cy = s.cy + oy, cz = s.cz + oz;
-#pragma unroll
-  for (int t = 0; t < kANT; t++) {
-    if (t < ng && ((mask >> st[t].bt) & 1u)) {
-      const TgtA tt = st[t];
-      if ((mono >> tt.bt) & 1u) {
+  double trace = 0.0;  // the part common to d(a.w)/dQ's diagonal
+#pragma unroll 1
+  for (int t = 0; t < ng; t++) {
+    const TgtA tt = st[t];
+    if ((mask >> tt.bt) & 1u) {
+      if (!FAR && ((mono >> tt.bt) & 1u)) {
         const double dx = cx - tt.x, dy = cy - tt.y, dz = cz - tt.z;
         const double r2 = dx * dx + dy * dy + dz * dz;
         if (r2 != 0) {
@@ -200,9 +239,7 @@ __device__ __forceinline__ void node_entry_pairs(const GravNode& s, unsigned mas
           const double Tx = s.mass * ir3 * tt.wx + f * dx;
           const double Ty = s.mass * ir3 * tt.wy + f * dy;
           const double Tz = s.mass * ir3 * tt.wz + f * dz;
-          tg[t][0] -= Tx;
-          tg[t][1] -= Ty;
-          tg[t][2] -= Tz;
+          tgt_add(acc, t, -Tx, -Ty, -Tz);
           lam[0] += Tx;
           lam[1] += Ty;
           lam[2] += Tz;
@@ -212,119 +249,103 @@ __device__ __forceinline__ void node_entry_pairs(const GravNode& s, unsigned mas
         const double rx = (tt.x - s.cx) - ox, ry = (tt.y - s.cy) - oy, rz = (tt.z - s.cz) - oz;
         const double r2 = fma(rx, rx, fma(ry, ry, rz * rz));
         const double ir = pt_rsqrt64(r2);
-        const double r = r2 * ir;
-        const SplineQ q = splineq_grad(r, ir, r2, s.soft + tt.e);
         const double qx = fma(s.qxx, rx, fma(s.qxy, ry, s.qxz * rz));
         const double qy = fma(s.qxy, rx, fma(s.qyy, ry, s.qyz * rz));
         const double qz = fma(s.qxz, rx, fma(s.qyz, ry, s.qzz * rz));
         const double qir = 0.5 * fma(qx, rx, fma(qy, ry, qz * rz));
-        const double qir3 = fma(q.b, s.mass, fma(q.d, qir, -q.c * s.tr));
         const double rw = fma(rx, tt.wx, fma(ry, tt.wy, rz * tt.wz));
         const double qw = fma(qx, tt.wx, fma(qy, tt.wy, qz * tt.wz));
-        const double Qwx = fma(s.qxx, tt.wx, fma(s.qxy, tt.wy, s.qxz * tt.wz));
-        const double Qwy = fma(s.qxy, tt.wx, fma(s.qyy, tt.wy, s.qyz * tt.wz));
-        const double Qwz = fma(s.qxz, tt.wx, fma(s.qyz, tt.wy, s.qzz * tt.wz));
-        const double k1 = fma(s.mass, q.br, fma(qir, q.dr_, -s.tr * q.cr)) * ir;
-        const double k2 = q.cr * ir;
-        // J = -qir3 w + (k2 (q.w) - k1 (r.w)) r - d (r.w) q + c Q w
+        double b, c, d, k1, k2;
+        if (FAR) {
+          const double a2 = ir * ir;
+          b = ir * a2;
+          c = 3.0 * b * a2;
+          d = 5.0 * c * a2;
+          k1 = fma(-c, s.mass, d * fma(-7.0 * a2, qir, s.tr));
+          k2 = -d;
+        } else {
+          const SplineQ q = splineq_grad(r2 * ir, ir, r2, s.soft + tt.e);
+          b = q.b;
+          c = q.c;
+          d = q.d;
+          k1 = fma(s.mass, q.br, fma(qir, q.dr_, -s.tr * q.cr)) * ir;
+          k2 = q.cr * ir;
+          lam[10] += fma(-fma(q.bt, s.mass, fma(q.dt_, qir, -q.ct * s.tr)), rw, q.ct * qw);
+        }
+        const double qir3 = fma(b, s.mass, fma(d, qir, -c * s.tr));
+        // J = -qir3 w + (k2 (q.w) - k1 (r.w)) r - d (r.w) q + c Q w; with
+        // p = c w - d (r.w) r / 2 its last two terms are Q p - d (r.w) q / 2
         const double s1 = fma(k2, qw, -k1 * rw);
-        const double drw = q.d * rw;
-        const double Jx = fma(-qir3, tt.wx, fma(s1, rx, fma(-drw, qx, q.c * Qwx)));
-        const double Jy = fma(-qir3, tt.wy, fma(s1, ry, fma(-drw, qy, q.c * Qwy)));
-        const double Jz = fma(-qir3, tt.wz, fma(s1, rz, fma(-drw, qz, q.c * Qwz)));
-        tg[t][0] += Jx;
-        tg[t][1] += Jy;
-        tg[t][2] += Jz;
+        const double hd = -0.5 * (d * rw);
+        const double px = fma(hd, rx, c * tt.wx), py = fma(hd, ry, c * tt.wy),
+                     pz = fma(hd, rz, c * tt.wz);
+        const double Qpx = fma(s.qxx, px, fma(s.qxy, py, s.qxz * pz));
+        const double Qpy = fma(s.qxy, px, fma(s.qyy, py, s.qyz * pz));
+        const double Qpz = fma(s.qxz, px, fma(s.qyz, py, s.qzz * pz));
+        const double Jx = fma(-qir3, tt.wx, fma(s1, rx, fma(hd, qx, Qpx)));
+        const double Jy = fma(-qir3, tt.wy, fma(s1, ry, fma(hd, qy, Qpy)));
+        const double Jz = fma(-qir3, tt.wz, fma(s1, rz, fma(hd, qz, Qpz)));
+        tgt_add(acc, t, Jx, Jy, Jz);
         lam[0] -= Jx;
         lam[1] -= Jy;
         lam[2] -= Jz;
-        lam[3] = fma(-q.b, rw, lam[3]);
-        // d(a.w)/dQ per stored component: (-d (r.w) / 2) r r^T + (c (r.w) / 2) I
-        // + c sym(w r^T), written as r_k p_l + r_l p_k (+ the trace part) with
-        // p = -d (r.w) r / 2 + c w
-        const double hd = -0.5 * drw, hc = 0.5 * q.c * rw;
-        const double qpx = fma(hd, rx, q.c * tt.wx), qpy = fma(hd, ry, q.c * tt.wy),
-                     qpz = fma(hd, rz, q.c * tt.wz);
-        lam[4] += fma(rx, qpx, hc);
-        lam[5] += fma(ry, qpx, rx * qpy);
-        lam[6] += fma(rz, qpx, rx * qpz);
-        lam[7] += fma(ry, qpy, hc);
-        lam[8] += fma(rz, qpy, ry * qpz);
-        lam[9] += fma(rz, qpz, hc);
-        lam[10] += fma(-fma(q.bt, s.mass, fma(q.dt_, qir, -q.ct * s.tr)), rw, q.ct * qw);
+        lam[3] = fma(-b, rw, lam[3]);
+        // d(a.w)/dQ per stored component: r_k p_l + r_l p_k, on the diagonal
+        // r_k p_k + c (r.w) / 2
+        lam[4] = fma(rx, px, lam[4]);
+        lam[5] = fma(ry, px, fma(rx, py, lam[5]));
+        lam[6] = fma(rz, px, fma(rx, pz, lam[6]));
+        lam[7] = fma(ry, py, lam[7]);
+        lam[8] = fma(rz, py, fma(ry, pz, lam[8]));
+        lam[9] = fma(rz, pz, lam[9]);
+        trace = fma(c, rw, trace);
       }
     }
   }
+  lam[4] = fma(0.5, trace, lam[4]);
+  lam[7] = fma(0.5, trace, lam[7]);
+  lam[9] = fma(0.5, trace, lam[9]);
 }
 
-// One source particle against the pass's targets (FP64), the softened form.
+// One source particle against the pass's targets (FP64).  FAR (wave-uniform):
+// every pair is beyond its softening, so not the target itself.  The source's
+// position gradient is summed before its mass factor.
+template <bool FAR>
 __device__ __forceinline__ void particle_pairs(double jx, double jy, double jz, double jm,
                                                double je, unsigned jmask,
                                                const TgtA* __restrict__ st, int ng,
-                                               double (&tg)[kANT][3], double& sgx, double& sgy,
+                                               double* __restrict__ acc, double& sgx, double& sgy,
                                                double& sgz, double& sgm) {
-#pragma unroll
-  for (int t = 0; t < kANT; t++) {
-    if (t < ng && ((jmask >> st[t].bt) & 1u)) {
-      const TgtA tt = st[t];
+  double kx = 0.0, ky = 0.0, kz = 0.0;
+#pragma unroll 2
+  for (int t = 0; t < ng; t++) {
+    const TgtA tt = st[t];
+    if ((jmask >> tt.bt) & 1u) {
       const double dx = jx - tt.x, dy = jy - tt.y, dz = jz - tt.z;
-      const double r2 = dx * dx + dy * dy + dz * dz;
-      if (r2 != 0) {
+      const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
+      if (FAR || r2 != 0) {
         const double ir = pt_rsqrt64(r2);
-        double bb, db;
-        spline_b_db(r2 * ir, ir, je + tt.e, bb, db);
-        const double dw = dx * tt.wx + dy * tt.wy + dz * tt.wz;
-        const double f = db * ir * dw;
-        const double Kx = jm * (bb * tt.wx + f * dx);
-        const double Ky = jm * (bb * tt.wy + f * dy);
-        const double Kz = jm * (bb * tt.wz + f * dz);
-        tg[t][0] -= Kx;
-        tg[t][1] -= Ky;
-        tg[t][2] -= Kz;
-        sgx += Kx;
-        sgy += Ky;
-        sgz += Kz;
-        sgm += bb * dw;
+        const double dw = fma(dx, tt.wx, fma(dy, tt.wy, dz * tt.wz));
+        double bb, f;  // f = b'(r) (d.w) / r
+        if (FAR) {
+          const double a2 = ir * ir;
+          bb = ir * a2;
+          f = -3.0 * (bb * a2) * dw;
+        } else {
+          double db;
+          spline_b_db(r2 * ir, ir, je + tt.e, bb, db);
+          f = db * ir * dw;
+        }
+        const double Kx = fma(bb, tt.wx, f * dx);
+        const double Ky = fma(bb, tt.wy, f * dy);
+        const double Kz = fma(bb, tt.wz, f * dz);
+        tgt_add(acc, t, -jm * Kx, -jm * Ky, -jm * Kz);
+        kx += Kx;
+        ky += Ky;
+        kz += Kz;
+        sgm = fma(bb, dw, sgm);
       }
     }
-  }
-}
-
-// One source particle of a far window (every pair beyond its softening, so
-// not the target itself) against all kANT targets of the pass (FP64), without
-// branches: a pair whose target bucket is not in the mask, and the padding
-// targets past the pass's count (bucket index 31, the position of a real
-// target, so r > 0), is evaluated with a zero cotangent w, which zeroes each
-// of its contributions (all are linear in w); consecutive targets' pairs then
-// interleave.  The source's position gradient is summed before its mass
-// factor.
-__device__ __forceinline__ void particle_pairs_far(double jx, double jy, double jz, double jm,
-                                                   unsigned jmask, const TgtA* __restrict__ st,
-                                                   double (&tg)[kANT][3], double& sgx,
-                                                   double& sgy, double& sgz, double& sgm) {
-  double kx = 0.0, ky = 0.0, kz = 0.0;
-#pragma unroll
-  for (int t = 0; t < kANT; t++) {
-    const TgtA tt = st[t];
-    const bool act = (jmask >> tt.bt) & 1u;
-    const double wx = act ? tt.wx : 0.0, wy = act ? tt.wy : 0.0, wz = act ? tt.wz : 0.0;
-    const double dx = jx - tt.x, dy = jy - tt.y, dz = jz - tt.z;
-    const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
-    const double ir = pt_rsqrt64(r2);
-    const double a2 = ir * ir;
-    const double bb = ir * a2;
-    const double dw = fma(dx, wx, fma(dy, wy, dz * wz));
-    const double f = -3.0 * (bb * a2) * dw;  // b'(r) (d.w) / r
-    const double Kx = fma(bb, wx, f * dx);
-    const double Ky = fma(bb, wy, f * dy);
-    const double Kz = fma(bb, wz, f * dz);
-    tg[t][0] = fma(-jm, Kx, tg[t][0]);
-    tg[t][1] = fma(-jm, Ky, tg[t][1]);
-    tg[t][2] = fma(-jm, Kz, tg[t][2]);
-    kx += Kx;
-    ky += Ky;
-    kz += Kz;
-    sgm = fma(bb, dw, sgm);
   }
   sgx += jm * kx;
   sgy += jm * ky;
@@ -340,10 +361,12 @@ __device__ __forceinline__ void particle_pairs_far(double jx, double jy, double 
 // is summed over the targets of a pass before one atomic add per field.  Leaf
 // sources: flattened to one source particle per lane (the leaf's mask
 // carried along); the source's gradient is summed over the targets of a pass
-// before its atomic adds.  Target gradients are wave-reduced per pass.
-__global__ void __launch_bounds__(kAdjThreads)
+// before its atomic adds.  Target gradients are summed in LDS (tgt_add).  One
+// wave per work-group, in an order that keeps every XCD supplied
+// (pt_part_item).
+__global__ void __launch_bounds__(PT_WAVE)
 adjoint_group_kernel(const Bucket* __restrict__ bk, const int32_t* __restrict__ gfirst,
-                     const int32_t* __restrict__ gnb, int64_t ns,
+                     const int32_t* __restrict__ gnb, const uint32_t* __restrict__ ngroups,
                      const TreeNode* __restrict__ nodes,
                     const GravNode* __restrict__ gn, const double* __restrict__ px,
                     const double* __restrict__ py, const double* __restrict__ pz,
@@ -356,40 +379,39 @@ adjoint_group_kernel(const Bucket* __restrict__ bk, const int32_t* __restrict__ 
                     double* __restrict__ gx, double* __restrict__ gy, double* __restrict__ gz,
                     double* __restrict__ gmass, double* __restrict__ lam_node, int64_t nn,
                     double* __restrict__ hot, int64_t nhot) {
-  __shared__ TgtA s_t[kAdjWaves][kANT];
-  __shared__ Bucket s_bk[kAdjWaves][PT_GROUP_BUCKETS];
-  __shared__ int32_t s_beg[kAdjWaves][PT_WAVE];
-  __shared__ double s_far[kAdjWaves][kPassFar];
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PT_WAVE);
-  const int lane = threadIdx.x & (PT_WAVE - 1);
-  const int64_t gi = (int64_t)blockIdx.x * kAdjWaves + wave;
-  if (gi >= ns) return;
+  __shared__ TgtA s_t[kANT];
+  __shared__ Bucket s_bk[PT_GROUP_BUCKETS];
+  __shared__ int32_t s_beg[PT_WAVE];
+  __shared__ double s_far[kPassFar];
+  __shared__ double s_acc[kANT * 3 * kAccStride];
+  const int lane = threadIdx.x;
+  const int64_t gi = pt_part_item((int32_t)ngroups[0]);
+  if (gi < 0) return;
   const int nbk = gnb[gi];
-  if (nbk <= 0) return;
   const int64_t b0 = gfirst[gi];
-  if (lane < nbk) s_bk[wave][lane] = bk[b0 + lane];
+  if (lane < nbk) s_bk[lane] = bk[b0 + lane];
   __builtin_amdgcn_wave_barrier();
   // the group's targets are consecutive: its buckets' ranges in order
-  const int64_t first = s_bk[wave][0].begin;
-  const int nt = (int)((int64_t)s_bk[wave][nbk - 1].begin + s_bk[wave][nbk - 1].count - first);
+  const int64_t first = s_bk[0].begin;
+  const int nt = (int)((int64_t)s_bk[nbk - 1].begin + s_bk[nbk - 1].count - first);
   const int64_t pc0 = pc_off[gi], pc1 = pc_off[gi + 1];
   const int64_t pp0 = pp_off[gi], pp1 = pp_off[gi + 1];
   if (lane < 7) {
     // the group's box and largest bucket softening
     double v = lane < 3 ? INFINITY : (lane < 6 ? -INFINITY : 0.0);
     for (int k = 0; k < nbk; k++) {
-      const Bucket& bb = s_bk[wave][k];
+      const Bucket& bb = s_bk[k];
       const double c[7] = {bb.lox, bb.loy, bb.loz, bb.hix, bb.hiy, bb.hiz, bb.soft};
       v = lane < 3 ? fmin(v, c[lane]) : fmax(v, c[lane]);
     }
-    s_far[wave][lane] = v;
+    s_far[lane] = v;
   }
   for (int g0 = 0; g0 < nt; g0 += kANT) {
     const int ng = (nt - g0) < kANT ? (nt - g0) : kANT;
     // member buckets with a target in this pass
     unsigned pass = 0;
     for (int k = 0; k < nbk; k++) {
-      const int64_t lo = s_bk[wave][k].begin, hi = lo + s_bk[wave][k].count;
+      const int64_t lo = s_bk[k].begin, hi = lo + s_bk[k].count;
       if (hi > first + g0 && lo < first + g0 + ng) pass |= 1u << k;
     }
     __builtin_amdgcn_wave_barrier();
@@ -397,24 +419,18 @@ adjoint_group_kernel(const Bucket* __restrict__ bk, const int32_t* __restrict__ 
       const int64_t i = first + g0 + lane;
       int bt = 0;
       for (int k = 1; k < nbk; k++)
-        if (i >= s_bk[wave][k].begin) bt = k;
-      s_t[wave][lane] = TgtA{px[i], py[i], pz[i], pe[i], wx[i], wy[i], wz[i], bt, 0};
-    } else if (lane < kANT) {
-      // padding for the branch-free far-window form: a real target's
-      // position, no bucket, zero cotangent
-      const int64_t i = first + g0;
-      s_t[wave][lane] = TgtA{px[i], py[i], pz[i], 0.0, 0.0, 0.0, 0.0, 31, 0};
+        if (i >= s_bk[k].begin) bt = k;
+      s_t[lane] = TgtA{px[i], py[i], pz[i], pe[i], wx[i], wy[i], wz[i], bt, 0};
     }
-    __builtin_amdgcn_wave_barrier();
-    double tg[kANT][3];
-#pragma unroll
-    for (int t = 0; t < kANT; t++) tg[t][0] = tg[t][1] = tg[t][2] = 0.0;
+    for (int k = lane; k < 3 * ng * kAccStride; k += PT_WAVE) s_acc[k] = 0.0;
+    __syncthreads();
+    double* const acc = s_acc + lane % kAccCols;
     if (lane == 0) {
       double emax = 0.0;
-      for (int t = 0; t < ng; t++) emax = s_t[wave][t].e > emax ? s_t[wave][t].e : emax;
-      s_far[wave][7] = emax;
+      for (int t = 0; t < ng; t++) emax = s_t[t].e > emax ? s_t[t].e : emax;
+      s_far[7] = emax;
     }
-    __builtin_amdgcn_wave_barrier();
+    __syncthreads();
 
     // ---- node() sources: in chunks in which every entry is far no member's
     // openSoftening can hold, so its tests are skipped
@@ -425,7 +441,7 @@ adjoint_group_kernel(const Bucket* __restrict__ bk, const int32_t* __restrict__ 
       if (mask != 0u) {
         sid = pc[e];
         const GravNode s = gn[sid];
-        const bool far = node_far_pass(s_far[wave], s.cx + ox, s.cy + oy, s.cz + oz, s.soft);
+        const bool far = node_far_pass(s_far, s.cx + ox, s.cy + oy, s.cz + oz, s.soft);
         // over the lanes holding an entry (the others are inactive here)
         const bool all_far = __ballot(!far) == 0ull;
         double lam[kNodeAdj];
@@ -437,11 +453,14 @@ adjoint_group_kernel(const Bucket* __restrict__ bk, const int32_t* __restrict__ 
         if (!all_far) {
           for (unsigned mm = mask; mm != 0u; mm &= mm - 1u) {
             const int k = __builtin_ctz(mm);
-            if (pt_open_softening(s.cx + ox, s.cy + oy, s.cz + oz, s.soft, s_bk[wave][k]))
+            if (pt_open_softening(s.cx + ox, s.cy + oy, s.cz + oz, s.soft, s_bk[k]))
               mono |= 1u << k;
           }
         }
-        node_entry_pairs(s, mask, mono, s_t[wave], ng, ox, oy, oz, tg, lam);
+        if (all_far)
+          node_entry_pairs<true>(s, mask, 0u, s_t, ng, ox, oy, oz, acc, lam);
+        else
+          node_entry_pairs<false>(s, mask, mono, s_t, ng, ox, oy, oz, acc, lam);
         double* dst = sid < nhot
                           ? hot + (int64_t)(blockIdx.x % kHotParts) * kNodeAdj * nhot + sid
                           : lam_node + sid;
@@ -463,7 +482,7 @@ adjoint_group_kernel(const Bucket* __restrict__ bk, const int32_t* __restrict__ 
         const TreeNode nd = nodes[pp[l]];
         cnt = nd.count;
         beg = nd.begin;
-        isnear = !leaf_far_pass(s_far[wave], nd.cx + ox, nd.cy + oy, nd.cz + oz, nd.leaf_reach,
+        isnear = !leaf_far_pass(s_far, nd.cx + ox, nd.cy + oy, nd.cz + oz, nd.leaf_reach,
                                 nd.leaf_soft);
       }
       const int cn = isnear ? cnt : 0, cf = isnear ? 0 : cnt;
@@ -479,7 +498,7 @@ adjoint_group_kernel(const Bucket* __restrict__ bk, const int32_t* __restrict__ 
         // a slot's entry: the lane of the last entry start at or below it in
         // this window (marks by start slot, a ballot of the marks), or the
         // previous window's last entry
-        int32_t* mark = s_beg[wave];
+        int32_t* mark = s_beg;
         mark[lane] = -1;
         __builtin_amdgcn_wave_barrier();
         if (cnt > 0 && exc >= s0 && exc < s0 + PT_WAVE) mark[exc - s0] = lane;
@@ -498,9 +517,9 @@ adjoint_group_kernel(const Bucket* __restrict__ bk, const int32_t* __restrict__ 
           const double jm = pm[j], je = pe[j];
           double sgx = 0.0, sgy = 0.0, sgz = 0.0, sgm = 0.0;
           if (wfar)
-            particle_pairs_far(jx, jy, jz, jm, jmask, s_t[wave], tg, sgx, sgy, sgz, sgm);
+            particle_pairs<true>(jx, jy, jz, jm, je, jmask, s_t, ng, acc, sgx, sgy, sgz, sgm);
           else
-            particle_pairs(jx, jy, jz, jm, je, jmask, s_t[wave], ng, tg, sgx, sgy, sgz, sgm);
+            particle_pairs<false>(jx, jy, jz, jm, je, jmask, s_t, ng, acc, sgx, sgy, sgz, sgm);
           atomicAdd(&gx[j], sgx);
           atomicAdd(&gy[j], sgy);
           atomicAdd(&gz[j], sgz);
@@ -510,20 +529,9 @@ adjoint_group_kernel(const Bucket* __restrict__ bk, const int32_t* __restrict__ 
       __builtin_amdgcn_wave_barrier();
     }
 
-#pragma unroll
-    for (int t = 0; t < kANT; t++) {
-      if (t < ng) {
-        const double rx = pt_wave_sum(tg[t][0]);
-        const double ry = pt_wave_sum(tg[t][1]);
-        const double rz = pt_wave_sum(tg[t][2]);
-        if (lane == t) {
-          const int64_t i = first + g0 + t;
-          atomicAdd(&gx[i], rx);
-          atomicAdd(&gy[i], ry);
-          atomicAdd(&gz[i], rz);
-        }
-      }
-    }
+    __syncthreads();
+    tgt_flush(s_acc, ng, first + g0, gx, gy, gz);
+    __syncthreads();
   }
 }
 
@@ -618,24 +626,110 @@ struct TgtA32 {
   int32_t bt;
 };
 
-// One source particle against the pass's targets (FP32 pairs, target
-// gradients summed in FP64).  far (wave-uniform): every pair is beyond its
-// softening (and so not the target itself).
-__device__ __forceinline__ void particle_pairs32(bool far, float jx, float jy, float jz, float jm,
-                                                 float je, unsigned jmask,
-                                                 const TgtA32* __restrict__ st, int ng,
-                                                 double (&tg)[kANT][3], float& sgx, float& sgy,
-                                                 float& sgz, float& sgm) {
-#pragma unroll
-  for (int t = 0; t < kANT; t++) {
-    if (t < ng && ((jmask >> st[t].bt) & 1u)) {
-      const TgtA32 tt = st[t];
+// node_entry_pairs in FP32; cx, cy, cz: the node's centre in the group's frame.
+template <bool FAR>
+__device__ __forceinline__ void node_entry_pairs32(const GravNode32& s, float cx, float cy,
+                                                   float cz, unsigned mask, unsigned mono,
+                                                   const TgtA32* __restrict__ st, int ng,
+                                                   double* __restrict__ acc,
+                                                   float (&lam)[kNodeAdj]) {
+  const float tr = 0.5f * (s.qxx + s.qyy + s.qzz);
+  float trace = 0.0f;
+#pragma unroll 1
+  for (int t = 0; t < ng; t++) {
+    const TgtA32 tt = st[t];
+    if ((mask >> tt.bt) & 1u) {
+      if (!FAR && ((mono >> tt.bt) & 1u)) {
+        const float dx = cx - tt.x, dy = cy - tt.y, dz = cz - tt.z;
+        const float r2 = dx * dx + dy * dy + dz * dz;
+        if (r2 != 0.0f) {
+          const float ir = __builtin_amdgcn_rsqf(r2);
+          const float ir3 = ir * ir * ir;
+          const float dw = dx * tt.wx + dy * tt.wy + dz * tt.wz;
+          const float f = -3.0f * s.mass * ir3 * ir * ir * dw;
+          const float Tx = s.mass * ir3 * tt.wx + f * dx;
+          const float Ty = s.mass * ir3 * tt.wy + f * dy;
+          const float Tz = s.mass * ir3 * tt.wz + f * dz;
+          tgt_add(acc, t, -(double)Tx, -(double)Ty, -(double)Tz);
+          lam[0] += Tx;
+          lam[1] += Ty;
+          lam[2] += Tz;
+          lam[3] += dw * ir3;
+        }
+      } else {
+        const float rx = tt.x - cx, ry = tt.y - cy, rz = tt.z - cz;
+        const float r2 = fmaf(rx, rx, fmaf(ry, ry, rz * rz));
+        const float ir = __builtin_amdgcn_rsqf(r2);
+        const float qx = fmaf(s.qxx, rx, fmaf(s.qxy, ry, s.qxz * rz));
+        const float qy = fmaf(s.qxy, rx, fmaf(s.qyy, ry, s.qyz * rz));
+        const float qz = fmaf(s.qxz, rx, fmaf(s.qyz, ry, s.qzz * rz));
+        const float qir = 0.5f * fmaf(qx, rx, fmaf(qy, ry, qz * rz));
+        const float rw = fmaf(rx, tt.wx, fmaf(ry, tt.wy, rz * tt.wz));
+        const float qw = fmaf(qx, tt.wx, fmaf(qy, tt.wy, qz * tt.wz));
+        float b, c, d, k1, k2;
+        if (FAR) {
+          const float a2 = ir * ir;
+          b = ir * a2;
+          c = 3.0f * b * a2;
+          d = 5.0f * c * a2;
+          k1 = fmaf(-c, s.mass, d * fmaf(-7.0f * a2, qir, tr));
+          k2 = -d;
+        } else {
+          const SplineQ32 q = splineq_grad32(r2 * ir, ir, r2, s.soft + tt.e);
+          b = q.b;
+          c = q.c;
+          d = q.d;
+          k1 = fmaf(s.mass, q.br, fmaf(qir, q.dr_, -tr * q.cr)) * ir;
+          k2 = q.cr * ir;
+          lam[10] += fmaf(-fmaf(q.bt, s.mass, fmaf(q.dt_, qir, -q.ct * tr)), rw, q.ct * qw);
+        }
+        const float qir3 = fmaf(b, s.mass, fmaf(d, qir, -c * tr));
+        const float s1 = fmaf(k2, qw, -k1 * rw);
+        const float hd = -0.5f * (d * rw);
+        const float px = fmaf(hd, rx, c * tt.wx), py = fmaf(hd, ry, c * tt.wy),
+                    pz = fmaf(hd, rz, c * tt.wz);
+        const float Qpx = fmaf(s.qxx, px, fmaf(s.qxy, py, s.qxz * pz));
+        const float Qpy = fmaf(s.qxy, px, fmaf(s.qyy, py, s.qyz * pz));
+        const float Qpz = fmaf(s.qxz, px, fmaf(s.qyz, py, s.qzz * pz));
+        const float Jx = fmaf(-qir3, tt.wx, fmaf(s1, rx, fmaf(hd, qx, Qpx)));
+        const float Jy = fmaf(-qir3, tt.wy, fmaf(s1, ry, fmaf(hd, qy, Qpy)));
+        const float Jz = fmaf(-qir3, tt.wz, fmaf(s1, rz, fmaf(hd, qz, Qpz)));
+        tgt_add(acc, t, (double)Jx, (double)Jy, (double)Jz);
+        lam[0] -= Jx;
+        lam[1] -= Jy;
+        lam[2] -= Jz;
+        lam[3] = fmaf(-b, rw, lam[3]);
+        lam[4] = fmaf(rx, px, lam[4]);
+        lam[5] = fmaf(ry, px, fmaf(rx, py, lam[5]));
+        lam[6] = fmaf(rz, px, fmaf(rx, pz, lam[6]));
+        lam[7] = fmaf(ry, py, lam[7]);
+        lam[8] = fmaf(rz, py, fmaf(ry, pz, lam[8]));
+        lam[9] = fmaf(rz, pz, lam[9]);
+        trace = fmaf(c, rw, trace);
+      }
+    }
+  }
+  lam[4] = fmaf(0.5f, trace, lam[4]);
+  lam[7] = fmaf(0.5f, trace, lam[7]);
+  lam[9] = fmaf(0.5f, trace, lam[9]);
+}
+
+// particle_pairs in FP32, the target gradients summed in FP64.
+template <bool FAR>
+__device__ __forceinline__ void particle_pairs32(float jx, float jy, float jz, float jm, float je,
+                                                 unsigned jmask, const TgtA32* __restrict__ st,
+                                                 int ng, double* __restrict__ acc, float& sgx,
+                                                 float& sgy, float& sgz, float& sgm) {
+#pragma unroll 2
+  for (int t = 0; t < ng; t++) {
+    const TgtA32 tt = st[t];
+    if ((jmask >> tt.bt) & 1u) {
       const float dx = jx - tt.x, dy = jy - tt.y, dz = jz - tt.z;
       const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-      if (far || r2 != 0.0f) {
+      if (FAR || r2 != 0.0f) {
         const float ir = __builtin_amdgcn_rsqf(r2);
         float bb, db;
-        if (far) {
+        if (FAR) {
           bb = ir * ir * ir;
           db = -3.0f * bb * ir;
         } else {
@@ -646,13 +740,11 @@ __device__ __forceinline__ void particle_pairs32(bool far, float jx, float jy, f
         const float Kx = jm * fmaf(bb, tt.wx, f * dx);
         const float Ky = jm * fmaf(bb, tt.wy, f * dy);
         const float Kz = jm * fmaf(bb, tt.wz, f * dz);
-        tg[t][0] -= (double)Kx;
-        tg[t][1] -= (double)Ky;
-        tg[t][2] -= (double)Kz;
+        tgt_add(acc, t, -(double)Kx, -(double)Ky, -(double)Kz);
         sgx += Kx;
         sgy += Ky;
         sgz += Kz;
-        sgm += bb * dw;
+        sgm = fmaf(bb, dw, sgm);
       }
     }
   }
@@ -661,9 +753,9 @@ __device__ __forceinline__ void particle_pairs32(bool far, float jx, float jy, f
 // adjoint_group_kernel in the FP32 form (same work mapping; node moments from
 // the FP32 copies, node centres and softening decisions from the FP64 fields
 // of the same records).
-__global__ void __launch_bounds__(kAdjThreads)
+__global__ void __launch_bounds__(PT_WAVE)
 adjoint_group32_kernel(const Bucket* __restrict__ bk, const int32_t* __restrict__ gfirst,
-                       const int32_t* __restrict__ gnb, int64_t ns,
+                       const int32_t* __restrict__ gnb, const uint32_t* __restrict__ ngroups,
                       const TreeNode* __restrict__ nodes, const GravNode32* __restrict__ gn32,
                       const double* __restrict__ px,
                       const double* __restrict__ py, const double* __restrict__ pz,
@@ -676,43 +768,42 @@ adjoint_group32_kernel(const Bucket* __restrict__ bk, const int32_t* __restrict_
                       double* __restrict__ gx, double* __restrict__ gy, double* __restrict__ gz,
                       double* __restrict__ gmass, double* __restrict__ lam_node, int64_t nn,
                       double* __restrict__ hot, int64_t nhot) {
-  __shared__ TgtA32 s_t[kAdjWaves][kANT];
-  __shared__ Bucket s_bk[kAdjWaves][PT_GROUP_BUCKETS];
-  __shared__ int32_t s_beg[kAdjWaves][PT_WAVE];
-  __shared__ double s_far[kAdjWaves][kPassFar];
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PT_WAVE);
-  const int lane = threadIdx.x & (PT_WAVE - 1);
-  const int64_t gi = (int64_t)blockIdx.x * kAdjWaves + wave;
-  if (gi >= ns) return;
+  __shared__ TgtA32 s_t[kANT];
+  __shared__ Bucket s_bk[PT_GROUP_BUCKETS];
+  __shared__ int32_t s_beg[PT_WAVE];
+  __shared__ double s_far[kPassFar];
+  __shared__ double s_acc[kANT * 3 * kAccStride];
+  const int lane = threadIdx.x;
+  const int64_t gi = pt_part_item((int32_t)ngroups[0]);
+  if (gi < 0) return;
   const int nbk = gnb[gi];
-  if (nbk <= 0) return;
   const int64_t b0 = gfirst[gi];
-  if (lane < nbk) s_bk[wave][lane] = bk[b0 + lane];
+  if (lane < nbk) s_bk[lane] = bk[b0 + lane];
   __builtin_amdgcn_wave_barrier();
   // the group's targets are consecutive: its buckets' ranges in order
-  const int64_t first = s_bk[wave][0].begin;
-  const int nt = (int)((int64_t)s_bk[wave][nbk - 1].begin + s_bk[wave][nbk - 1].count - first);
+  const int64_t first = s_bk[0].begin;
+  const int nt = (int)((int64_t)s_bk[nbk - 1].begin + s_bk[nbk - 1].count - first);
   // FP32 frame: the centre of the box around the group's bucket boxes
-  double lx = s_bk[wave][0].lox, ly = s_bk[wave][0].loy, lz = s_bk[wave][0].loz;
-  double hx = s_bk[wave][0].hix, hy = s_bk[wave][0].hiy, hz = s_bk[wave][0].hiz;
+  double lx = s_bk[0].lox, ly = s_bk[0].loy, lz = s_bk[0].loz;
+  double hx = s_bk[0].hix, hy = s_bk[0].hiy, hz = s_bk[0].hiz;
   for (int k = 1; k < nbk; k++) {
-    lx = fmin(lx, s_bk[wave][k].lox);
-    ly = fmin(ly, s_bk[wave][k].loy);
-    lz = fmin(lz, s_bk[wave][k].loz);
-    hx = fmax(hx, s_bk[wave][k].hix);
-    hy = fmax(hy, s_bk[wave][k].hiy);
-    hz = fmax(hz, s_bk[wave][k].hiz);
+    lx = fmin(lx, s_bk[k].lox);
+    ly = fmin(ly, s_bk[k].loy);
+    lz = fmin(lz, s_bk[k].loz);
+    hx = fmax(hx, s_bk[k].hix);
+    hy = fmax(hy, s_bk[k].hiy);
+    hz = fmax(hz, s_bk[k].hiz);
   }
   const double ccx = (lx + hx) * 0.5, ccy = (ly + hy) * 0.5, ccz = (lz + hz) * 0.5;
   if (lane < 7) {
     // the group's box and largest bucket softening
     double v = lane < 3 ? INFINITY : (lane < 6 ? -INFINITY : 0.0);
     for (int k = 0; k < nbk; k++) {
-      const Bucket& bb = s_bk[wave][k];
+      const Bucket& bb = s_bk[k];
       const double c[7] = {bb.lox, bb.loy, bb.loz, bb.hix, bb.hiy, bb.hiz, bb.soft};
       v = lane < 3 ? fmin(v, c[lane]) : fmax(v, c[lane]);
     }
-    s_far[wave][lane] = v;
+    s_far[lane] = v;
   }
   const int64_t pc0 = pc_off[gi], pc1 = pc_off[gi + 1];
   const int64_t pp0 = pp_off[gi], pp1 = pp_off[gi + 1];
@@ -721,7 +812,7 @@ adjoint_group32_kernel(const Bucket* __restrict__ bk, const int32_t* __restrict_
     // member buckets with a target in this pass
     unsigned pass = 0;
     for (int k = 0; k < nbk; k++) {
-      const int64_t lo = s_bk[wave][k].begin, hi = lo + s_bk[wave][k].count;
+      const int64_t lo = s_bk[k].begin, hi = lo + s_bk[k].count;
       if (hi > first + g0 && lo < first + g0 + ng) pass |= 1u << k;
     }
     __builtin_amdgcn_wave_barrier();
@@ -729,20 +820,19 @@ adjoint_group32_kernel(const Bucket* __restrict__ bk, const int32_t* __restrict_
       const int64_t i = first + g0 + lane;
       int bt = 0;
       for (int k = 1; k < nbk; k++)
-        if (i >= s_bk[wave][k].begin) bt = k;
-      s_t[wave][lane] = TgtA32{(float)(px[i] - ccx), (float)(py[i] - ccy), (float)(pz[i] - ccz),
+        if (i >= s_bk[k].begin) bt = k;
+      s_t[lane] = TgtA32{(float)(px[i] - ccx), (float)(py[i] - ccy), (float)(pz[i] - ccz),
                                (float)pe[i], (float)wx[i], (float)wy[i], (float)wz[i], bt};
     }
-    __builtin_amdgcn_wave_barrier();
-    double tg[kANT][3];
-#pragma unroll
-    for (int t = 0; t < kANT; t++) tg[t][0] = tg[t][1] = tg[t][2] = 0.0;
+    for (int k = lane; k < 3 * ng * kAccStride; k += PT_WAVE) s_acc[k] = 0.0;
+    __syncthreads();
+    double* const acc = s_acc + lane % kAccCols;
     if (lane == 0) {
       double emax = 0.0;
-      for (int t = 0; t < ng; t++) emax = fmax(emax, (double)s_t[wave][t].e);
-      s_far[wave][7] = emax;
+      for (int t = 0; t < ng; t++) emax = fmax(emax, (double)s_t[t].e);
+      s_far[7] = emax;
     }
-    __builtin_amdgcn_wave_barrier();
+    __syncthreads();
 
     // ---- node() sources
     for (int64_t e0 = pc0; e0 < pc1; e0 += PT_WAVE) {
@@ -753,89 +843,24 @@ adjoint_group32_kernel(const Bucket* __restrict__ bk, const int32_t* __restrict_
         const GravNode32 s = gn32[sid];
         const double cxd = s.cx + ox, cyd = s.cy + oy, czd = s.cz + oz;
         // over the lanes holding an entry (the others are inactive here)
-        const bool all_far = __ballot(!node_far_pass(s_far[wave], cxd, cyd, czd, s.soft64)) == 0ull;
+        const bool all_far = __ballot(!node_far_pass(s_far, cxd, cyd, czd, s.soft64)) == 0ull;
         // members for which openSoftening sends it to addGravity (none when
         // every entry of the chunk is far)
         unsigned mono = 0;
         if (!all_far) {
           for (unsigned mm = mask; mm != 0u; mm &= mm - 1u) {
             const int k = __builtin_ctz(mm);
-            if (pt_open_softening(cxd, cyd, czd, s.soft64, s_bk[wave][k])) mono |= 1u << k;
+            if (pt_open_softening(cxd, cyd, czd, s.soft64, s_bk[k])) mono |= 1u << k;
           }
         }
         const float cx = (float)(cxd - ccx), cy = (float)(cyd - ccy), cz = (float)(czd - ccz);
-        const float tr = 0.5f * (s.qxx + s.qyy + s.qzz);
         float lam[kNodeAdj];
 #pragma unroll
         for (int k = 0; k < kNodeAdj; k++) lam[k] = 0.0f;
-#pragma unroll
-        for (int t = 0; t < kANT; t++) {
-          if (t < ng && ((mask >> s_t[wave][t].bt) & 1u)) {
-            const TgtA32 tt = s_t[wave][t];
-            if ((mono >> tt.bt) & 1u) {
-              const float dx = cx - tt.x, dy = cy - tt.y, dz = cz - tt.z;
-              const float r2 = dx * dx + dy * dy + dz * dz;
-              if (r2 != 0.0f) {
-                const float ir = __builtin_amdgcn_rsqf(r2);
-                const float ir3 = ir * ir * ir;
-                const float dw = dx * tt.wx + dy * tt.wy + dz * tt.wz;
-                const float f = -3.0f * s.mass * ir3 * ir * ir * dw;
-                const float Tx = s.mass * ir3 * tt.wx + f * dx;
-                const float Ty = s.mass * ir3 * tt.wy + f * dy;
-                const float Tz = s.mass * ir3 * tt.wz + f * dz;
-                tg[t][0] -= (double)Tx;
-                tg[t][1] -= (double)Ty;
-                tg[t][2] -= (double)Tz;
-                lam[0] += Tx;
-                lam[1] += Ty;
-                lam[2] += Tz;
-                lam[3] += dw * ir3;
-              }
-            } else {
-              const float rx = tt.x - cx, ry = tt.y - cy, rz = tt.z - cz;
-              const float r2 = fmaf(rx, rx, fmaf(ry, ry, rz * rz));
-              const float ir = __builtin_amdgcn_rsqf(r2);
-              const float r = r2 * ir;
-              const SplineQ32 q = splineq_grad32(r, ir, r2, s.soft + tt.e);
-              const float qx = fmaf(s.qxx, rx, fmaf(s.qxy, ry, s.qxz * rz));
-              const float qy = fmaf(s.qxy, rx, fmaf(s.qyy, ry, s.qyz * rz));
-              const float qz = fmaf(s.qxz, rx, fmaf(s.qyz, ry, s.qzz * rz));
-              const float qir = 0.5f * fmaf(qx, rx, fmaf(qy, ry, qz * rz));
-              const float qir3 = fmaf(q.b, s.mass, fmaf(q.d, qir, -q.c * tr));
-              const float rw = fmaf(rx, tt.wx, fmaf(ry, tt.wy, rz * tt.wz));
-              const float qw = fmaf(qx, tt.wx, fmaf(qy, tt.wy, qz * tt.wz));
-              const float Qwx = fmaf(s.qxx, tt.wx, fmaf(s.qxy, tt.wy, s.qxz * tt.wz));
-              const float Qwy = fmaf(s.qxy, tt.wx, fmaf(s.qyy, tt.wy, s.qyz * tt.wz));
-              const float Qwz = fmaf(s.qxz, tt.wx, fmaf(s.qyz, tt.wy, s.qzz * tt.wz));
-              const float k1 = fmaf(s.mass, q.br, fmaf(qir, q.dr_, -tr * q.cr)) * ir;
-              const float k2 = q.cr * ir;
-              // J = -qir3 w + (k2 (q.w) - k1 (r.w)) r - d (r.w) q + c Q w
-              const float s1 = fmaf(k2, qw, -k1 * rw);
-              const float drw = q.d * rw;
-              const float Jx = fmaf(-qir3, tt.wx, fmaf(s1, rx, fmaf(-drw, qx, q.c * Qwx)));
-              const float Jy = fmaf(-qir3, tt.wy, fmaf(s1, ry, fmaf(-drw, qy, q.c * Qwy)));
-              const float Jz = fmaf(-qir3, tt.wz, fmaf(s1, rz, fmaf(-drw, qz, q.c * Qwz)));
-              tg[t][0] += (double)Jx;
-              tg[t][1] += (double)Jy;
-              tg[t][2] += (double)Jz;
-              lam[0] -= Jx;
-              lam[1] -= Jy;
-              lam[2] -= Jz;
-              lam[3] = fmaf(-q.b, rw, lam[3]);
-              // d(a.w)/dQ as r_k p_l + r_l p_k (+ the trace part), p = -d (r.w) r / 2 + c w
-              const float hd = -0.5f * drw, hc = 0.5f * q.c * rw;
-              const float qpx = fmaf(hd, rx, q.c * tt.wx), qpy = fmaf(hd, ry, q.c * tt.wy),
-                          qpz = fmaf(hd, rz, q.c * tt.wz);
-              lam[4] += fmaf(rx, qpx, hc);
-              lam[5] += fmaf(ry, qpx, rx * qpy);
-              lam[6] += fmaf(rz, qpx, rx * qpz);
-              lam[7] += fmaf(ry, qpy, hc);
-              lam[8] += fmaf(rz, qpy, ry * qpz);
-              lam[9] += fmaf(rz, qpz, hc);
-              lam[10] += fmaf(-fmaf(q.bt, s.mass, fmaf(q.dt_, qir, -q.ct * tr)), rw, q.ct * qw);
-            }
-          }
-        }
+        if (all_far)
+          node_entry_pairs32<true>(s, cx, cy, cz, mask, 0u, s_t, ng, acc, lam);
+        else
+          node_entry_pairs32<false>(s, cx, cy, cz, mask, mono, s_t, ng, acc, lam);
         double* dst = sid < nhot
                           ? hot + (int64_t)(blockIdx.x % kHotParts) * kNodeAdj * nhot + sid
                           : lam_node + sid;
@@ -857,7 +882,7 @@ adjoint_group32_kernel(const Bucket* __restrict__ bk, const int32_t* __restrict_
         const TreeNode nd = nodes[pp[l]];
         cnt = nd.count;
         beg = nd.begin;
-        isnear = !leaf_far_pass(s_far[wave], nd.cx + ox, nd.cy + oy, nd.cz + oz, nd.leaf_reach,
+        isnear = !leaf_far_pass(s_far, nd.cx + ox, nd.cy + oy, nd.cz + oz, nd.leaf_reach,
                                 nd.leaf_soft);
       }
       const int cn = isnear ? cnt : 0, cf = isnear ? 0 : cnt;
@@ -873,7 +898,7 @@ adjoint_group32_kernel(const Bucket* __restrict__ bk, const int32_t* __restrict_
         // a slot's entry: the lane of the last entry start at or below it in
         // this window (marks by start slot, a ballot of the marks), or the
         // previous window's last entry
-        int32_t* mark = s_beg[wave];
+        int32_t* mark = s_beg;
         mark[lane] = -1;
         __builtin_amdgcn_wave_barrier();
         if (cnt > 0 && exc >= s0 && exc < s0 + PT_WAVE) mark[exc - s0] = lane;
@@ -892,7 +917,10 @@ adjoint_group32_kernel(const Bucket* __restrict__ bk, const int32_t* __restrict_
                       jz = (float)((pz[j] + oz) - ccz);
           const float jm = (float)pm[j], je = (float)pe[j];
           float sgx = 0.0f, sgy = 0.0f, sgz = 0.0f, sgm = 0.0f;
-          particle_pairs32(wfar, jx, jy, jz, jm, je, jmask, s_t[wave], ng, tg, sgx, sgy, sgz, sgm);
+          if (wfar)
+            particle_pairs32<true>(jx, jy, jz, jm, je, jmask, s_t, ng, acc, sgx, sgy, sgz, sgm);
+          else
+            particle_pairs32<false>(jx, jy, jz, jm, je, jmask, s_t, ng, acc, sgx, sgy, sgz, sgm);
           atomicAdd(&gx[j], (double)sgx);
           atomicAdd(&gy[j], (double)sgy);
           atomicAdd(&gz[j], (double)sgz);
@@ -902,20 +930,9 @@ adjoint_group32_kernel(const Bucket* __restrict__ bk, const int32_t* __restrict_
       __builtin_amdgcn_wave_barrier();
     }
 
-#pragma unroll
-    for (int t = 0; t < kANT; t++) {
-      if (t < ng) {
-        const double rx = pt_wave_sum(tg[t][0]);
-        const double ry = pt_wave_sum(tg[t][1]);
-        const double rz = pt_wave_sum(tg[t][2]);
-        if (lane == t) {
-          const int64_t i = first + g0 + t;
-          atomicAdd(&gx[i], rx);
-          atomicAdd(&gy[i], ry);
-          atomicAdd(&gz[i], rz);
-        }
-      }
-    }
+    __syncthreads();
+    tgt_flush(s_acc, ng, first + g0, gx, gy, gz);
+    __syncthreads();
   }
 }
 
@@ -1148,8 +1165,9 @@ int64_t pt_adjoint_node_scratch(int64_t nn) {
 int pt_node_adjoint_fields() { return kNodeAdj; }
 
 int pt_launch_adjoint_groups(int precision, const Bucket* bk, const int32_t* gfirst,
-                             const int32_t* gnb, int64_t ns, const TreeNode* nodes,
-                             const GravNode* gn, const GravNode32* gn32, const double* x,
+                             const int32_t* gnb, const uint32_t* ngroups, int64_t ns,
+                             const TreeNode* nodes, const GravNode* gn,
+                             const GravNode32* gn32, const double* x,
                              const double* y, const double* z, const double* m, const double* e,
                              const int64_t* pp_off, const int32_t* pp, const uint8_t* ppm,
                              const int64_t* pc_off, const int32_t* pc, const uint8_t* pcm,
@@ -1161,15 +1179,15 @@ int pt_launch_adjoint_groups(int precision, const Bucket* bk, const int32_t* gfi
   // the node cotangents, then the private copies of the hot ones
   const int64_t nhot = std::min<int64_t>(nn, kHotNodes);
   double* hot = lam_node + (int64_t)kNodeAdj * nn;
-  const unsigned grid = (unsigned)((ns + kAdjWaves - 1) / kAdjWaves);
+  const unsigned grid = (unsigned)pt_part_blocks(ns);
   if (precision != 0)  // the compensated-FP32 precision
-    adjoint_group32_kernel<<<grid, kAdjThreads, 0, s>>>(
-        bk, gfirst, gnb, ns, nodes, gn32, x, y, z, m, e, pp_off, pp, ppm, pc_off, pc, pcm, off[0],
-        off[1], off[2], wx, wy, wz, gx, gy, gz, gm, lam_node, nn, hot, nhot);
+    adjoint_group32_kernel<<<grid, PT_WAVE, 0, s>>>(
+        bk, gfirst, gnb, ngroups, nodes, gn32, x, y, z, m, e, pp_off, pp, ppm, pc_off, pc, pcm,
+        off[0], off[1], off[2], wx, wy, wz, gx, gy, gz, gm, lam_node, nn, hot, nhot);
   else
-    adjoint_group_kernel<<<grid, kAdjThreads, 0, s>>>(
-        bk, gfirst, gnb, ns, nodes, gn, x, y, z, m, e, pp_off, pp, ppm, pc_off, pc, pcm, off[0],
-        off[1], off[2], wx, wy, wz, gx, gy, gz, gm, lam_node, nn, hot, nhot);
+    adjoint_group_kernel<<<grid, PT_WAVE, 0, s>>>(
+        bk, gfirst, gnb, ngroups, nodes, gn, x, y, z, m, e, pp_off, pp, ppm, pc_off, pc, pcm,
+        off[0], off[1], off[2], wx, wy, wz, gx, gy, gz, gm, lam_node, nn, hot, nhot);
   hot_reduce_kernel<<<grid_for(nhot * kNodeAdj), 256, 0, s>>>(hot, nhot, lam_node, nn);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }

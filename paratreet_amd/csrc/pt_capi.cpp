@@ -116,7 +116,7 @@ struct pt_ctx {
   DBuf<double> adj;       // adjoint work arrays (17n)
   DBuf<double> lam_node;  // node cotangents, field-major
   // bucket groups and their member-masked lists (the adjoint's lists)
-  DBuf<int32_t> gfirst, gnb, gpp_cnt, gpc_cnt, gpp, gpc;
+  DBuf<int32_t> gslots, gpp, gpc;
   DBuf<uint8_t> gppm, gpcm;
   DBuf<int64_t> gpp_off, gpc_off;
   int64_t n_gpp = 0, n_gpc = 0;
@@ -386,7 +386,7 @@ void pt_ctx_destroy(pt_ctx* c) {
   release(c->pp_off); release(c->pc_off); release(c->i64_total);
   release(c->counters); release(c->derr); release(c->scratch);
   release(c->ckpt); release(c->seg); release(c->adj); release(c->lam_node);
-  release(c->gfirst); release(c->gnb); release(c->gpp_cnt); release(c->gpc_cnt);
+  release(c->gslots);
   release(c->gpp); release(c->gpc); release(c->gppm); release(c->gpcm);
   release(c->gpp_off); release(c->gpc_off);
   release(c->dual_a); release(c->dual_b); release(c->dual_pp); release(c->dual_pc);
@@ -976,6 +976,23 @@ static int group_cap(pt_ctx* c, pt_precision precision, int64_t n_rep) {
   return per_slot >= (n_rep > 1 ? 16 : f32 ? 8 : 4) ? 8 : 0;
 }
 
+// Bucket groups of at most cap particles and `most` buckets: nb entries of
+// first and count each, their number in *ngroups (device).
+static pt_status bucket_groups(pt_ctx* c, int cap, int most, int32_t* first, int32_t* count,
+                               uint32_t* ngroups) {
+  pt_status st;
+  const int64_t nb = c->nb, nw = pt_fgroup_windows(nb);
+  PT_TRY_HIP(c, ensure(c->fg_tfirst, nb));
+  PT_TRY_HIP(c, ensure(c->fg_tnb, nb));
+  PT_TRY_HIP(c, ensure(c->fg_wcount, nw));
+  PT_TRY_HIP(c, ensure(c->fg_woff, nw));
+  if ((st = ensure_scratch(c, pt_scan_scratch_bytes(nw)))) return st;
+  PT_TRY_LAUNCH(c, pt_launch_fgroups(c->bk.p, nb, cap, most, c->fg_tfirst.p, c->fg_tnb.p,
+                                     c->fg_wcount.p, c->fg_woff.p, c->scratch.p, ngroups,
+                                     first, count, c->stream));
+  return PT_OK;
+}
+
 // Fused walk + interactions (no lists), with a large-stack rerun if the walk
 // stack overflowed for some bucket.
 static pt_status gravity_fused(pt_ctx* c, double theta, const double offset[3],
@@ -998,19 +1015,11 @@ static pt_status gravity_fused(pt_ctx* c, double theta, const double offset[3],
   PT_TRY_HIP(c, ensure(c->cpart, nblk * 4));
   if (grouped) {
     // the bucket groups of this tree (every replica walks with them)
-    const int64_t nw = pt_fgroup_windows(nb);
-    PT_TRY_HIP(c, ensure(c->fg_tfirst, nb));
-    PT_TRY_HIP(c, ensure(c->fg_tnb, nb));
     PT_TRY_HIP(c, ensure(c->fg_first, nb));
     PT_TRY_HIP(c, ensure(c->fg_nb, nb));
-    PT_TRY_HIP(c, ensure(c->fg_wcount, nw));
-    PT_TRY_HIP(c, ensure(c->fg_woff, nw));
     PT_TRY_HIP(c, ensure(c->fg_ng, 1));
-    if ((st = ensure_scratch(c, pt_scan_scratch_bytes(nw)))) return st;
     Timer t(c, PT_T_TRAVERSE);
-    PT_TRY_LAUNCH(c, pt_launch_fgroups(c->bk.p, nb, cap, c->fg_tfirst.p, c->fg_tnb.p, c->fg_wcount.p,
-                                       c->fg_woff.p, c->scratch.p, c->fg_ng.p, c->fg_first.p,
-                                       c->fg_nb.p, c->stream));
+    if ((st = bucket_groups(c, cap, PT_WAVE, c->fg_first.p, c->fg_nb.p, c->fg_ng.p))) return st;
   }
   // the visitor offsets: one, or the (2N+1)^3 period replicas in the order of
   // ExMain::traversalFn (examples/Gravity.C:35-46), each added to `offset`;
@@ -1304,22 +1313,27 @@ pt_status group_lists(pt_ctx* c, double theta) {
   const int64_t ns = pt_group_slots(nb);
   if (ns <= 0) return fail(c, PT_ERR_STATE, "no buckets");
   Timer t(c, PT_T_TRAVERSE);
-  PT_TRY_HIP(c, ensure(c->gfirst, ns));
-  PT_TRY_HIP(c, ensure(c->gnb, ns));
-  PT_TRY_HIP(c, ensure(c->gpp_cnt, ns));
-  PT_TRY_HIP(c, ensure(c->gpc_cnt, ns));
+  // per slot, zero behind the last group: first bucket, buckets, list lengths;
+  // then the number of groups
+  PT_TRY_HIP(c, ensure(c->gslots, 4 * ns + 1));
+  int32_t* const gfirst = c->gslots.p;
+  int32_t *const gnb = gfirst + ns, *const gpp_cnt = gfirst + 2 * ns,
+          *const gpc_cnt = gfirst + 3 * ns;
+  uint32_t* const ngroups = (uint32_t*)(gfirst + 4 * ns);
   PT_TRY_HIP(c, ensure(c->gpp_off, ns + 1));
   PT_TRY_HIP(c, ensure(c->gpc_off, ns + 1));
   if ((st = ensure_scratch(c, pt_scan_scratch_bytes(ns + 1)))) return st;
   PT_TRY_LAUNCH(c, pt_launch_fill_u32((uint32_t*)c->derr.p, 1, 0u, c->stream));
-  PT_TRY_LAUNCH(c, pt_launch_group_buckets(c->bk.p, nb, c->gfirst.p, c->gnb.p, c->stream));
-  PT_TRY_LAUNCH(c, pt_launch_group_traverse(false, c->tnode.p, c->bk.p, c->gfirst.p, c->gnb.p,
-                                            ns, gf, c->offset, c->gpp_cnt.p, c->gpc_cnt.p,
+  PT_TRY_LAUNCH(c, pt_launch_fill_u32((uint32_t*)c->gslots.p, 4 * ns, 0u, c->stream));
+  if ((st = bucket_groups(c, PT_GROUP_TARGETS, PT_GROUP_BUCKETS, gfirst, gnb, ngroups)))
+    return st;
+  PT_TRY_LAUNCH(c, pt_launch_group_traverse(false, c->tnode.p, c->bk.p, gfirst, gnb, ngroups,
+                                            ns, gf, c->offset, gpp_cnt, gpc_cnt,
                                             nullptr, nullptr, nullptr, nullptr, nullptr, nullptr,
                                             c->derr.p, c->stream));
-  PT_TRY_LAUNCH(c, pt_exclusive_scan_i32_to_i64(c->gpp_cnt.p, c->gpp_off.p, ns, c->scratch.p,
+  PT_TRY_LAUNCH(c, pt_exclusive_scan_i32_to_i64(gpp_cnt, c->gpp_off.p, ns, c->scratch.p,
                                                 c->gpp_off.p + ns, c->stream));
-  PT_TRY_LAUNCH(c, pt_exclusive_scan_i32_to_i64(c->gpc_cnt.p, c->gpc_off.p, ns, c->scratch.p,
+  PT_TRY_LAUNCH(c, pt_exclusive_scan_i32_to_i64(gpc_cnt, c->gpc_off.p, ns, c->scratch.p,
                                                 c->gpc_off.p + ns, c->stream));
   int64_t tot[2] = {0, 0};
   int32_t herr = 0;
@@ -1333,7 +1347,7 @@ pt_status group_lists(pt_ctx* c, double theta) {
   PT_TRY_HIP(c, ensure(c->gppm, std::max<int64_t>(tot[0], 1)));
   PT_TRY_HIP(c, ensure(c->gpc, std::max<int64_t>(tot[1], 1)));
   PT_TRY_HIP(c, ensure(c->gpcm, std::max<int64_t>(tot[1], 1)));
-  PT_TRY_LAUNCH(c, pt_launch_group_traverse(true, c->tnode.p, c->bk.p, c->gfirst.p, c->gnb.p,
+  PT_TRY_LAUNCH(c, pt_launch_group_traverse(true, c->tnode.p, c->bk.p, gfirst, gnb, ngroups,
                                             ns, gf, c->offset, nullptr, nullptr, c->gpp_off.p,
                                             c->gpc_off.p, c->gpp.p, c->gppm.p, c->gpc.p,
                                             c->gpcm.p, c->derr.p, c->stream));
@@ -1366,11 +1380,12 @@ pt_status vjp_accumulate(pt_ctx* c, int mode, double theta, const AdjViews& v, c
   if ((st = zero(c, c->lam_node.p, nscr))) return st;
   if ((st = zero(c, v.gsx, 4 * std::max<int64_t>(n, 1)))) return st;  // gsx gsy gsz gsm
   PT_TRY_LAUNCH(c, pt_launch_gather3(c->perm.p, n, wx, wy, wz, v.wsx, v.wsy, v.wsz, c->stream));
+  const int64_t ns = pt_group_slots(c->nb);
   PT_TRY_LAUNCH(c, pt_launch_adjoint_groups(
-                       c->adj_prec, c->bk.p, c->gfirst.p, c->gnb.p, pt_group_slots(c->nb),
-                       c->tnode.p, c->gn.p, c->gn32.p, c->xs.p, c->ys.p, c->zs.p, c->ms.p,
-                       c->es.p, c->gpp_off.p, c->gpp.p, c->gppm.p, c->gpc_off.p, c->gpc.p,
-                       c->gpcm.p, c->offset, v.wsx, v.wsy, v.wsz, v.gsx, v.gsy, v.gsz, v.gsm,
+                       c->adj_prec, c->bk.p, c->gslots.p, c->gslots.p + ns,
+                       (uint32_t*)(c->gslots.p + 4 * ns), ns, c->tnode.p, c->gn.p, c->gn32.p,
+                       c->xs.p, c->ys.p, c->zs.p, c->ms.p, c->es.p, c->gpp_off.p, c->gpp.p,
+                       c->gppm.p, c->gpc_off.p, c->gpc.p, c->gpcm.p, c->offset, v.wsx, v.wsy, v.wsz, v.gsx, v.gsy, v.gsz, v.gsm,
                        c->lam_node.p, nn, c->stream));
   PT_TRY_LAUNCH(c, pt_launch_adjoint_down(n, c->bucket_of.p, c->bucket_node.p, c->nparent.p,
                                           c->gn.p, c->lam_node.p, nn, c->xs.p,
@@ -1680,8 +1695,8 @@ pt_status pt_get_group_lists(pt_ctx* c, double theta, int64_t sizes[3], int32_t*
     if (!gnb || !pp_off || !pp || !ppm || !pc_off || !pc || !pcm)
       return fail(c, PT_ERR_ARG, "null output array");
     const hipMemcpyKind d2h = hipMemcpyDeviceToHost;
-    PT_TRY_HIP(c, hipMemcpyAsync(gfirst, c->gfirst.p, ns * 4, d2h, c->stream));
-    PT_TRY_HIP(c, hipMemcpyAsync(gnb, c->gnb.p, ns * 4, d2h, c->stream));
+    PT_TRY_HIP(c, hipMemcpyAsync(gfirst, c->gslots.p, ns * 4, d2h, c->stream));
+    PT_TRY_HIP(c, hipMemcpyAsync(gnb, c->gslots.p + ns, ns * 4, d2h, c->stream));
     PT_TRY_HIP(c, hipMemcpyAsync(pp_off, c->gpp_off.p, (ns + 1) * 8, d2h, c->stream));
     PT_TRY_HIP(c, hipMemcpyAsync(pc_off, c->gpc_off.p, (ns + 1) * 8, d2h, c->stream));
     if (c->n_gpp > 0) {

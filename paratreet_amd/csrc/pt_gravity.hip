@@ -1858,14 +1858,14 @@ grouped_gravity_kernel(const Bucket* __restrict__ bk, int64_t nb,
 
 // Bucket groups of the grouped kernel, formed greedily inside windows of
 // kFgWindow consecutive buckets: a group closes when the next bucket would
-// take it past cap (<= 64) particles, so a bucket of more than cap is a
-// group of its own.  One wave per window: the lanes load the window's counts, the greedy
-// pass runs on wave-uniform values.  Window w writes its groups to slots
+// take it past cap (<= 64) particles or `most` buckets, so a bucket of more
+// than cap is a group of its own.  One wave per window: the lanes load the
+// window's counts, the greedy pass runs on wave-uniform values.  Window w writes its groups to slots
 // [w kFgWindow, w kFgWindow + wcount[w]) of tfirst / tnb.
 constexpr int kFgWindow = PT_WAVE;
 
 __global__ void __launch_bounds__(256)
-fgroup_window_kernel(const Bucket* __restrict__ bk, int64_t nb, int cap,
+fgroup_window_kernel(const Bucket* __restrict__ bk, int64_t nb, int cap, int most,
                      int32_t* __restrict__ tfirst, int32_t* __restrict__ tnb,
                      uint32_t* __restrict__ wcount) {
   const int64_t w = (int64_t)blockIdx.x * 4 + threadIdx.x / PT_WAVE;
@@ -1878,7 +1878,7 @@ fgroup_window_kernel(const Bucket* __restrict__ bk, int64_t nb, int cap,
   int slot = 0, start = 0, tot = 0;
   for (int k = 0; k < n; k++) {
     const int c = __builtin_amdgcn_readlane(cnt, k);
-    if (k > start && tot + c > cap) {
+    if (k > start && (tot + c > cap || k - start >= most)) {
       if (lane == 0) {
         tfirst[b0 + slot] = (int32_t)(b0 + start);
         tnb[b0 + slot] = k - start;
@@ -1960,13 +1960,13 @@ int64_t pt_gravity_blocks(int64_t nb, int64_t n, int cap) {
   return 8 * ((groups + 7) / 8 + 1);
 }
 
-int pt_launch_fgroups(const Bucket* bk, int64_t nb, int cap, int32_t* tfirst, int32_t* tnb,
-                      uint32_t* wcount, uint32_t* woff, void* scratch, uint32_t* ngroups,
-                      int32_t* gfirst, int32_t* gnb, hipStream_t s) {
+int pt_launch_fgroups(const Bucket* bk, int64_t nb, int cap, int most, int32_t* tfirst,
+                      int32_t* tnb, uint32_t* wcount, uint32_t* woff, void* scratch,
+                      uint32_t* ngroups, int32_t* gfirst, int32_t* gnb, hipStream_t s) {
   if (nb <= 0) return 0;
   if (cap < 2 || cap > PT_WAVE) return -1;
   const int64_t nw = pt_fgroup_windows(nb);
-  fgroup_window_kernel<<<(unsigned)((nw + 3) / 4), 256, 0, s>>>(bk, nb, cap, tfirst, tnb,
+  fgroup_window_kernel<<<(unsigned)((nw + 3) / 4), 256, 0, s>>>(bk, nb, cap, most, tfirst, tnb,
                                                                  wcount);
   if (hipGetLastError() != hipSuccess) return -1;
   if (pt_exclusive_scan_u32(wcount, woff, nw, scratch, ngroups, s) != 0) return -1;

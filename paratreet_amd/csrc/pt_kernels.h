@@ -139,16 +139,16 @@ struct PtReplicas {
 int pt_launch_replica_table(int nr, const double off[3], const double period[3], double* tab,
                             hipStream_t s);
 // Bucket groups of the grouped fused kernel: runs of consecutive buckets of
-// at most cap (2..64) particles in all (a larger bucket alone), formed inside
-// windows of 64 buckets and compacted in order into gfirst / gnb, their
+// at most cap (2..64) particles in all (a larger bucket alone) and `most`
+// buckets, formed inside windows of 64 buckets and compacted in order into gfirst / gnb, their
 // number in *ngroups (device).  tfirst / tnb / gfirst / gnb hold nb entries,
 // wcount / woff pt_fgroup_windows(nb); scratch: pt_scan_scratch_bytes of the
 // window count.
 int64_t pt_fgroup_windows(int64_t nb);
 int64_t pt_fgroup_max_groups(int64_t nb, int64_t n, int cap);
-int pt_launch_fgroups(const Bucket* bk, int64_t nb, int cap, int32_t* tfirst, int32_t* tnb,
-                      uint32_t* wcount, uint32_t* woff, void* scratch, uint32_t* ngroups,
-                      int32_t* gfirst, int32_t* gnb, hipStream_t s);
+int pt_launch_fgroups(const Bucket* bk, int64_t nb, int cap, int most, int32_t* tfirst,
+                      int32_t* tnb, uint32_t* wcount, uint32_t* woff, void* scratch,
+                      uint32_t* ngroups, int32_t* gfirst, int32_t* gnb, hipStream_t s);
 // The fused walk + interactions: a shared walk per bucket group, or with
 // gfirst null (cap 0) one walk per bucket; counters as partials of
 // pt_gravity_blocks(nb, n, cap) work-groups.  precision 0 FP64, otherwise the
@@ -219,15 +219,12 @@ int pt_launch_min(const double* v, int64_t n, double* parts, int max_parts, doub
 
 // Bucket groups of the adjoint: runs of consecutive buckets (their particles
 // are consecutive) of at most PT_GROUP_BUCKETS buckets and, unless a single
-// bucket is larger, PT_GROUP_TARGETS particles, formed greedily inside aligned
-// windows of PT_GROUP_BUCKETS buckets.  Window w owns the slots
-// [w * PT_GROUP_BUCKETS, (w + 1) * PT_GROUP_BUCKETS); unused slots hold
-// gnb = 0.  pt_group_slots(nb) slots in all.
+// bucket is larger, PT_GROUP_TARGETS particles (pt_launch_fgroups).  The group
+// arrays have pt_group_slots(nb) entries, the groups first, their number on
+// the device; the rest hold gnb = 0.
 #define PT_GROUP_BUCKETS 8
 #define PT_GROUP_TARGETS 16
 int64_t pt_group_slots(int64_t nb);
-int pt_launch_group_buckets(const Bucket* bk, int64_t nb, int32_t* gfirst, int32_t* gnb,
-                            hipStream_t s);
 // The walk of pt_launch_traverse for every bucket of a group at once: a node
 // is visited when some member bucket visits it, and each list entry carries
 // the member mask (bit k = the group's k-th bucket) for which the node is a
@@ -236,9 +233,9 @@ int pt_launch_group_buckets(const Bucket* bk, int64_t nb, int32_t* gfirst, int32
 // Count pass (fill false: pp_cnt/pc_cnt per slot) and fill pass; err is set
 // when a walk stack overflows.
 int pt_launch_group_traverse(bool fill, const TreeNode* nodes, const Bucket* bk,
-                             const int32_t* gfirst, const int32_t* gnb, int64_t ns, double gf,
-                             const double off[3], int32_t* pp_cnt, int32_t* pc_cnt,
-                             const int64_t* pp_off, const int64_t* pc_off, int32_t* pp,
+                             const int32_t* gfirst, const int32_t* gnb, const uint32_t* ngroups,
+                             int64_t ns, double gf, const double off[3], int32_t* pp_cnt,
+                             int32_t* pc_cnt, const int64_t* pp_off, const int64_t* pc_off, int32_t* pp,
                              uint8_t* ppm, int32_t* pc, uint8_t* pcm, int32_t* err,
                              hipStream_t s);
 
@@ -250,8 +247,9 @@ int pt_launch_group_traverse(bool fill, const TreeNode* nodes, const Bucket* bk,
 int pt_node_adjoint_fields();
 int64_t pt_adjoint_node_scratch(int64_t nn);
 int pt_launch_adjoint_groups(int precision, const Bucket* bk, const int32_t* gfirst,
-                             const int32_t* gnb, int64_t ns, const TreeNode* nodes,
-                             const GravNode* gn, const GravNode32* gn32, const double* x,
+                             const int32_t* gnb, const uint32_t* ngroups, int64_t ns,
+                             const TreeNode* nodes, const GravNode* gn,
+                             const GravNode32* gn32, const double* x,
                              const double* y, const double* z, const double* m, const double* e,
                              const int64_t* pp_off, const int32_t* pp, const uint8_t* ppm,
                              const int64_t* pc_off, const int32_t* pc, const uint8_t* pcm,

@@ -306,6 +306,31 @@ __device__ __forceinline__ WalkLane pt_walk_step(const TreeNode* __restrict__ no
                                          leafm, closem, ho, gm, limit);
 }
 
+// The item of work-group i of a launch over n > 0 items, or -1: the items are
+// cut into kParts equal parts, and XCD x (work-groups are dispatched
+// round-robin over the 8 XCDs) takes parts x, x + 8, ..., each in order.
+// Neighbours, which share most of their source nodes, so share its L2; with 64
+// parts per XCD each XCD has its share of every region, where one contiguous
+// eighth per XCD leaves the chip to the XCD of the densest region; and the
+// work-groups without an item are the last ones, where unused items spread
+// over the index range had left whole XCDs idle (256k clustered particles,
+// FP64 adjoint: 7400 -> 4900 us; walk 430 -> 210 us).  pt_part_blocks(n)
+// work-groups serve any number of items up to n.  The result is made a scalar:
+// a divide leaves it in vector registers, and with it every address derived
+// from it.
+constexpr int kParts = 8 * 64;
+
+__device__ __forceinline__ int32_t pt_part_item(int32_t n) {
+  const int most = (n + kParts - 1) / kParts;
+  const int j = (int)(blockIdx.x / 8);
+  const int part = j / most * 8 + (int)(blockIdx.x % 8);
+  const int32_t item = (int32_t)((int64_t)n * part / kParts) + j % most;
+  const bool mine = part < kParts && item < (int32_t)((int64_t)n * (part + 1) / kParts);
+  return __builtin_amdgcn_readfirstlane(mine ? item : -1);
+}
+
+inline int64_t pt_part_blocks(int64_t n) { return (n + kParts - 1) / kParts * kParts; }
+
 // XCD-aware bucket order: work-groups are dispatched round-robin over the 8
 // XCDs, so group i is given the (i % 8)-th contiguous eighth of the buckets;
 // neighbouring buckets (which share most of their source nodes) then run on
