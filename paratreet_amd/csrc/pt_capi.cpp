@@ -114,7 +114,7 @@ struct pt_ctx {
   DBuf<double> ckpt;      // checkpoints, 6n each (x y z vx vy vz), + final state
   DBuf<double> seg;       // positions of the steps of one segment, 3n each
   DBuf<double> adj;       // adjoint work arrays (17n)
-  DBuf<double> lam_node;  // node cotangents, field-major
+  DBuf<double> lam_node;  // node cotangents, a record per node
   // bucket groups and their member-masked lists (the adjoint's lists)
   DBuf<int32_t> gslots, gpp, gpc;
   DBuf<uint8_t> gppm, gpcm;
@@ -1200,16 +1200,18 @@ namespace {
 struct AdjViews {
   double *lx, *ly, *lz, *lvx, *lvy, *lvz, *lm;   // caller order
   double *wx, *wy, *wz;                          // caller order
-  double *wsx, *wsy, *wsz, *gsx, *gsy, *gsz, *gsm;  // sorted order
+  double *wsx, *wsy, *wsz;                       // sorted order
+  double *gs;  // sorted order, records of 4: position gradient, mass gradient
 };
 
 pt_status adj_views(pt_ctx* c, AdjViews* v) {
   const int64_t n = std::max<int64_t>(c->n, 1);
   PT_TRY_HIP(c, ensure(c->adj, 17 * n));
   double* p = c->adj.p;
-  double** f[17] = {&v->lx, &v->ly, &v->lz, &v->lvx, &v->lvy, &v->lvz, &v->lm, &v->wx, &v->wy,
-                    &v->wz, &v->wsx, &v->wsy, &v->wsz, &v->gsx, &v->gsy, &v->gsz, &v->gsm};
-  for (int k = 0; k < 17; k++) *f[k] = p + k * n;
+  double** f[13] = {&v->lx, &v->ly, &v->lz, &v->lvx, &v->lvy, &v->lvz, &v->lm,
+                    &v->wx, &v->wy, &v->wz, &v->wsx, &v->wsy, &v->wsz};
+  v->gs = p;  // first, for the alignment of its records
+  for (int k = 0; k < 13; k++) *f[k] = p + (4 + k) * n;
   return PT_OK;
 }
 
@@ -1378,21 +1380,19 @@ pt_status vjp_accumulate(pt_ctx* c, int mode, double theta, const AdjViews& v, c
   PT_TRY_HIP(c, ensure(c->lam_node, nscr));
   Timer t(c, PT_T_ADJOINT);
   if ((st = zero(c, c->lam_node.p, nscr))) return st;
-  if ((st = zero(c, v.gsx, 4 * std::max<int64_t>(n, 1)))) return st;  // gsx gsy gsz gsm
+  if ((st = zero(c, v.gs, 4 * n))) return st;
   PT_TRY_LAUNCH(c, pt_launch_gather3(c->perm.p, n, wx, wy, wz, v.wsx, v.wsy, v.wsz, c->stream));
   const int64_t ns = pt_group_slots(c->nb);
   PT_TRY_LAUNCH(c, pt_launch_adjoint_groups(
                        c->adj_prec, c->bk.p, c->gslots.p, c->gslots.p + ns,
                        (uint32_t*)(c->gslots.p + 4 * ns), ns, c->tnode.p, c->gn.p, c->gn32.p,
                        c->xs.p, c->ys.p, c->zs.p, c->ms.p, c->es.p, c->gpp_off.p, c->gpp.p,
-                       c->gppm.p, c->gpc_off.p, c->gpc.p, c->gpcm.p, c->offset, v.wsx, v.wsy, v.wsz, v.gsx, v.gsy, v.gsz, v.gsm,
-                       c->lam_node.p, nn, c->stream));
+                       c->gppm.p, c->gpc_off.p, c->gpc.p, c->gpcm.p, c->offset, v.wsx, v.wsy, v.wsz, v.gs, c->lam_node.p, nn,
+                       c->stream));
   PT_TRY_LAUNCH(c, pt_launch_adjoint_down(n, c->bucket_of.p, c->bucket_node.p, c->nparent.p,
-                                          c->gn.p, c->lam_node.p, nn, c->xs.p,
-                                          c->ys.p, c->zs.p, c->ms.p, c->es.p, v.gsx, v.gsy,
-                                          v.gsz, v.gsm, c->stream));
-  PT_TRY_LAUNCH(c, pt_launch_scatter_add4(c->perm.p, n, v.gsx, v.gsy, v.gsz, v.gsm, gx, gy, gz,
-                                          gm, c->stream));
+                                          c->gn.p, c->lam_node.p, v.gs, c->perm.p, c->xs.p,
+                                          c->ys.p, c->zs.p, c->ms.p, c->es.p, gx, gy, gz, gm,
+                                          c->stream));
   return PT_OK;
 }
 
@@ -1423,12 +1423,12 @@ pt_status pt_force_vjp(pt_ctx* c, double theta, pt_force_mode mode, const double
     return fail(c, PT_ERR_UNSUPPORTED, "no adjoint of the periodic replicas");
   AdjViews v;
   if ((st = adj_views(c, &v))) return st;
-  // the sorted-order block (gsx..) doubles as the host staging area before
+  // the sorted-order block (gs) doubles as the host staging area before
   // and after the tree stages use it
-  if ((st = load3(c, w, where, v.wx, v.wy, v.wz, v.gsx))) return st;
+  if ((st = load3(c, w, where, v.wx, v.wy, v.wz, v.gs))) return st;
   if ((st = zero(c, v.lx, 3 * c->n)) || (st = zero(c, v.lm, c->n))) return st;
   if ((st = vjp_accumulate(c, mode, theta, v, v.wx, v.wy, v.wz, v.lx, v.ly, v.lz, v.lm))) return st;
-  if ((st = store3(c, v.lx, v.ly, v.lz, grad_x, where, v.gsx))) return st;
+  if ((st = store3(c, v.lx, v.ly, v.lz, grad_x, where, v.gs))) return st;
   if ((st = store1(c, v.lm, grad_m, where))) return st;
   PT_TRY_HIP(c, hipStreamSynchronize(c->stream));
   return PT_OK;
@@ -1494,8 +1494,8 @@ pt_status pt_leapfrog_adjoint(pt_ctx* c, const double* lam_x, const double* lam_
   PT_TRY_HIP(c, ensure(c->seg, (int64_t)std::min(every, std::max(steps, 1)) * 3 * n));
   double* final_state = c->ckpt.p + nseg * 6 * n;
   if ((st = save_state(c, final_state))) return st;
-  if ((st = load3(c, lam_x, where, v.lx, v.ly, v.lz, v.gsx))) return st;
-  if ((st = load3(c, lam_v, where, v.lvx, v.lvy, v.lvz, v.gsx))) return st;
+  if ((st = load3(c, lam_x, where, v.lx, v.ly, v.lz, v.gs))) return st;
+  if ((st = load3(c, lam_v, where, v.lvx, v.lvy, v.lvz, v.gs))) return st;
   if ((st = zero(c, v.lm, n))) return st;
   for (int64_t s = nseg - 1; s >= 0 && steps > 0; s--) {
     const int32_t k0 = (int32_t)(s * every);
@@ -1522,8 +1522,8 @@ pt_status pt_leapfrog_adjoint(pt_ctx* c, const double* lam_x, const double* lam_
         return st;
     }
   }
-  if ((st = store3(c, v.lx, v.ly, v.lz, grad_x, where, v.gsx))) return st;
-  if ((st = store3(c, v.lvx, v.lvy, v.lvz, grad_v, where, v.gsx))) return st;
+  if ((st = store3(c, v.lx, v.ly, v.lz, grad_x, where, v.gs))) return st;
+  if ((st = store3(c, v.lvx, v.lvy, v.lvz, grad_v, where, v.gs))) return st;
   if ((st = store1(c, v.lm, grad_m, where))) return st;
   if ((st = load_state(c, final_state, true))) return st;
   PT_TRY_HIP(c, hipStreamSynchronize(c->stream));

@@ -242,9 +242,8 @@ int pt_launch_group_traverse(bool fill, const TreeNode* nodes, const Bucket* bk,
 // Adjoint of the interactions over the group lists (precision 0: FP64;
 // otherwise FP32 pair arithmetic on group-centre-shifted coordinates with
 // FP64 sums).  lam_node holds pt_adjoint_node_scratch(nn) doubles, all zero
-// on entry (node cotangents field-major, then private copies of the hot
-// ones); g* accumulate.
-int pt_node_adjoint_fields();
+// on entry (a record of node cotangents per node, then private copies of the
+// hot ones'); gs: per particle a record x, y, z, mass, which accumulates.
 int64_t pt_adjoint_node_scratch(int64_t nn);
 int pt_launch_adjoint_groups(int precision, const Bucket* bk, const int32_t* gfirst,
                              const int32_t* gnb, const uint32_t* ngroups, int64_t ns,
@@ -254,13 +253,16 @@ int pt_launch_adjoint_groups(int precision, const Bucket* bk, const int32_t* gfi
                              const int64_t* pp_off, const int32_t* pp, const uint8_t* ppm,
                              const int64_t* pc_off, const int32_t* pc, const uint8_t* pcm,
                              const double off[3], const double* wx, const double* wy,
-                             const double* wz, double* gx, double* gy, double* gz, double* gm,
-                             double* lam_node, int64_t nn, hipStream_t s);
+                             const double* wz, double* gs, double* lam_node, int64_t nn,
+                             hipStream_t s);
+// The node cotangents pushed down to the particles, added with the particles'
+// own (gs, in sorted order) to the caller-order sums.
 int pt_launch_adjoint_down(int64_t n, const uint32_t* bucket_of, const int32_t* bucket_node,
                            const int32_t* parent, const GravNode* gn,
-                           const double* lam_node, int64_t nn, const double* x, const double* y,
-                           const double* z, const double* m, const double* e, double* gx,
-                           double* gy, double* gz, double* gm, hipStream_t s);
+                           const double* lam_node, const double* gs, const uint32_t* perm,
+                           const double* x, const double* y, const double* z, const double* m,
+                           const double* e, double* gx, double* gy, double* gz, double* gm,
+                           hipStream_t s);
 int pt_launch_direct_all(int64_t n, const double* x, const double* y, const double* z,
                          const double* m, const double* e, double* ax, double* ay, double* az,
                          double* pot, hipStream_t s);
@@ -273,9 +275,6 @@ int pt_launch_adjoint_w(int64_t n, double dt, const double* lx, const double* ly
                         double* wy, double* wz, hipStream_t s);
 int pt_launch_gather3(const uint32_t* perm, int64_t n, const double* a, const double* b,
                       const double* c, double* as, double* bs, double* cs, hipStream_t s);
-int pt_launch_scatter_add4(const uint32_t* perm, int64_t n, const double* a, const double* b,
-                           const double* c, const double* d, double* oa, double* ob, double* oc,
-                           double* od, hipStream_t s);
 int pt_launch_split3(int64_t n, const double* v, double* a, double* b, double* c, hipStream_t s);
 int pt_launch_join3(int64_t n, const double* a, const double* b, const double* c, double* v,
                     hipStream_t s);

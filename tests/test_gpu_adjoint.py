@@ -200,6 +200,34 @@ def test_tree_vjp_fp32c_against_fp64():
         d.set_adjoint_precision(7)
 
 
+@pytest.mark.parametrize("n,bucket", [(2, 1), (65, 1), (700, 40), (3000, 17), (3000, 130),
+                                      (9000, 12), (70000, 4)])
+def test_tree_vjp_group_edges(n, bucket):
+    """Groups of one target, of a bucket of several passes, and list shares
+    from eight waves per group down to one: with every node opened the tree
+    VJP is the direct one to FP64 rounding of its sums (1e-12), and at theta
+    0.7, with softened, monopole and far pairs, the identities hold in FP64 and
+    the FP32 form agrees to FP32 rounding."""
+    from paratreet_amd import _lib
+    from paratreet_amd.gravity import FORCE_DIRECT, FORCE_TREE
+    pos, _, m, e = _plummer(n, 29, 0.03)
+    w = np.random.default_rng(7).standard_normal(pos.shape)
+    d = _driver(bucket)
+    a = _tree_acc(d, pos, m, e, 0.7)
+    if n <= 9000:
+        g, gm = d.force_vjp(w, theta=1e-3, mode=FORCE_TREE)
+        gd, gmd = d.force_vjp(w, mode=FORCE_DIRECT)
+        assert np.linalg.norm(g - gd) <= 1e-12 * np.linalg.norm(gd)
+        assert np.linalg.norm(gm - gmd) <= 1e-12 * np.linalg.norm(gmd)
+    g, gm = d.force_vjp(w, theta=0.7, mode=FORCE_TREE)
+    assert np.abs(g.sum(0)).max() < 1e-10 * np.abs(g).sum()
+    assert abs(np.dot(m, gm) - np.sum(w * a)) < 1e-11 * np.sum(np.abs(w * a))
+    d.set_adjoint_precision(_lib.PT_FP32C)
+    g32, gm32 = d.force_vjp(w, theta=0.7, mode=FORCE_TREE)
+    assert np.linalg.norm(g32 - g) < 1e-5 * np.linalg.norm(g)
+    assert np.linalg.norm(gm32 - gm) < 1e-5 * np.linalg.norm(gm)
+
+
 # ---------------------------------------------------------------- trajectory
 
 STEPS, DT = 10, 1e-3
