@@ -92,7 +92,6 @@ struct pt_ctx {
   double gm = 0.0;  // GravityVisitor::monopole_gravity_factor
   DBuf<double> reptab;  // offsets of the periodic replicas
   DBuf<double> ewt;  // Ewald Fourier table (periodic build)
-  DBuf<int32_t> ewcount;
   DBuf<unsigned long long> cpart;  // per-block counter partials
   // bucket groups of the grouped fused kernel (pt_set_fused_grouping): 0 one
   // walk per bucket, 1 automatic, 2..64 the groups' particle cap
@@ -376,7 +375,6 @@ void pt_ctx_destroy(pt_ctx* c) {
   release(c->tstat); release(c->tinternal); release(c->tmeta);
   release(c->prec);
   release(c->ewt); release(c->reptab);
-  release(c->ewcount);
   release(c->hraw); release(c->hn); release(c->ho);
   release(c->bucket_node); release(c->nd); release(c->ord_h); release(c->ord_b);
   release(c->tnode); release(c->gn); release(c->gn32); release(c->bk); release(c->cpart);
@@ -1071,18 +1069,17 @@ static pt_status gravity_fused(pt_ctx* c, double theta, const double offset[3],
     if (c->cfg.periodic) {
       // LeafEwaldFn after the replicas (examples/Gravity.C:47-50)
       Timer t(c, PT_T_FORCE);
-      PT_TRY_HIP(c, ensure(c->ewt, 5 * pt_ewald_table_entries()));
-      PT_TRY_HIP(c, ensure(c->ewcount, 1));
+      PT_TRY_HIP(c, ensure(c->ewt, 2 * pt_ewald_table_entries()));
       if (hexa)
         PT_TRY_LAUNCH(c, pt_launch_ewald_hexa(c->n, c->xs.p, c->ys.p, c->zs.p, c->nd.p, c->nn,
                                               c->hn.p, c->cfg.period[0], c->cfg.n_replicas,
-                                              c->ewt.p, c->ewcount.p, c->axs.p, c->ays.p,
-                                              c->azs.p, c->pots.p, c->stream));
+                                              c->ewt.p, c->axs.p, c->ays.p, c->azs.p,
+                                              c->pots.p, c->stream));
       else
         PT_TRY_LAUNCH(c, pt_launch_ewald(c->n, c->xs.p, c->ys.p, c->zs.p, c->nd.p, c->nn,
                                          c->cfg.period[0], c->cfg.n_replicas, c->ewt.p,
-                                         c->ewcount.p, c->axs.p, c->ays.p, c->azs.p,
-                                         c->pots.p, c->stream));
+                                         c->axs.p, c->ays.p, c->azs.p, c->pots.p,
+                                         c->stream));
     }
     // the last replica's counters, the unsort to caller order and the one
     // read-back; a rerun (stack overflow, rare) repeats every replica

@@ -166,19 +166,19 @@ int pt_launch_gravity(int precision, bool big_stack, const Bucket* bk, const int
 
 // Ewald lattice correction of the periodic build (quadrupole form) from the
 // root's moments (node 0 of nd), added to the sorted results.  table holds
-// 4 * pt_ewald_table_entries() doubles, count one int.
+// pt_ewald_table_entries() doubles.
 int64_t pt_ewald_table_entries();
 int pt_launch_ewald(int64_t n, const double* x, const double* y, const double* z,
                     const double* nd, int64_t nn, double L, int n_replicas, double* table,
-                    int32_t* count, double* ax, double* ay, double* az, double* pot,
+                    double* ax, double* ay, double* az, double* pot,
                     hipStream_t s);
 
 // LeafEwaldFn of the HEXADECAPOLE build: the root's moments to fourth order
 // (nd for mass and centre, hn[0] for the reduced moments); table holds
-// 5 * pt_ewald_table_entries() doubles.
+// 2 * pt_ewald_table_entries() doubles.
 int pt_launch_ewald_hexa(int64_t n, const double* x, const double* y, const double* z,
                          const double* nd, int64_t nn, const HexNode* hn, double L,
-                         int n_replicas, double* table, int32_t* count, double* ax, double* ay,
+                         int n_replicas, double* table, double* ax, double* ay,
                          double* az, double* pot, hipStream_t s);
 
 int pt_launch_gather(const uint32_t* perm, int64_t n, const ParticleRec* rec, double* xs,

@@ -193,7 +193,7 @@ fill_u64_kernel(unsigned long long* __restrict__ p, int64_t n, unsigned long lon
 // removes the bare 1/r part the tree summed; a two-term series replaces the
 // closed forms below r^2 = 1.2e-3 L^2) and the Fourier terms of the integer
 // vectors 0 < |h| <= 2.8, with alpha = 2 / L, L = dxPeriod.  Same
-// operations, in the same order, as the oracle's restatement.
+// operations per term as the oracle's restatement.
 // ---------------------------------------------------------------------------
 
 constexpr double kEwAlphaFac = 2.0;  // alpha = 2 / L
@@ -201,48 +201,134 @@ constexpr double kEwCut = 2.6;       // real-space radius, in L
 constexpr double kEwHCut = 2.8;      // Fourier radius, in units of 2 pi / L
 constexpr double kPi = 3.14159265358979323846;
 
-// One thread: the Fourier table {2 pi h / L, C(h)} in the lattice order of the
-// loops (h_x outermost); C(h) = -(e^{-k4 h^2}/(pi h^2 L)) (M - (2 pi/L)^2 h.q.h/2)
+// One wave, a vector per lane: the Fourier coefficients C(h) in lattice order
+// (h_x outermost, the whole cube; those beyond the radius are not written):
+// C(h) = -(e^{-k4 h^2}/(pi h^2 L)) (M - (2 pi/L)^2 h.q.h/2)
 // (the sine coefficients vanish at quadrupole order).
-__global__ void ewald_table_kernel(const double* __restrict__ nd, int64_t nn, double L,
-                                   double* __restrict__ table, int32_t* __restrict__ count) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+__global__ void __launch_bounds__(PT_WAVE)
+ewald_table_kernel(const double* __restrict__ nd, int64_t nn, double L,
+                   double* __restrict__ table) {
   const double mass = nd[PT_ND_MASS];
   double q[6];
   for (int k = 0; k < 6; k++) q[k] = nd[PT_ND_Q(k)];
   const double alpha = kEwAlphaFac / L, alpha2 = alpha * alpha;
   const double k4 = kPi * kPi / (alpha2 * L * L);
-  const int hr = (int)ceil(kEwHCut);
-  int nh = 0;
-  for (int hx = -hr; hx <= hr; hx++)
-    for (int hy = -hr; hy <= hr; hy++)
-      for (int hz = -hr; hz <= hr; hz++) {
-        const int h2 = hx * hx + hy * hy + hz * hz;
-        if (h2 == 0 || h2 > kEwHCut * kEwHCut) continue;
-        const double g0 = exp(-k4 * h2) / (kPi * h2 * L);
-        const double w = 2.0 * kPi / L;
-        const double hqh = 0.5 * (hx * (q[0] * hx + q[1] * hy + q[2] * hz) +
-                                  hy * (q[1] * hx + q[3] * hy + q[4] * hz) +
-                                  hz * (q[2] * hx + q[4] * hy + q[5] * hz));
-        table[4 * nh + 0] = w * hx;
-        table[4 * nh + 1] = w * hy;
-        table[4 * nh + 2] = w * hz;
-        table[4 * nh + 3] = -(g0 * mass - w * w * g0 * hqh);
-        nh++;
-      }
-  *count = nh;
+  const int hr = (int)ceil(kEwHCut), side = 2 * hr + 1;
+  for (int c0 = 0; c0 < side * side * side; c0 += PT_WAVE) {
+    const int c = c0 + (int)threadIdx.x;
+    const int hx = c / (side * side) - hr, hy = c / side % side - hr, hz = c % side - hr;
+    const int h2 = hx * hx + hy * hy + hz * hz;
+    const bool keep = c < side * side * side && h2 != 0 && h2 <= kEwHCut * kEwHCut;
+    if (keep) {
+      const double g0 = exp(-k4 * h2) / (kPi * h2 * L);
+      const double w = 2.0 * kPi / L;
+      const double hqh = 0.5 * (hx * (q[0] * hx + q[1] * hy + q[2] * hz) +
+                                hy * (q[1] * hx + q[3] * hy + q[4] * hz) +
+                                hz * (q[2] * hx + q[4] * hy + q[5] * hz));
+      table[c] = -(g0 * mass - w * w * g0 * hqh);
+    }
+  }
 }
 
-// One thread per particle (sorted order); adds to the accelerations and
-// potentials the replica traversals left.
-__global__ void __launch_bounds__(256)
+// Work-groups of 64 particles (sorted order, one per lane), whose waves share
+// the lattice: wave w takes every kEwWaves-th vector of both sums, and the
+// partial sums are added in wave order to the accelerations and potentials the
+// replica traversals left.  Bound by the FP64 arithmetic of exp and erfc, about
+// a hundred of each per particle (50k particles: 107 -> 93 us with the Fourier
+// phases as products, the table 17 -> 5 us).  Against extended precision the
+// partial sums halve the rounding of the lattice sum (2.4e-16 of it for
+// 4.7e-16), and the products keep that of the Fourier sum (2.5e-16 for 3.1e-16).
+constexpr int kEwWaves = 8;
+constexpr int kEwThreads = kEwWaves * PT_WAVE;
+
+struct EwaldSum {
+  double part[kEwWaves][4][PT_WAVE];
+};
+
+// The sums over the work-group's waves, into the particle's values.
+__device__ __forceinline__ void ewald_add(EwaldSum& sum, int wave, int lane, int64_t i, int64_t n,
+                                          double fx, double fy, double fz, double p,
+                                          double* __restrict__ ax, double* __restrict__ ay,
+                                          double* __restrict__ az, double* __restrict__ pot) {
+  sum.part[wave][0][lane] = fx;
+  sum.part[wave][1][lane] = fy;
+  sum.part[wave][2][lane] = fz;
+  sum.part[wave][3][lane] = p;
+  __syncthreads();
+  if (wave < 4 && i < n) {
+    double v = 0.0;
+    for (int w = 0; w < kEwWaves; w++) v += sum.part[w][wave][lane];
+    (wave == 0 ? ax : (wave == 1 ? ay : (wave == 2 ? az : pot)))[i] += v;
+  }
+}
+
+// The Fourier terms of a wave, hy = wave - 3 (the last wave has none): h and
+// -h give equal terms, so the half space hx > 0, or hx = 0 and (hy, hz) > 0 in
+// turn, counts twice.  The phases are products of powers of three unit
+// complex numbers, three sincos in all where a term each took 160; with HEXA
+// the table has sine coefficients too.
+template <bool HEXA>
+__device__ __forceinline__ void ewald_fourier(const double* __restrict__ table, double L, int wave,
+                                              double dx, double dy, double dz, double& fx,
+                                              double& fy, double& fz, double& p) {
+  constexpr int hr = 3, side = 2 * hr + 1;
+  static_assert(kEwHCut > hr - 1 && kEwHCut <= hr && side <= kEwWaves, "lattice of the table");
+  const int hy = wave - hr;
+  if (hy > hr) return;
+  const double w = 2.0 * kPi / L;
+  double ycos, ysin, xcos, xsin, c1, s1;
+  sincos(w * hy * dy, &ysin, &ycos);
+  sincos(w * dx, &xsin, &xcos);
+  sincos(w * dz, &s1, &c1);
+  const double c2 = c1 * c1 - s1 * s1, s2 = 2.0 * c1 * s1;
+  const double zc[hr + 1] = {1.0, c1, c2, c2 * c1 - s2 * s1};
+  const double zs[hr + 1] = {0.0, s1, s2, s2 * c1 + c2 * s1};
+  double gx = 0.0, gy = 0.0, gz = 0.0, gp = 0.0;
+  double ac = ycos, as = ysin;  // e^{i w (hx dx + hy dy)}
+#pragma unroll
+  for (int hx = 0; hx <= hr; hx++) {
+#pragma unroll
+    for (int hz = -hr; hz <= hr; hz++) {
+      const bool half = hx > 0 || hy > 0 || (hy == 0 && hz > 0);
+      if (half && hx * hx + hy * hy + hz * hz <= kEwHCut * kEwHCut) {
+        const int az = hz < 0 ? -hz : hz;
+        const double bc = zc[az], bs = hz < 0 ? -zs[az] : zs[az];
+        const double c = ac * bc - as * bs, sn = as * bc + ac * bs;
+        const int e = ((hx + hr) * side + hy + hr) * side + hz + hr;
+        double f;
+        if (HEXA) {
+          const double cc = table[2 * e], cs = table[2 * e + 1];
+          gp += cc * c + cs * sn;
+          f = cc * sn - cs * c;
+        } else {
+          gp += table[e] * c;
+          f = table[e] * sn;
+        }
+        gx += hx * f;
+        gy += hy * f;
+        gz += hz * f;
+      }
+    }
+    const double nc = ac * xcos - as * xsin;
+    as = as * xcos + ac * xsin;
+    ac = nc;
+  }
+  p += 2.0 * gp;
+  fx += 2.0 * w * gx;
+  fy += 2.0 * w * gy;
+  fz += 2.0 * w * gz;
+}
+
+__global__ void __launch_bounds__(kEwThreads)
 ewald_kernel(int64_t n, const double* __restrict__ x, const double* __restrict__ y,
              const double* __restrict__ z, const double* __restrict__ nd, int64_t nn, double L,
-             int n_replicas, const double* __restrict__ table, const int32_t* __restrict__ count,
-             double* __restrict__ ax, double* __restrict__ ay, double* __restrict__ az,
+             int n_replicas, const double* __restrict__ table, double* __restrict__ ax, double* __restrict__ ay, double* __restrict__ az,
              double* __restrict__ pot) {
-  const int64_t i = blockIdx.x * 256ll + threadIdx.x;
-  if (i >= n) return;
+  __shared__ EwaldSum sum;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PT_WAVE);
+  const int lane = threadIdx.x & (PT_WAVE - 1);
+  const int64_t i = blockIdx.x * (int64_t)PT_WAVE + lane;
+  const int64_t il = i < n ? i : n - 1;  // lanes past the end repeat the last particle
   const double mass = nd[PT_ND_MASS];
   const double cm[3] = {nd[PT_ND_CM], nd[PT_ND_CM + 1], nd[PT_ND_CM + 2]};
   double q[6];
@@ -254,64 +340,48 @@ ewald_kernel(int64_t n, const double* __restrict__ x, const double* __restrict__
   int nrep = (int)ceil(kEwCut);
   if (n_replicas > nrep) nrep = n_replicas;
   const double cut2 = kEwCut * kEwCut * L * L, inner2 = 1.2e-3 * L * L;
-  double p = mass * k1, fx = 0.0, fy = 0.0, fz = 0.0;
-  const double dx = x[i] - cm[0], dy = y[i] - cm[1], dz = z[i] - cm[2];
-  for (int ix = -nrep; ix <= nrep; ix++) {
-    const bool hole_x = ix >= -n_replicas && ix <= n_replicas;
-    const double rx = dx + ix * L;
-    for (int iy = -nrep; iy <= nrep; iy++) {
-      const bool hole_xy = hole_x && iy >= -n_replicas && iy <= n_replicas;
-      const double ry = dy + iy * L;
-      for (int iz = -nrep; iz <= nrep; iz++) {
-        const bool hole = hole_xy && iz >= -n_replicas && iz <= n_replicas;
-        const double rz = dz + iz * L;
-        const double r2 = rx * rx + ry * ry + rz * rz;
-        if (r2 > cut2 && !hole) continue;
-        double g0, g1, g2, g3;
-        if (r2 < inner2) {
-          const double s2 = r2 * alpha2;
-          double an = ka;
-          g0 = an * ((1.0 / 3.0) * s2 - 1.0);
-          an *= 2.0 * alpha2;
-          g1 = an * ((1.0 / 5.0) * s2 - (1.0 / 3.0));
-          an *= 2.0 * alpha2;
-          g2 = an * ((1.0 / 7.0) * s2 - (1.0 / 5.0));
-          an *= 2.0 * alpha2;
-          g3 = an * ((1.0 / 9.0) * s2 - (1.0 / 7.0));
-        } else {
-          const double r = sqrt(r2);
-          const double ir2 = 1.0 / r2;
-          const double a = exp(-r2 * alpha2) * ka * ir2;
-          g0 = (hole ? -erf(alpha * r) : erfc(alpha * r)) / r;
-          g1 = g0 * ir2 + a;
-          g2 = 3.0 * g1 * ir2 + 2.0 * alpha2 * a;
-          g3 = 5.0 * g2 * ir2 + 4.0 * alpha2 * alpha2 * a;
-        }
-        const double qx = q[0] * rx + q[1] * ry + q[2] * rz;
-        const double qy = q[1] * rx + q[3] * ry + q[4] * rz;
-        const double qz = q[2] * rx + q[4] * ry + q[5] * rz;
-        const double qrr = 0.5 * (qx * rx + qy * ry + qz * rz);
-        const double qta = g1 * mass - g2 * q2 + g3 * qrr;
-        p -= g0 * mass - g1 * q2 + g2 * qrr;
-        fx += g2 * qx - rx * qta;
-        fy += g2 * qy - ry * qta;
-        fz += g2 * qz - rz * qta;
-      }
+  double p = wave == 0 ? mass * k1 : 0.0, fx = 0.0, fy = 0.0, fz = 0.0;
+  const double dx = x[il] - cm[0], dy = y[il] - cm[1], dz = z[il] - cm[2];
+  const int side = 2 * nrep + 1;
+  for (int c = wave; c < side * side * side; c += kEwWaves) {
+    const int ix = c / (side * side) - nrep, iy = c / side % side - nrep, iz = c % side - nrep;
+    const bool hole = ix >= -n_replicas && ix <= n_replicas && iy >= -n_replicas &&
+                      iy <= n_replicas && iz >= -n_replicas && iz <= n_replicas;
+    const double rx = dx + ix * L, ry = dy + iy * L, rz = dz + iz * L;
+    const double r2 = rx * rx + ry * ry + rz * rz;
+    if (r2 > cut2 && !hole) continue;
+    double g0, g1, g2, g3;
+    if (r2 < inner2) {
+      const double s2 = r2 * alpha2;
+      double an = ka;
+      g0 = an * ((1.0 / 3.0) * s2 - 1.0);
+      an *= 2.0 * alpha2;
+      g1 = an * ((1.0 / 5.0) * s2 - (1.0 / 3.0));
+      an *= 2.0 * alpha2;
+      g2 = an * ((1.0 / 7.0) * s2 - (1.0 / 5.0));
+      an *= 2.0 * alpha2;
+      g3 = an * ((1.0 / 9.0) * s2 - (1.0 / 7.0));
+    } else {
+      const double r = sqrt(r2);
+      const double ir2 = 1.0 / r2;
+      const double a = exp(-r2 * alpha2) * ka * ir2;
+      g0 = (hole ? -erf(alpha * r) : erfc(alpha * r)) / r;
+      g1 = g0 * ir2 + a;
+      g2 = 3.0 * g1 * ir2 + 2.0 * alpha2 * a;
+      g3 = 5.0 * g2 * ir2 + 4.0 * alpha2 * alpha2 * a;
     }
+    const double qx = q[0] * rx + q[1] * ry + q[2] * rz;
+    const double qy = q[1] * rx + q[3] * ry + q[4] * rz;
+    const double qz = q[2] * rx + q[4] * ry + q[5] * rz;
+    const double qrr = 0.5 * (qx * rx + qy * ry + qz * rz);
+    const double qta = g1 * mass - g2 * q2 + g3 * qrr;
+    p -= g0 * mass - g1 * q2 + g2 * qrr;
+    fx += g2 * qx - rx * qta;
+    fy += g2 * qy - ry * qta;
+    fz += g2 * qz - rz * qta;
   }
-  const int nh = *count;
-  for (int k = 0; k < nh; k++) {
-    const double hd = table[4 * k] * dx + table[4 * k + 1] * dy + table[4 * k + 2] * dz;
-    const double c = cos(hd), sn = sin(hd), cf = table[4 * k + 3];
-    p += cf * c;
-    fx += table[4 * k] * (cf * sn);
-    fy += table[4 * k + 1] * (cf * sn);
-    fz += table[4 * k + 2] * (cf * sn);
-  }
-  ax[i] += fx;
-  ay[i] += fy;
-  az[i] += fz;
-  pot[i] += p;
+  ewald_fourier<false>(table, L, wave, dx, dy, dz, fx, fy, fz, p);
+  ewald_add(sum, wave, lane, i, n, fx, fy, fz, p, ax, ay, az, pot);
 }
 
 // ---------------------------------------------------------------------------
@@ -323,7 +393,7 @@ ewald_kernel(int64_t n, const double* __restrict__ x, const double* __restrict__
 // the quadrupole: g0..g5 in real space, and in Fourier space a cosine
 // coefficient -g (m - w^2 M2[h^2]/2 + w^4 M4[h^4]/24) and a sine coefficient
 // g w^3 M3[h^3]/6 per vector (w = 2 pi / L, g = e^{-k4 h^2}/(pi h^2 L)).
-// Same operations, in the same order, as the oracle's restatement.
+// Same operations per term as the oracle's restatement.
 // ---------------------------------------------------------------------------
 
 struct Momc {
@@ -376,52 +446,48 @@ __device__ __forceinline__ void momc_contract(const Momc& M, double x, double y,
           M.xzzz * xzz + M.yyyz * yyy + M.yyzz * yyz + M.yzzz * yzz + M.zzzz * zzz;
 }
 
-// One thread: the Fourier table {2 pi h / L, C(h), S(h)} in the lattice order
-// of the loops (h_x outermost).
-__global__ void ewald_hexa_table_kernel(const double* __restrict__ nd, int64_t nn,
-                                        const HexNode* __restrict__ hn, double L,
-                                        double* __restrict__ table, int32_t* __restrict__ count) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+// One wave, a vector per lane: the Fourier coefficients {C(h), S(h)} in lattice
+// order.
+__global__ void __launch_bounds__(PT_WAVE)
+ewald_hexa_table_kernel(const double* __restrict__ nd, int64_t nn,
+                        const HexNode* __restrict__ hn, double L, double* __restrict__ table) {
   const double mass = nd[PT_ND_MASS];
   Momc M;
   momc_from_reduced(mass, hn[0].h, M);
   const double alpha = kEwAlphaFac / L, alpha2 = alpha * alpha;
   const double k4 = kPi * kPi / (alpha2 * L * L);
   const double w = 2.0 * kPi / L;
-  const int hr = (int)ceil(kEwHCut);
-  int nh = 0;
-  for (int hx = -hr; hx <= hr; hx++)
-    for (int hy = -hr; hy <= hr; hy++)
-      for (int hz = -hr; hz <= hr; hz++) {
-        const int h2 = hx * hx + hy * hy + hz * hz;
-        if (h2 == 0 || h2 > kEwHCut * kEwHCut) continue;
-        const double g = exp(-k4 * h2) / (kPi * h2 * L);
-        double q2[3], q3[3], q4[3];
-        momc_contract(M, hx, hy, hz, q2, q3, q4);
-        const double m2 = 0.5 * (q2[0] * hx + q2[1] * hy + q2[2] * hz);
-        const double m3 = (1.0 / 3.0) * (q3[0] * hx + q3[1] * hy + q3[2] * hz);
-        const double m4 = 0.25 * (q4[0] * hx + q4[1] * hy + q4[2] * hz);
-        table[5 * nh + 0] = w * hx;
-        table[5 * nh + 1] = w * hy;
-        table[5 * nh + 2] = w * hz;
-        table[5 * nh + 3] = -g * (mass - w * w * m2 + w * w * w * w * m4);
-        table[5 * nh + 4] = g * w * w * w * m3;
-        nh++;
-      }
-  *count = nh;
+  const int hr = (int)ceil(kEwHCut), side = 2 * hr + 1;
+  for (int c0 = 0; c0 < side * side * side; c0 += PT_WAVE) {
+    const int c = c0 + (int)threadIdx.x;
+    const int hx = c / (side * side) - hr, hy = c / side % side - hr, hz = c % side - hr;
+    const int h2 = hx * hx + hy * hy + hz * hz;
+    const bool keep = c < side * side * side && h2 != 0 && h2 <= kEwHCut * kEwHCut;
+    if (keep) {
+      const double g = exp(-k4 * h2) / (kPi * h2 * L);
+      double q2[3], q3[3], q4[3];
+      momc_contract(M, hx, hy, hz, q2, q3, q4);
+      const double m2 = 0.5 * (q2[0] * hx + q2[1] * hy + q2[2] * hz);
+      const double m3 = (1.0 / 3.0) * (q3[0] * hx + q3[1] * hy + q3[2] * hz);
+      const double m4 = 0.25 * (q4[0] * hx + q4[1] * hy + q4[2] * hz);
+      table[2 * c] = -g * (mass - w * w * m2 + w * w * w * w * m4);
+      table[2 * c + 1] = g * w * w * w * m3;
+    }
+  }
 }
 
-// One thread per particle (sorted order); adds to the accelerations and
-// potentials the replica traversals left.
-__global__ void __launch_bounds__(256)
+// ewald_kernel's split of particles and lattice.
+__global__ void __launch_bounds__(kEwThreads)
 ewald_hexa_kernel(int64_t n, const double* __restrict__ x, const double* __restrict__ y,
                   const double* __restrict__ z, const double* __restrict__ nd, int64_t nn,
                   const HexNode* __restrict__ hn, double L, int n_replicas,
-                  const double* __restrict__ table, const int32_t* __restrict__ count,
-                  double* __restrict__ ax, double* __restrict__ ay, double* __restrict__ az,
+                  const double* __restrict__ table, double* __restrict__ ax, double* __restrict__ ay, double* __restrict__ az,
                   double* __restrict__ pot) {
-  const int64_t i = blockIdx.x * 256ll + threadIdx.x;
-  if (i >= n) return;
+  __shared__ EwaldSum sum;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PT_WAVE);
+  const int lane = threadIdx.x & (PT_WAVE - 1);
+  const int64_t i = blockIdx.x * (int64_t)PT_WAVE + lane;
+  const int64_t il = i < n ? i : n - 1;  // lanes past the end repeat the last particle
   const double mass = nd[PT_ND_MASS];
   const double cm[3] = {nd[PT_ND_CM], nd[PT_ND_CM + 1], nd[PT_ND_CM + 2]};
   Momc M;
@@ -439,81 +505,64 @@ ewald_hexa_kernel(int64_t n, const double* __restrict__ x, const double* __restr
   int nrep = (int)ceil(kEwCut);
   if (n_replicas > nrep) nrep = n_replicas;
   const double cut2 = kEwCut * kEwCut * L * L, inner2 = 1.2e-3 * L * L;
-  double p = mass * k1, fx = 0.0, fy = 0.0, fz = 0.0;
-  const double dx = x[i] - cm[0], dy = y[i] - cm[1], dz = z[i] - cm[2];
-  for (int ix = -nrep; ix <= nrep; ix++) {
-    const bool hole_x = ix >= -n_replicas && ix <= n_replicas;
-    const double rx = dx + ix * L;
-    for (int iy = -nrep; iy <= nrep; iy++) {
-      const bool hole_xy = hole_x && iy >= -n_replicas && iy <= n_replicas;
-      const double ry = dy + iy * L;
-      for (int iz = -nrep; iz <= nrep; iz++) {
-        const bool hole = hole_xy && iz >= -n_replicas && iz <= n_replicas;
-        const double rz = dz + iz * L;
-        const double r2 = rx * rx + ry * ry + rz * rz;
-        if (r2 > cut2 && !hole) continue;
-        double g0, g1, g2, g3, g4, g5;
-        if (r2 < inner2) {
-          const double s2 = r2 * alpha2;
-          double an = ka;
-          g0 = an * ((1.0 / 3.0) * s2 - 1.0);
-          an *= 2.0 * alpha2;
-          g1 = an * ((1.0 / 5.0) * s2 - (1.0 / 3.0));
-          an *= 2.0 * alpha2;
-          g2 = an * ((1.0 / 7.0) * s2 - (1.0 / 5.0));
-          an *= 2.0 * alpha2;
-          g3 = an * ((1.0 / 9.0) * s2 - (1.0 / 7.0));
-          an *= 2.0 * alpha2;
-          g4 = an * ((1.0 / 11.0) * s2 - (1.0 / 9.0));
-          an *= 2.0 * alpha2;
-          g5 = an * ((1.0 / 13.0) * s2 - (1.0 / 11.0));
-        } else {
-          const double r = sqrt(r2);
-          const double ir2 = 1.0 / r2;
-          const double a = exp(-r2 * alpha2) * ka * ir2;
-          g0 = (hole ? -erf(alpha * r) : erfc(alpha * r)) / r;
-          g1 = g0 * ir2 + a;
-          double an = 2.0 * alpha2;
-          g2 = 3.0 * g1 * ir2 + an * a;
-          an *= 2.0 * alpha2;
-          g3 = 5.0 * g2 * ir2 + an * a;
-          an *= 2.0 * alpha2;
-          g4 = 7.0 * g3 * ir2 + an * a;
-          an *= 2.0 * alpha2;
-          g5 = 9.0 * g4 * ir2 + an * a;
-        }
-        double q2[3], q3[3], q4[3];
-        momc_contract(M, rx, ry, rz, q2, q3, q4);
-        const double Q4vx = Q4xx * rx + Q4xy * ry + Q4xz * rz;
-        const double Q4vy = Q4xy * rx + Q4yy * ry + Q4yz * rz;
-        const double Q4vz = Q4xz * rx + Q4yz * ry + Q4zz * rz;
-        const double Q2mir = 0.5 * (q2[0] * rx + q2[1] * ry + q2[2] * rz) -
-                             (Q3x * rx + Q3y * ry + Q3z * rz) + Q4;
-        const double Q3mir = (1.0 / 3.0) * (q3[0] * rx + q3[1] * ry + q3[2] * rz) -
-                             0.5 * (Q4vx * rx + Q4vy * ry + Q4vz * rz);
-        const double Q4mir = 0.25 * (q4[0] * rx + q4[1] * ry + q4[2] * rz);
-        const double Qta = g1 * mass - g2 * Q2 + g3 * Q2mir + g4 * Q3mir + g5 * Q4mir;
-        p -= g0 * mass - g1 * Q2 + g2 * Q2mir + g3 * Q3mir + g4 * Q4mir;
-        fx += g2 * (q2[0] - Q3x) + g3 * (q3[0] - Q4vx) + g4 * q4[0] - rx * Qta;
-        fy += g2 * (q2[1] - Q3y) + g3 * (q3[1] - Q4vy) + g4 * q4[1] - ry * Qta;
-        fz += g2 * (q2[2] - Q3z) + g3 * (q3[2] - Q4vz) + g4 * q4[2] - rz * Qta;
-      }
+  double p = wave == 0 ? mass * k1 : 0.0, fx = 0.0, fy = 0.0, fz = 0.0;
+  const double dx = x[il] - cm[0], dy = y[il] - cm[1], dz = z[il] - cm[2];
+  const int side = 2 * nrep + 1;
+  for (int c = wave; c < side * side * side; c += kEwWaves) {
+    const int ix = c / (side * side) - nrep, iy = c / side % side - nrep, iz = c % side - nrep;
+    const bool hole = ix >= -n_replicas && ix <= n_replicas && iy >= -n_replicas &&
+                      iy <= n_replicas && iz >= -n_replicas && iz <= n_replicas;
+    const double rx = dx + ix * L, ry = dy + iy * L, rz = dz + iz * L;
+    const double r2 = rx * rx + ry * ry + rz * rz;
+    if (r2 > cut2 && !hole) continue;
+    double g0, g1, g2, g3, g4, g5;
+    if (r2 < inner2) {
+      const double s2 = r2 * alpha2;
+      double an = ka;
+      g0 = an * ((1.0 / 3.0) * s2 - 1.0);
+      an *= 2.0 * alpha2;
+      g1 = an * ((1.0 / 5.0) * s2 - (1.0 / 3.0));
+      an *= 2.0 * alpha2;
+      g2 = an * ((1.0 / 7.0) * s2 - (1.0 / 5.0));
+      an *= 2.0 * alpha2;
+      g3 = an * ((1.0 / 9.0) * s2 - (1.0 / 7.0));
+      an *= 2.0 * alpha2;
+      g4 = an * ((1.0 / 11.0) * s2 - (1.0 / 9.0));
+      an *= 2.0 * alpha2;
+      g5 = an * ((1.0 / 13.0) * s2 - (1.0 / 11.0));
+    } else {
+      const double r = sqrt(r2);
+      const double ir2 = 1.0 / r2;
+      const double a = exp(-r2 * alpha2) * ka * ir2;
+      g0 = (hole ? -erf(alpha * r) : erfc(alpha * r)) / r;
+      g1 = g0 * ir2 + a;
+      double an = 2.0 * alpha2;
+      g2 = 3.0 * g1 * ir2 + an * a;
+      an *= 2.0 * alpha2;
+      g3 = 5.0 * g2 * ir2 + an * a;
+      an *= 2.0 * alpha2;
+      g4 = 7.0 * g3 * ir2 + an * a;
+      an *= 2.0 * alpha2;
+      g5 = 9.0 * g4 * ir2 + an * a;
     }
+    double q2[3], q3[3], q4[3];
+    momc_contract(M, rx, ry, rz, q2, q3, q4);
+    const double Q4vx = Q4xx * rx + Q4xy * ry + Q4xz * rz;
+    const double Q4vy = Q4xy * rx + Q4yy * ry + Q4yz * rz;
+    const double Q4vz = Q4xz * rx + Q4yz * ry + Q4zz * rz;
+    const double Q2mir = 0.5 * (q2[0] * rx + q2[1] * ry + q2[2] * rz) -
+                         (Q3x * rx + Q3y * ry + Q3z * rz) + Q4;
+    const double Q3mir = (1.0 / 3.0) * (q3[0] * rx + q3[1] * ry + q3[2] * rz) -
+                         0.5 * (Q4vx * rx + Q4vy * ry + Q4vz * rz);
+    const double Q4mir = 0.25 * (q4[0] * rx + q4[1] * ry + q4[2] * rz);
+    const double Qta = g1 * mass - g2 * Q2 + g3 * Q2mir + g4 * Q3mir + g5 * Q4mir;
+    p -= g0 * mass - g1 * Q2 + g2 * Q2mir + g3 * Q3mir + g4 * Q4mir;
+    fx += g2 * (q2[0] - Q3x) + g3 * (q3[0] - Q4vx) + g4 * q4[0] - rx * Qta;
+    fy += g2 * (q2[1] - Q3y) + g3 * (q3[1] - Q4vy) + g4 * q4[1] - ry * Qta;
+    fz += g2 * (q2[2] - Q3z) + g3 * (q3[2] - Q4vz) + g4 * q4[2] - rz * Qta;
   }
-  const int nh = *count;
-  for (int k = 0; k < nh; k++) {
-    const double hd = table[5 * k] * dx + table[5 * k + 1] * dy + table[5 * k + 2] * dz;
-    const double c = cos(hd), sn = sin(hd), cc = table[5 * k + 3], cs = table[5 * k + 4];
-    p += cc * c + cs * sn;
-    const double f = cc * sn - cs * c;
-    fx += table[5 * k] * f;
-    fy += table[5 * k + 1] * f;
-    fz += table[5 * k + 2] * f;
-  }
-  ax[i] += fx;
-  ay[i] += fy;
-  az[i] += fz;
-  pot[i] += p;
+  ewald_fourier<true>(table, L, wave, dx, dy, dz, fx, fy, fz, p);
+  ewald_add(sum, wave, lane, i, n, fx, fy, fz, p, ax, ay, az, pot);
 }
 
 }  // namespace
@@ -574,30 +623,29 @@ int pt_launch_fill_u64(unsigned long long* p, int64_t n, unsigned long long v, h
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-// Fourier table entries the Ewald kernels can hold: the integer vectors of a
-// 7^3 cube (the cut 2.8 keeps 80 of them); doubles per entry: 4 in the
-// quadrupole form, 5 in the HEXADECAPOLE form.
+// Fourier table entries of the Ewald kernels: the integer vectors of a 7^3 cube
+// (the cut 2.8 keeps 80 of them); doubles per entry: 1 in the quadrupole form,
+// 2 in the HEXADECAPOLE form.
 int64_t pt_ewald_table_entries() { return 343; }
 
 int pt_launch_ewald(int64_t n, const double* x, const double* y, const double* z,
                     const double* nd, int64_t nn, double L, int n_replicas, double* table,
-                    int32_t* count, double* ax, double* ay, double* az, double* pot,
+                    double* ax, double* ay, double* az, double* pot,
                     hipStream_t s) {
   if (n <= 0) return 0;
-  ewald_table_kernel<<<1, 64, 0, s>>>(nd, nn, L, table, count);
-  ewald_kernel<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(n, x, y, z, nd, nn, L, n_replicas,
-                                                           table, count, ax, ay, az, pot);
+  ewald_table_kernel<<<1, PT_WAVE, 0, s>>>(nd, nn, L, table);
+  ewald_kernel<<<(unsigned)((n + PT_WAVE - 1) / PT_WAVE), kEwThreads, 0, s>>>(
+      n, x, y, z, nd, nn, L, n_replicas, table, ax, ay, az, pot);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
 int pt_launch_ewald_hexa(int64_t n, const double* x, const double* y, const double* z,
                          const double* nd, int64_t nn, const HexNode* hn, double L,
-                         int n_replicas, double* table, int32_t* count, double* ax, double* ay,
+                         int n_replicas, double* table, double* ax, double* ay,
                          double* az, double* pot, hipStream_t s) {
   if (n <= 0) return 0;
-  ewald_hexa_table_kernel<<<1, 64, 0, s>>>(nd, nn, hn, L, table, count);
-  ewald_hexa_kernel<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(n, x, y, z, nd, nn, hn, L,
-                                                                n_replicas, table, count, ax, ay,
-                                                                az, pot);
+  ewald_hexa_table_kernel<<<1, PT_WAVE, 0, s>>>(nd, nn, hn, L, table);
+  ewald_hexa_kernel<<<(unsigned)((n + PT_WAVE - 1) / PT_WAVE), kEwThreads, 0, s>>>(
+      n, x, y, z, nd, nn, hn, L, n_replicas, table, ax, ay, az, pot);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
