@@ -6,17 +6,19 @@
 // which is the order the oracle defines.
 //
 // Per 8-bit digit pass:
-//   1. count_kernel   -- LDS histogram of each 2048-key tile, written
-//                        digit-major so one exclusive scan yields every
-//                        (digit, tile) output offset;
-//   2. device-wide exclusive scan of the 256 x tiles table;
-//   3. scatter_kernel -- each wave ranks its 512-key sub-tile in 8 rounds of
+//   1. count_kernel   -- LDS histogram of each tile of 512 to 2048 keys;
+//   2. with many tiles, the counts digit-major and one device-wide exclusive
+//      scan of the 256 x tiles table, which yields every (digit, tile) output
+//      offset; with few, the counts tile-major and summed by step 3;
+//   3. scatter_kernel -- each wave ranks its quarter of the tile in rounds of
 //                        64 with an 8-ballot digit match and per-wave LDS
 //                        counters; ranks become tile-local positions, keys are
 //                        staged through LDS and written out in digit runs so
 //                        the HBM writes are contiguous.
 #include "pt_common.h"
 #include "pt_kernels.h"
+
+#include <algorithm>
 
 namespace {
 
@@ -25,33 +27,66 @@ constexpr int kSortWaves = kSortThreads / PT_WAVE;
 constexpr int kSortItems = 8;
 constexpr int kSortTile = kSortThreads * kSortItems;  // 2048 keys per block
 constexpr int kRadix = 256;
+// Up to this many tiles the scatter kernel sums the digit counts before its
+// tile itself, 2 launches a pass instead of 5, and small sets take smaller
+// tiles, whose rounds are fewer (the passes are a chain of latencies: launches,
+// loads, rounds of ranking).  Sort of 4 digits, us, scan launches / own sums
+// with 2, 4, 8 keys per thread: 30k keys 84 / 41, 46, -; 64k 86 / 51, 47, 54;
+// 100k 87 / -, 54, 58; 8 digits of 200k 185 / -, -, 142.
+constexpr int kOwnTiles = 128;
+constexpr int64_t kOwnMax2 = 32768;
+constexpr int64_t kOwnMax4 = (int64_t)kOwnTiles * kSortThreads * 4;
+constexpr int64_t kOwnMax8 = (int64_t)kOwnTiles * kSortTile;
 
+// OWN: the counts are written tile-major, else digit-major.
+template <int ITEMS, bool OWN>
 __global__ void __launch_bounds__(kSortThreads)
 count_kernel(const uint64_t* __restrict__ keys, int64_t n, int shift, int ntiles,
              uint32_t* __restrict__ counts) {
   __shared__ uint32_t hist[kRadix];
   hist[threadIdx.x] = 0;
   __syncthreads();
-  const int64_t base = (int64_t)blockIdx.x * kSortTile;
-#pragma unroll 4
-  for (int j = 0; j < kSortItems; j++) {
+  const int64_t base = (int64_t)blockIdx.x * (kSortThreads * ITEMS);
+#pragma unroll
+  for (int j = 0; j < ITEMS; j++) {
     const int64_t i = base + (int64_t)j * kSortThreads + threadIdx.x;
     if (i < n) atomicAdd(&hist[(unsigned)(keys[i] >> shift) & (kRadix - 1)], 1u);
   }
   __syncthreads();
-  counts[(int64_t)threadIdx.x * ntiles + blockIdx.x] = hist[threadIdx.x];
+  counts[OWN ? (int64_t)blockIdx.x * kRadix + threadIdx.x
+             : (int64_t)threadIdx.x * ntiles + blockIdx.x] = hist[threadIdx.x];
 }
 
-// FIRST: the payload is the key's input index (vals_in unused).
-template <bool FIRST>
+// Exclusive prefix of v over the work-group's threads.
+__device__ __forceinline__ uint32_t sort_block_excl(uint32_t v, uint32_t* s_wsum) {
+  const int lane = threadIdx.x & (PT_WAVE - 1), wave = threadIdx.x / PT_WAVE;
+  uint32_t t = v;
+#pragma unroll
+  for (int d = 1; d < PT_WAVE; d <<= 1) {
+    const uint32_t o = __shfl_up(t, d, PT_WAVE);
+    if (lane >= d) t += o;
+  }
+  if (lane == PT_WAVE - 1) s_wsum[wave] = t;
+  __syncthreads();
+  for (int w = 0; w < wave; w++) t += s_wsum[w];
+  __syncthreads();
+  return t - v;
+}
+
+// FIRST: the payload is the key's input index (vals_in unused).  OWN: offsets
+// holds the tile-major counts, else their digit-major exclusive scan.
+template <bool FIRST, int ITEMS, bool OWN>
 __global__ void __launch_bounds__(kSortThreads)
 scatter_kernel(const uint64_t* __restrict__ keys_in, const uint32_t* __restrict__ vals_in,
                int64_t n, int shift, int ntiles, const uint32_t* __restrict__ offsets,
                uint64_t* __restrict__ keys_out, uint32_t* __restrict__ vals_out) {
   __shared__ uint32_t wave_run[kSortWaves][kRadix];
   __shared__ uint32_t tile_off[kRadix];
-  __shared__ uint64_t s_keys[kSortTile];
-  __shared__ uint32_t s_vals[kSortTile];
+  constexpr int kTile = kSortThreads * ITEMS;
+  __shared__ uint64_t s_keys[kTile];
+  __shared__ uint32_t s_vals[kTile];
+  __shared__ uint32_t s_dst[kRadix];  // output slot of each digit's first key, less its tile slot
+  __shared__ uint32_t s_wsum[kSortWaves];
 
   const int lane = threadIdx.x & (PT_WAVE - 1);
   const int wave = threadIdx.x / PT_WAVE;
@@ -59,15 +94,26 @@ scatter_kernel(const uint64_t* __restrict__ keys_in, const uint32_t* __restrict_
     (&wave_run[0][0])[i] = 0;
   __syncthreads();
 
-  const int64_t tile_base = (int64_t)blockIdx.x * kSortTile;
-  const int64_t wave_base = tile_base + (int64_t)wave * (kSortItems * PT_WAVE);
-  uint64_t k[kSortItems];
-  uint32_t v[kSortItems];
-  uint32_t rank[kSortItems];
+  // the thread's digit: its keys in all tiles and in the tiles before this one
+  uint32_t all = 0, before_tile = 0;
+  if (OWN) {
+#pragma unroll 8
+    for (int t = 0; t < ntiles; t++) {
+      const uint32_t c = offsets[t * kRadix + threadIdx.x];
+      all += c;
+      before_tile += t < (int)blockIdx.x ? c : 0u;
+    }
+  }
+
+  const int64_t tile_base = (int64_t)blockIdx.x * kTile;
+  const int64_t wave_base = tile_base + (int64_t)wave * (ITEMS * PT_WAVE);
+  uint64_t k[ITEMS];
+  uint32_t v[ITEMS];
+  uint32_t rank[ITEMS];
   const unsigned long long lt_mask = (1ull << lane) - 1ull;
 
 #pragma unroll
-  for (int r = 0; r < kSortItems; r++) {
+  for (int r = 0; r < ITEMS; r++) {
     const int64_t i = wave_base + (int64_t)r * PT_WAVE + lane;
     const bool valid = i < n;
     k[r] = valid ? keys_in[i] : ~0ull;
@@ -100,24 +146,16 @@ scatter_kernel(const uint64_t* __restrict__ keys_in, const uint32_t* __restrict_
       wave_run[w][d] = acc;
       acc += c;
     }
-    // exclusive scan of the tile's digit totals
-    uint32_t t = acc;
-#pragma unroll
-    for (int dd = 1; dd < PT_WAVE; dd <<= 1) {
-      const uint32_t o = __shfl_up(t, dd, PT_WAVE);
-      if (lane >= dd) t += o;
-    }
-    __shared__ uint32_t s_wsum[kSortWaves];
-    if (lane == PT_WAVE - 1) s_wsum[wave] = t;
-    __syncthreads();
-    uint32_t woff = 0;
-    for (int w = 0; w < wave; w++) woff += s_wsum[w];
-    tile_off[d] = woff + t - acc;
+    const uint32_t off = sort_block_excl(acc, s_wsum);
+    tile_off[d] = off;
+    const uint32_t out = OWN ? sort_block_excl(all, s_wsum) + before_tile
+                             : offsets[(int64_t)d * ntiles + blockIdx.x];
+    s_dst[d] = out - off;
   }
   __syncthreads();
 
 #pragma unroll
-  for (int r = 0; r < kSortItems; r++) {
+  for (int r = 0; r < ITEMS; r++) {
     const int64_t i = wave_base + (int64_t)r * PT_WAVE + lane;
     if (i < n) {
       const uint32_t d = (uint32_t)(k[r] >> shift) & (kRadix - 1);
@@ -128,11 +166,11 @@ scatter_kernel(const uint64_t* __restrict__ keys_in, const uint32_t* __restrict_
   }
   __syncthreads();
 
-  const int64_t tile_n = (n - tile_base) < kSortTile ? (n - tile_base) : kSortTile;
+  const int64_t tile_n = (n - tile_base) < kTile ? (n - tile_base) : kTile;
   for (int j = threadIdx.x; j < tile_n; j += kSortThreads) {
     const uint64_t kk = s_keys[j];
     const uint32_t d = (uint32_t)(kk >> shift) & (kRadix - 1);
-    const int64_t dst = (int64_t)offsets[(int64_t)d * ntiles + blockIdx.x] + (j - tile_off[d]);
+    const uint32_t dst = s_dst[d] + (uint32_t)j;  // modulo 2^32, below n
     keys_out[dst] = kk;
     vals_out[dst] = s_vals[j];
   }
@@ -144,11 +182,29 @@ iota_kernel(uint32_t* __restrict__ v, int64_t n) {
   if (i < n) v[i] = (uint32_t)i;
 }
 
+// One digit pass; the first has no payload to read (vin null).
+template <int ITEMS, bool OWN>
+int sort_pass(const uint64_t* kin, const uint32_t* vin, int64_t n, int shift, int ntiles,
+              uint32_t* counts, void* scan_scratch, uint64_t* kout, uint32_t* vout,
+              hipStream_t s) {
+  count_kernel<ITEMS, OWN><<<ntiles, kSortThreads, 0, s>>>(kin, n, shift, ntiles, counts);
+  if (!OWN && pt_exclusive_scan_u32(counts, counts, (int64_t)ntiles * kRadix, scan_scratch,
+                                    nullptr, s) != 0)
+    return -1;
+  if (!vin)
+    scatter_kernel<true, ITEMS, OWN><<<ntiles, kSortThreads, 0, s>>>(kin, vin, n, shift, ntiles,
+                                                                     counts, kout, vout);
+  else
+    scatter_kernel<false, ITEMS, OWN><<<ntiles, kSortThreads, 0, s>>>(kin, vin, n, shift, ntiles,
+                                                                      counts, kout, vout);
+  return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
 }  // namespace
 
 int64_t pt_sort_scratch_bytes(int64_t n) {
   const int64_t ntiles = (n + kSortTile - 1) / kSortTile;
-  const int64_t table = ntiles * kRadix;
+  const int64_t table = std::max<int64_t>(ntiles, kOwnTiles) * kRadix;
   // counts table + scan scratch + ping-pong key/value buffers
   return table * 4 + pt_scan_scratch_bytes(table) + n * 8 + n * 4 + 1024;
 }
@@ -166,7 +222,8 @@ int pt_radix_sort(const uint64_t* src, uint64_t* keys, uint32_t* vals, int64_t n
     return hipGetLastError() == hipSuccess ? 0 : -1;
   }
   if (n > 0x7fffffffll) return -1;
-  const int ntiles = (int)((n + kSortTile - 1) / kSortTile);
+  const int tile = n <= kOwnMax2 ? kSortThreads * 2 : (n <= kOwnMax4 ? kSortThreads * 4 : kSortTile);
+  const int ntiles = (int)((n + tile - 1) / tile);
   const int64_t table = (int64_t)ntiles * kRadix;
   char* p = (char*)scratch;
   uint32_t* counts = (uint32_t*)p;
@@ -187,14 +244,16 @@ int pt_radix_sort(const uint64_t* src, uint64_t* keys, uint32_t* vals, int64_t n
     const bool to_final = ((passes - 1 - p) % 2) == 0;
     uint64_t* kout = to_final ? keys : k2;
     uint32_t* vout = to_final ? vals : v2;
-    count_kernel<<<ntiles, kSortThreads, 0, s>>>(kin, n, shift, ntiles, counts);
-    if (pt_exclusive_scan_u32(counts, counts, table, scan_scratch, nullptr, s) != 0) return -1;
-    if (p == 0)
-      scatter_kernel<true><<<ntiles, kSortThreads, 0, s>>>(kin, vin, n, shift, ntiles, counts, kout,
-                                                           vout);
+    int st = 0;
+    if (n <= kOwnMax2)
+      st = sort_pass<2, true>(kin, vin, n, shift, ntiles, counts, scan_scratch, kout, vout, s);
+    else if (n <= kOwnMax4)
+      st = sort_pass<4, true>(kin, vin, n, shift, ntiles, counts, scan_scratch, kout, vout, s);
+    else if (n <= kOwnMax8)
+      st = sort_pass<8, true>(kin, vin, n, shift, ntiles, counts, scan_scratch, kout, vout, s);
     else
-      scatter_kernel<false><<<ntiles, kSortThreads, 0, s>>>(kin, vin, n, shift, ntiles, counts,
-                                                            kout, vout);
+      st = sort_pass<8, false>(kin, vin, n, shift, ntiles, counts, scan_scratch, kout, vout, s);
+    if (st != 0) return st;
     kin = kout;
     vin = vout;
   }
