@@ -48,8 +48,6 @@
 
 namespace {
 
-constexpr int kWaves = 4;
-constexpr int kThreads = kWaves * PT_WAVE;
 constexpr int kGroupMax = PT_WAVE;  // targets per pass (one per lane at most)
 // Walk stack entries after an overflow of the kernel's usual stack (the
 // deepest walks measured, a CPU replay of this walk order over 4000 sampled
@@ -890,8 +888,11 @@ __device__ __forceinline__ void finish_group(W_t& W, const Group& g, const Lanes
 // kernels
 // ---------------------------------------------------------------------------
 
+// One wave per bucket and work-group: a work-group of four holds its LDS and
+// registers until its longest list ends (200k particles, FP64: 1180 us with
+// four, 1068 with one).
 template <bool F32>
-__global__ void __launch_bounds__(kThreads)
+__global__ void __launch_bounds__(PT_WAVE)
 interact_kernel(const Bucket* __restrict__ bk, int64_t nb, const TreeNode* __restrict__ nodes,
                 const GravNode* __restrict__ gn, const GravNode32* __restrict__ gn32,
                 const double* __restrict__ px,
@@ -902,12 +903,10 @@ interact_kernel(const Bucket* __restrict__ bk, int64_t nb, const TreeNode* __res
                 double oy, double oz, double* __restrict__ ax, double* __restrict__ ay,
                 double* __restrict__ az, double* __restrict__ pot) {
   using W_t = WaveLds<F32, 8>;
-  __shared__ W_t lds[kWaves];
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PT_WAVE);
-  const int lane = threadIdx.x & (PT_WAVE - 1);
-  const int64_t bi = pt_xcd_block(blockIdx.x, gridDim.x) * kWaves + wave;
+  __shared__ W_t W;
+  const int lane = threadIdx.x;
+  const int64_t bi = pt_xcd_block(blockIdx.x, gridDim.x);
   if (bi >= nb) return;
-  W_t& W = lds[wave];
   const Bucket b = bk[bi];
   const double ccx = (b.lox + b.hix) * 0.5, ccy = (b.loy + b.hiy) * 0.5,
                ccz = (b.loz + b.hiz) * 0.5;
@@ -1165,7 +1164,7 @@ __device__ __forceinline__ void do_nodes_hexa32(W_t& W, int32_t ent, int nsrc, c
   __builtin_amdgcn_wave_barrier();
 }
 
-__global__ void __launch_bounds__(kThreads)
+__global__ void __launch_bounds__(PT_WAVE)
 interact_hexa_kernel(const Bucket* __restrict__ bk, int64_t nb,
                      const TreeNode* __restrict__ nodes, const HexNode* __restrict__ hn,
                      const double* __restrict__ px, const double* __restrict__ py,
@@ -1175,12 +1174,10 @@ interact_hexa_kernel(const Bucket* __restrict__ bk, int64_t nb,
                      const int32_t* __restrict__ pc, double ox, double oy, double oz,
                      double* __restrict__ ax, double* __restrict__ ay, double* __restrict__ az,
                      double* __restrict__ pot) {
-  __shared__ HexaLds lds[kWaves];
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PT_WAVE);
-  const int lane = threadIdx.x & (PT_WAVE - 1);
-  const int64_t bi = pt_xcd_block(blockIdx.x, gridDim.x) * kWaves + wave;
+  __shared__ HexaLds W;
+  const int lane = threadIdx.x;
+  const int64_t bi = pt_xcd_block(blockIdx.x, gridDim.x);
   if (bi >= nb) return;
-  HexaLds& W = lds[wave];
   const Bucket b = bk[bi];
   const double ccx = (b.lox + b.hix) * 0.5, ccy = (b.loy + b.hiy) * 0.5,
                ccz = (b.loz + b.hiz) * 0.5;
@@ -1912,8 +1909,6 @@ fgroup_compact_kernel(int64_t nb, const int32_t* __restrict__ tfirst,
   }
 }
 
-inline unsigned grid_for(int64_t nb) { return (unsigned)((nb + kWaves - 1) / kWaves); }
-
 }  // namespace
 
 int pt_launch_interact(int precision, const Bucket* bk, int64_t nb, const TreeNode* nodes,
@@ -1923,11 +1918,11 @@ int pt_launch_interact(int precision, const Bucket* bk, int64_t nb, const TreeNo
                        double* ay, double* az, double* pot, hipStream_t s) {
   if (nb <= 0) return 0;
   if (precision == 0) {
-    interact_kernel<false><<<grid_for(nb), kThreads, 0, s>>>(bk, nb, nodes, gn, gn32, x, y, z, m,
+    interact_kernel<false><<<(unsigned)nb, PT_WAVE, 0, s>>>(bk, nb, nodes, gn, gn32, x, y, z, m,
                                                              e, pp_off, pp, pc_off, pc, off[0],
                                                              off[1], off[2], ax, ay, az, pot);
   } else {
-    interact_kernel<true><<<grid_for(nb), kThreads, 0, s>>>(bk, nb, nodes, gn, gn32, x, y, z, m,
+    interact_kernel<true><<<(unsigned)nb, PT_WAVE, 0, s>>>(bk, nb, nodes, gn, gn32, x, y, z, m,
                                                             e, pp_off, pp, pc_off, pc, off[0], off[1],
                                                             off[2], ax, ay, az, pot);
   }
@@ -1941,7 +1936,7 @@ int pt_launch_interact_hexa(const Bucket* bk, int64_t nb, const TreeNode* nodes,
                             const double off[3], double* ax, double* ay, double* az, double* pot,
                             hipStream_t s) {
   if (nb <= 0) return 0;
-  interact_hexa_kernel<<<grid_for(nb), kThreads, 0, s>>>(bk, nb, nodes, hn, x, y, z, m, e, pp_off,
+  interact_hexa_kernel<<<(unsigned)nb, PT_WAVE, 0, s>>>(bk, nb, nodes, hn, x, y, z, m, e, pp_off,
                                                          pp, pc_off, pc, off[0], off[1], off[2],
                                                          ax, ay, az, pot);
   return hipGetLastError() == hipSuccess ? 0 : -1;
