@@ -27,15 +27,15 @@
 //
 // Kernels:
 //   interact_kernel  -- reads the per-bucket lists of pt_traverse;
-//   gravity_kernel   -- walks the tree itself (pt_walk.h, same decisions) and
-//                       evaluates each 64-entry chunk of closed nodes / leaf
-//                       sources as soon as the walk has produced it, so no
-//                       list ever reaches HBM;
-//   grouped_gravity_kernel -- the same per bucket run of at most 64
-//                       particles: one walk with the run's union box shares
-//                       every source all its buckets agree on, each bucket
-//                       walks on its own only below the nodes they decide
-//                       differently (the default of pt_compute_forces).
+//   grouped_gravity_kernel -- walks the tree itself (pt_walk.h, same
+//                       decisions) and evaluates each 64-entry chunk of closed
+//                       nodes / leaf sources as soon as the walk has produced
+//                       it, so no list ever reaches HBM.  Per bucket, or per
+//                       run of buckets of at most 64 particles: one walk with
+//                       the run's union box shares every source all its
+//                       buckets agree on, each bucket walks on its own only
+//                       below the nodes they decide differently (the default
+//                       of pt_compute_forces).
 //
 // This file is compiled with -ffp-contract=off because it contains the walk's
 // opening test; the interaction arithmetic uses explicit fma() where the
